@@ -1382,7 +1382,8 @@ __global__ __launch_bounds__(kBlock) void k_gemm_b(const LayerArgs a) {
 bool gemm_path_ok(const ftm_moe_layer& L, int T) {
   if (L.act_dtype != FTM_DT_BF16) return false;
   const int f = L.w13.fmt;
-  if (f != FTM_FMT_FP8_BLOCK && f != FTM_FMT_INT8_PACKED && f != FTM_FMT_MXFP4 && f != FTM_FMT_BF16) return false;
+  if (f != FTM_FMT_FP8_BLOCK && f != FTM_FMT_INT8_PACKED && f != FTM_FMT_MXFP4 && f != FTM_FMT_BF16 && !tile_gptq_ok(L))
+    return false;
   if (L.hidden % 64 != 0 || L.inter % 64 != 0 || (L.shared_inter > 0 && L.shared_inter % 64 != 0)) return false;
   if ((f == FTM_FMT_FP8_BLOCK || f == FTM_FMT_INT8_PACKED) &&
       (L.w13.group % kGK != 0 || L.w2.group % kGK != 0))
@@ -1426,7 +1427,7 @@ bool mx_gemm_ok(const ftm_moe_layer& L) {
 }
 
 const char* gemm_a_kernel_name(const ftm_moe_layer& L) {
-  return mx_gemm_ok(L) ? "k_gemm_mx" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
+  return L.w13.fmt == FTM_FMT_GPTQ_INT4 ? "k_tile" : mx_gemm_ok(L) ? "k_gemm_mx" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
 }
 
 template <int FMT, bool SONLY = false>
@@ -1449,6 +1450,7 @@ static bool mxb_reg_ok(const ftm_moe_layer& L, long T, int KP) {
 }
 
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T) {
+  if (L.w13.fmt == FTM_FMT_GPTQ_INT4) return "k_tile";
   if (!mx_gemm_ok(L)) return "k_gemm_b";
   return mxb_reg_ok(L, T, L.topk + (L.shared_inter > 0 ? 1 : 0)) ? "k_gemm_mxb_f8" : "k_gemm_mx";
 }
@@ -1547,6 +1549,7 @@ void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out,
                         hipStream_t st, int which, bool xq_ready) {
   const LayerArgs a = make_args(L, x, out, T, ws, wl);
   switch (L.w13.fmt) {
+    case FTM_FMT_GPTQ_INT4: launch_tile_gptq(a, st, which); break;
     case FTM_FMT_FP8_BLOCK: launch_gemm_t<FTM_FMT_FP8_BLOCK>(a, st, which, xq_ready); break;
     case FTM_FMT_INT8_PACKED: launch_gemm_t<FTM_FMT_INT8_PACKED>(a, st, which, xq_ready); break;
     case FTM_FMT_MXFP4: launch_gemm_t<FTM_FMT_MXFP4>(a, st, which, xq_ready); break;

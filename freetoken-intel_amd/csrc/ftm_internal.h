@@ -151,6 +151,8 @@ const char* gemm_a_kernel_name(const ftm_moe_layer& L);  // the stage A tile ker
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T);  // the stage B tile kernel at T tokens
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready = false);
+// GPTQ layers whose expert stages the register-fed tiles take (ftm_tile.hip).
+bool tile_gptq_ok(const ftm_moe_layer& L);
 // MXFP4 stage A on the scaled-MFMA tiles (k_gemm_a_mx) above the crossover.
 bool mx_gemm_ok(const ftm_moe_layer& L);
 // k_quant_mx: the input (T x H bf16) into the xq region's two-term e4m3 split.

@@ -1,0 +1,77 @@
+"""GPU: the expert stages above the token crossover on the register-fed tiles
+(64 rows x 256 weight rows, ftm_tile.hip) against the oracle, at the sizes
+where a tile can go wrong: partly filled row blocks, a second M tile of one
+row, channels and columns that end inside a tile, one and several K steps,
+scale groups wider than a step, a shared expert beside the routed ones."""
+from dataclasses import replace
+
+import numpy as np
+import pytest
+import torch
+
+import ftm_oracle as O
+from ftm_helpers import np_, oracle_spec, rel_rms, to_f32
+
+from ftmoe import _native as nat
+from ftmoe import synthetic as S
+
+pytestmark = pytest.mark.gpu
+
+# The oracle rounds h and the router weights to bf16 as the layer does; what
+# is left is the output's rounding (2^-9 / sqrt(3) = 1.1e-3 relative RMS) and
+# h values that fall on the other side of a rounding boundary in another
+# summation order.
+REL_RMS = 4e-3
+
+
+def _check(syn, gpu, ids=None, w=None):
+    T = syn.x.shape[0]
+    ref = O.layer_reference(oracle_spec(syn), np_(syn.x), ids=ids, w=w)
+    dsyn = syn.to(gpu)
+    layer = S.build_layer(dsyn)
+    if ids is None:
+        run = lambda: layer.forward(dsyn.x)  # noqa: E731
+    else:
+        i, v = torch.from_numpy(ids).to(gpu), torch.from_numpy(w).to(gpu)
+        run = lambda: layer.forward_routed(dsyn.x, i, v)  # noqa: E731
+    out = run()
+    torch.cuda.synchronize()
+    err = rel_rms(to_f32(out), ref["out"])
+    assert err < REL_RMS, err
+    assert torch.equal(run(), out)
+    return layer
+
+
+def _skewed(T, E, k, counts, seed):
+    """Caller routing that gives expert e counts[e] tokens (the rest spread over the others)."""
+    rng = np.random.RandomState(seed)
+    ids = np.full((T, k), -1, np.int32)
+    for e, c in enumerate(counts):
+        rows = rng.choice(np.flatnonzero((ids >= 0).sum(1) < k), c, replace=False)
+        for t in rows:
+            ids[t, (ids[t] >= 0).sum()] = e
+    return ids, O.round_bf16(rng.rand(T, k).astype(np.float32))
+
+
+@pytest.mark.parametrize("T,H,I,shared,group", [(64, 256, 384, 0, 128), (129, 384, 128, 0, 128), (200, 256, 256, 192, 128),
+                                                (90, 512, 256, 128, 256)])
+def test_gptq_tiles_match_oracle(gpu, T, H, I, shared, group):
+    """GPTQ with zero points of every value and groups of one or two K steps."""
+    cfg = replace(S.SMALL["c2_gptq"], H=H, I=I, shared_inter=shared, group=group)
+    syn = S.generate(cfg, T=T, seed=T + H)
+    g = torch.Generator().manual_seed(T)
+    for n in ("qzeros_gate_up", "qzeros_down"):
+        z = syn.bank[n]
+        syn.bank[n] = torch.randint(-2**31, 2**31 - 1, z.shape, generator=g, dtype=torch.int64).to(torch.int32)
+    layer = _check(syn, gpu)
+    assert layer.stage_kernel(T, nat.STAGE_W13) == "k_tile"
+    assert layer.stage_kernel(T, nat.STAGE_W2) == "k_tile"
+
+
+@pytest.mark.parametrize("name", ["c2_gptq"])
+def test_tiles_with_uneven_experts(gpu, name):
+    """Experts of 1, 15, 16, 17, 32, 33, 64, 65 and 129 rows, some of none."""
+    T, E, k = 144, 16, 4
+    syn = S.generate(replace(S.SMALL[name], E=E, k=k), T=T, seed=9)
+    ids, w = _skewed(T, E, k, [1, 15, 16, 17, 0, 32, 33, 64, 65, 129, 0, 48], 3)
+    _check(syn, gpu, ids, w)
