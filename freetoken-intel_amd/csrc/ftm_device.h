@@ -479,6 +479,42 @@ __device__ __forceinline__ float e4m3_at(uint32_t w) {
   return __builtin_amdgcn_cvt_f32_fp8((int)w, B);
 }
 
+// The two-term e4m3 split of 8 bf16 values (the scaled MFMAs' activations,
+// described at k_quant_mx in ftm_moe.hip) by a quad of lanes, which holds one
+// 32-element block: hi and lo codes, and the block's e8m0 scales (hi, lo << 8).
+struct MxPiece {
+  u32x2 hi, lo;
+  uint32_t sc;
+};
+__device__ __forceinline__ MxPiece mx_piece(u32x4 w) {
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = __uint_as_float(w[j] << 16);
+    v[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
+  }
+  // largest |x| bit pattern of the block (Inf and NaN: >= 0x7f800000)
+  int mb = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) mb = max(mb, (int)(__float_as_uint(v[j]) & 0x7fffffffu));
+  mb = max(mb, dpp_i<kDppXor1>(mb));
+  mb = max(mb, dpp_i<kDppXor2>(mb));
+  // E + 120 clamped to >= 0 (amax < 2^-120 keeps |x / s_hi| < 2^8 as well)
+  const uint32_t chi = (uint32_t)max((mb >> 23) - 7, 0);
+  const uint32_t clo = chi >= 4u ? chi - 4u : 0u;
+  const float inv = __uint_as_float((254u - chi) << 23);        // 1 / s_hi
+  const float flo = __uint_as_float((127u + chi - clo) << 23);  // s_hi / s_lo
+  uint32_t hw[2], lw[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float s0 = v[4 * h] * inv, s1 = v[4 * h + 1] * inv, s2 = v[4 * h + 2] * inv, s3 = v[4 * h + 3] * inv;
+    hw[h] = f32x4_to_e4m3(s0, s1, s2, s3);
+    lw[h] = f32x4_to_e4m3((s0 - e4m3_at<0>(hw[h])) * flo, (s1 - e4m3_at<1>(hw[h])) * flo,
+                          (s2 - e4m3_at<2>(hw[h])) * flo, (s3 - e4m3_at<3>(hw[h])) * flo);
+  }
+  return MxPiece{(u32x2){hw[0], hw[1]}, (u32x2){lw[0], lw[1]}, mb < 0x7f800000 ? (chi | (clo << 8)) : 0xffffu};
+}
+
 // ---------------------------------------------------------------- K-major engine
 // Formats whose weight rows are contiguous along K: FP8 block, INT8 packed,
 // MXFP4, BF16.  One "wave-load" = every lane loading 16 bytes of its row

@@ -153,6 +153,8 @@ void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out,
                         hipStream_t st, int which, bool xq_ready = false);
 // GPTQ layers whose expert stages the register-fed tiles take (ftm_tile.hip).
 bool tile_gptq_ok(const ftm_moe_layer& L);
+// FP8 stage B above the crossover on k_gemm_mxb_f8 (else k_gemm_mx).
+bool tile_mxb_ok(const ftm_moe_layer& L, int T);
 // MXFP4 stage A on the scaled-MFMA tiles (k_gemm_a_mx) above the crossover.
 bool mx_gemm_ok(const ftm_moe_layer& L);
 // k_quant_mx: the input (T x H bf16) into the xq region's two-term e4m3 split.

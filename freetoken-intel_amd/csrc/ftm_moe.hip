@@ -62,36 +62,12 @@ __device__ __forceinline__ void quant_mx_piece(const uint16_t* __restrict__ x, i
   const int k0 = 8 * q;
   u32x4 w = (u32x4){0u, 0u, 0u, 0u};
   if (k0 < H) w = *(const u32x4*)(x + (size_t)t * H + k0);  // H % 32 == 0: a block is whole or past the end
-  float v[8];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[2 * j] = __uint_as_float(w[j] << 16);
-    v[2 * j + 1] = __uint_as_float(w[j] & 0xffff0000u);
-  }
-  // largest |x| bit pattern of the block (Inf and NaN: >= 0x7f800000)
-  int mb = 0;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) mb = max(mb, (int)(__float_as_uint(v[j]) & 0x7fffffffu));
-  mb = max(mb, dpp_i<kDppXor1>(mb));
-  mb = max(mb, dpp_i<kDppXor2>(mb));
-  // E + 120 clamped to >= 0 (amax < 2^-120 keeps |x / s_hi| < 2^8 as well)
-  const uint32_t chi = (uint32_t)max((mb >> 23) - 7, 0);
-  const uint32_t clo = chi >= 4u ? chi - 4u : 0u;
-  const float inv = __uint_as_float((254u - chi) << 23);        // 1 / s_hi
-  const float flo = __uint_as_float((127u + chi - clo) << 23);  // s_hi / s_lo
-  uint32_t hw[2], lw[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const float s0 = v[4 * h] * inv, s1 = v[4 * h + 1] * inv, s2 = v[4 * h + 2] * inv, s3 = v[4 * h + 3] * inv;
-    hw[h] = f32x4_to_e4m3(s0, s1, s2, s3);
-    lw[h] = f32x4_to_e4m3((s0 - e4m3_at<0>(hw[h])) * flo, (s1 - e4m3_at<1>(hw[h])) * flo,
-                          (s2 - e4m3_at<2>(hw[h])) * flo, (s3 - e4m3_at<3>(hw[h])) * flo);
-  }
+  const MxPiece pq = mx_piece(w);
   const int c = q >> 4, p = q & 15;
   uint8_t* o = xq + (size_t)t * (size_t)((H + 127) / 128 * kMxChunk) + (size_t)c * kMxChunk;
-  *(u32x2*)(o + 8 * p) = (u32x2){hw[0], hw[1]};
-  *(u32x2*)(o + 128 + 8 * p) = (u32x2){lw[0], lw[1]};
-  if ((p & 3) == 0) *(uint16_t*)(o + 256 + (p >> 1)) = (uint16_t)(mb < 0x7f800000 ? (chi | (clo << 8)) : 0xffffu);
+  *(u32x2*)(o + 8 * p) = pq.hi;
+  *(u32x2*)(o + 128 + 8 * p) = pq.lo;
+  if ((p & 3) == 0) *(uint16_t*)(o + 256 + (p >> 1)) = (uint16_t)pq.sc;
   if (p == 0) *(u32x2*)(o + 264) = (u32x2){0u, 0u};
 }
 

@@ -55,11 +55,11 @@ __device__ __forceinline__ int tile_fa(int r) {
 
 // Tile row (weight row of the projection) of MFMA column block nj, lane
 // column m, of a wave whose first rows are base[0] (nj 0, 1) and base[1] (2,
-// 3): K-major formats 16 consecutive rows a block, GPTQ two neighbouring
-// columns a lane (one 8-byte load).
+// 3): two neighbouring rows a lane (GPTQ: one 8-byte load of two columns), so
+// that a lane's results are neighbours too.
 template <int FMT>
 __device__ __forceinline__ int tile_row(const int (&base)[2], int nj, int m) {
-  return FMT == FTM_FMT_GPTQ_INT4 ? base[nj >> 1] + 2 * m + (nj & 1) : base[nj >> 1] + 16 * (nj & 1) + m;
+  return base[nj >> 1] + 2 * m + (nj & 1);
 }
 
 // One step's packed weights of a wave and the raw words of its scales.
@@ -358,9 +358,63 @@ __device__ __forceinline__ float tile_act(float g, float u, const LayerArgs& a) 
   return act_fn(ACT, g, u, a.L.swiglu_alpha, a.L.swiglu_limit);
 }
 
+template <class F>
+__device__ __forceinline__ void tile_with_act(int act, F&& f) {
+  switch (act) {
+    case FTM_ACT_SILU: f(std::integral_constant<int, FTM_ACT_SILU>{}); break;
+    case FTM_ACT_GELU: f(std::integral_constant<int, FTM_ACT_GELU>{}); break;
+    case FTM_ACT_RELU: f(std::integral_constant<int, FTM_ACT_RELU>{}); break;
+    default: f(std::integral_constant<int, FTM_ACT_SWIGLU_OAI>{}); break;
+  }
+}
+
+// Stage A's epilogue: h = bf16(act(gate + b_g) * (up + b_u)) of the tile in
+// LDS rows of kTHPitch bytes.
+template <int FMT, int MI>
+__device__ __forceinline__ void tile_stage_h(const LayerArgs& a, int n0, const float (&bf)[4], char* lds,
+                                             const f32x4 (&acc)[MI][4]) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  auto stage = [&](auto act) {
+#pragma unroll
+    for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float h0 = tile_act<decltype(act)::value>(acc[mi][0][r] + bf[0], acc[mi][2][r] + bf[2], a);
+        const float h1 = tile_act<decltype(act)::value>(acc[mi][1][r] + bf[1], acc[mi][3][r] + bf[3], a);
+        *(uint32_t*)(lds + (16 * mi + 4 * g + r) * kTHPitch + 64 * wave + 4 * m) = pack_bf16x2(h0, h1);
+      }
+  };
+  tile_with_act(a.L.act, stage);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Stage B's epilogue: router-weighted fp32 rows into the slot buffer.
+template <int FMT, int MI>
+__device__ __forceinline__ void tile_store_y(const LayerArgs& a, const ProjSlot& W, const int (&base)[2],
+                                             const float (&bf)[4], int rows, const int* s_pair, const float* s_w,
+                                             const f32x4 (&acc)[MI][4]) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * mi + 4 * g + r;
+      if (row < rows) {
+        float* y = a.ybuf + (size_t)s_pair[row] * a.L.hidden;
+        const float w = s_w[row];
+#pragma unroll
+        for (int nj = 0; nj < 4; nj += 2) {  // N is a multiple of 64: both columns of a lane or none
+          const int col = tile_row<FMT>(base, nj, m);
+          if (col < W.N) *(f32x2*)(y + col) = (f32x2){(acc[mi][nj][r] + bf[nj]) * w, (acc[mi][nj + 1][r] + bf[nj + 1]) * w};
+        }
+      }
+    }
+}
+
 template <int FMT, int MODE, int MI, bool STB>
 __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                         const int* s_pair, const float* s_w, float* s_bias, float* Xs) {
+                                         const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
   using F = TileFmt<FMT>;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -377,9 +431,6 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
     arow[i] = abase + (size_t)(STB ? pr : pr / KP) * arb;
   }
   const int base[2] = {n0 + (STB ? 64 : 32) * wave, STB ? n0 + 64 * wave + 32 : Iu + n0 + 32 * wave};
-  // the tile's biases as fp32 in LDS (read in the epilogue)
-  const int brow = STB || tid < kTN / 2 ? n0 + tid : Iu + n0 + tid - kTN / 2;
-  s_bias[tid] = W.bias != nullptr && brow < W.N ? load_scalar(W.bias, brow, W.bias_dt) : 0.0f;
   f32x4 acc[MI][4];
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)
@@ -392,43 +443,9 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) bf[nj] = s_bias[tile_row<FMT>(lb, nj, m)];
   if constexpr (STB) {
-    // router-weighted fp32 rows into the slot buffer
-#pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * mi + 4 * g + r;
-        if (row < rows) {
-          float* y = a.ybuf + (size_t)s_pair[row] * H;
-          const float w = s_w[row];
-#pragma unroll
-          for (int nj = 0; nj < 4; ++nj) {
-            const int col = tile_row<FMT>(base, nj, m);
-            if (col < W.N) y[col] = (acc[mi][nj][r] + bf[nj]) * w;
-          }
-        }
-      }
+    tile_store_y<FMT, MI>(a, W, base, bf, rows, s_pair, s_w, acc);
   } else {
-    // h rows staged in the ring, then copied out in 16-byte pieces
-    auto stage = [&](auto act) {
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            const float h = tile_act<decltype(act)::value>(acc[mi][j][r] + bf[j], acc[mi][2 + j][r] + bf[2 + j], a);
-            const int ch = tile_row<FMT>(base, j, m) - n0;
-            *(uint16_t*)(lds + (16 * mi + 4 * g + r) * kTHPitch + 2 * ch) = f32_to_bf16(h);
-          }
-    };
-    switch (a.L.act) {
-      case FTM_ACT_SILU: stage(std::integral_constant<int, FTM_ACT_SILU>{}); break;
-      case FTM_ACT_GELU: stage(std::integral_constant<int, FTM_ACT_GELU>{}); break;
-      case FTM_ACT_RELU: stage(std::integral_constant<int, FTM_ACT_RELU>{}); break;
-      default: stage(std::integral_constant<int, FTM_ACT_SWIGLU_OAI>{}); break;
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    tile_stage_h<FMT, MI>(a, n0, bf, lds, acc);
     for (int q = tid; q < 16 * MI * 16; q += kBlock) {
       const int row = q >> 4, pc = q & 15;
       if (row < rows && n0 + 8 * pc < Iu)
@@ -438,13 +455,10 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
   }
 }
 
-// One item: a tile of 64 rows x 128 channels (stage A) or 256 columns (B).
-// Items run expert by expert (ascending compact index), within an expert over
-// its M tiles first: the workgroups in flight on an XCD then share an
-// expert's weight columns and its activation rows in that XCD's L2.
+// The tile on the instantiation for its number of 16-row blocks.
 template <int FMT, int MODE, bool STB>
 __device__ __forceinline__ void tile_rows(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                          const int* s_pair, const float* s_w, float* s_bias, float* Xs) {
+                                          const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
   if (rows > 32) tile_run<FMT, MODE, 4, STB>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias, Xs);
   else tile_run<FMT, MODE, 2, STB>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias, Xs);
 }
@@ -458,17 +472,23 @@ constexpr int tile_ring(bool shared) {
                                                                       : TileFmt<FMT>::kRing;
 }
 
-template <int FMT, int MODE, bool STB>
-__global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a, int ring) {
-  char* lds = ftm_tile_lds;
-  int* s_pair = (int*)(lds + ring);
-  float* s_w = (float*)(s_pair + kTM);
-  float* s_bias = s_w + kTM;
-  float* Xs = s_bias + kTN;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int item = xcd_item(blockIdx.x, gridDim.x);
+// One item: a tile of 64 rows x 128 channels (stage A) or 256 columns (B).
+// Items run expert by expert (ascending compact index), within an expert over
+// its M tiles first: the workgroups in flight on an XCD then share an
+// expert's weight columns and its activation rows in that XCD's L2.  The
+// shared expert's items come last.  rows <= 0: no item.
+struct TileItem {
+  const int32_t* list;  // the expert's pairs (null: the shared expert)
+  int m0, rows, n0, slot;
+  bool shared;
+};
+
+template <bool STB>
+__device__ __forceinline__ TileItem tile_item(const LayerArgs& a) {
+  const int lane = threadIdx.x & 63;
   const int I = a.L.inter, Is = a.L.shared_inter, H = a.L.hidden;
-  const int ntn = STB ? (H + kTN - 1) / kTN : (I + kTN / 2 - 1) / (kTN / 2);
+  constexpr int tn = STB ? kTN : kTN / 2;
+  const int ntn = ((STB ? H : I) + tn - 1) / tn;
   // lane l owns compact experts 8 l .. 8 l + 7 (E <= 512)
   const Rsrc cres = make_rsrc(a.ucnt, (uint32_t)((a.L.num_experts + 8) / 8) * 32u);
   const u32x4 c0 = bload16(cres, 32u * (uint32_t)lane), c1 = bload16(cres, 32u * (uint32_t)lane + 16u);
@@ -487,10 +507,14 @@ __global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a, int ring)
     if (lane >= off) incl += o;
   }
   const int routed = __builtin_amdgcn_readlane(incl, 63) * ntn;
-  const int32_t* list = nullptr;
-  int m0, cnt, n0, slot = 0;
-  bool shared = false;
-  if (item < routed) {
+  const int nts = Is == 0 ? 0 : ((STB ? H : Is) + tn - 1) / tn, mts = (a.T + kTM - 1) / kTM;
+  // the grid is an upper bound: both kinds are spread over the XCDs by the
+  // items there are (spread over the grid, the last XCDs would find none)
+  const int bid = (int)blockIdx.x - nts * mts;
+  TileItem t = {nullptr, 0, 0, 0, 0, false};
+  if (bid >= routed) return t;
+  if (bid >= 0) {
+    const int item = xcd_item(bid, routed);
     int b = (incl - lsum) * ntn, fu = -1, fl = 0, fc = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -504,47 +528,429 @@ __global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a, int ring)
     }
     const int src = (int)__builtin_ctzll(__ballot(fu >= 0));
     const int u = __builtin_amdgcn_readlane(fu, src), loc = __builtin_amdgcn_readlane(fl, src);
-    cnt = __builtin_amdgcn_readlane(fc, src);
+    const int cnt = __builtin_amdgcn_readlane(fc, src);
     const int mt = (cnt + kTM - 1) / kTM;
-    m0 = (loc % mt) * kTM;
-    n0 = loc / mt;
+    t.n0 = loc / mt;
+    t.m0 = (loc - t.n0 * mt) * kTM;
+    t.rows = cnt - t.m0;
     const int e = __builtin_amdgcn_readfirstlane(a.uniq[u]);
-    list = a.lists + (size_t)e * a.T;
-    slot = __builtin_amdgcn_readfirstlane(a.L.slot_of_expert ? a.L.slot_of_expert[e] : e);
+    t.list = a.lists + (size_t)e * a.T;
+    t.slot = __builtin_amdgcn_readfirstlane(a.L.slot_of_expert ? a.L.slot_of_expert[e] : e);
   } else {
-    const int nts = STB ? ntn : (Is + kTN / 2 - 1) / (kTN / 2), mts = (a.T + kTM - 1) / kTM;
-    const int loc = item - routed;
-    if (Is == 0 || loc >= nts * mts) return;
-    m0 = (loc % mts) * kTM;
-    n0 = loc / mts;
-    cnt = a.T;
-    shared = true;
+    const int loc = xcd_item(blockIdx.x, nts * mts);
+    t.n0 = loc / mts;
+    t.m0 = (loc - t.n0 * mts) * kTM;
+    t.rows = a.T - t.m0;
+    t.shared = true;
   }
-  n0 *= STB ? kTN : kTN / 2;
-  const int rows = cnt - m0 < kTM ? cnt - m0 : kTM;
+  t.rows = t.rows < kTM ? t.rows : kTM;
+  t.n0 *= tn;
+  return t;
+}
+
+// The tile's pairs, biases (fp32) and (stage B) router weights in LDS.
+template <bool STB>
+__device__ __forceinline__ void tile_tables(const LayerArgs& a, const TileItem& t, int* s_pair, float* s_w,
+                                            float* s_bias) {
+  const int tid = threadIdx.x;
+  const ftm_proj& PW = STB ? a.L.w2 : a.L.w13;
+  float bias = 0.0f;
+  if (!t.shared && PW.bias != nullptr && t.slot >= 0 && t.slot < PW.num_slots) {
+    const int row = STB || tid < kTN / 2 ? t.n0 + tid : a.L.inter + t.n0 + tid - kTN / 2;
+    if (row < PW.N) bias = load_scalar((const char*)PW.bias + (int64_t)t.slot * PW.bias_stride, row, PW.bias_dtype);
+  }
   if (tid < kTM) {
-    const int p = tid < rows ? (list != nullptr ? list[m0 + tid] : (m0 + tid) * a.KP + a.L.topk) : 0;
+    const int p = tid < t.rows ? (t.list != nullptr ? t.list[t.m0 + tid] : (t.m0 + tid) * a.KP + a.L.topk) : 0;
     s_pair[tid] = p;
-    if (STB) s_w[tid] = tid < rows ? a.wts[p] : 0.0f;
+    if (STB) s_w[tid] = tid < t.rows ? a.wts[p] : 0.0f;
   }
+  s_bias[tid] = bias;
   __syncthreads();
-  if (shared) {
+}
+
+// A non-resident expert's tile: its rows contribute zeros (stage B), and the
+// error word says so.
+template <bool STB>
+__device__ __forceinline__ void tile_missing(const LayerArgs& a, const TileItem& t, const int* s_pair) {
+  if (STB) {
+    const int H = a.L.hidden;
+    for (int idx = threadIdx.x; idx < kTM * kTN; idx += kBlock) {
+      const int row = idx / kTN, col = t.n0 + idx % kTN;
+      if (row < t.rows && col < H) a.ybuf[(size_t)s_pair[row] * H + col] = 0.0f;
+    }
+  }
+  if (threadIdx.x == 0) atomicOr(&a.ctrl[kCtrlError], 1);
+}
+
+template <int FMT, int MODE, bool STB>
+__global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a, int ring) {
+  char* lds = ftm_tile_lds;
+  int* s_pair = (int*)(lds + ring);
+  float* s_w = (float*)(s_pair + kTM);
+  float* s_bias = s_w + kTM;
+  float* Xs = s_bias + kTN;
+  const TileItem t = tile_item<STB>(a);
+  if (t.rows <= 0) return;
+  tile_tables<STB>(a, t, s_pair, s_w, s_bias);
+  const int H = a.L.hidden, I = a.L.inter, Is = a.L.shared_inter;
+  const int n0 = t.n0, rows = t.rows, slot = t.slot;
+  if (t.shared) {
     const ProjSlot W = STB ? shared_view(a.L.shared_w2, H, Is) : shared_view(a.L.shared_w13, 2 * Is, H);
     tile_rows<FTM_FMT_BF16, kScaleNone, STB>(a, W, Is, n0, rows, lds, s_pair, s_w, s_bias, Xs);
     return;
   }
   const ftm_proj& PW = STB ? a.L.w2 : a.L.w13;
   if (slot < 0 || slot >= PW.num_slots) {
-    if (STB) {  // non-resident expert: its rows contribute zeros
-      for (int idx = tid; idx < kTM * kTN; idx += kBlock) {
-        const int row = idx / kTN, col = n0 + idx % kTN;
-        if (row < rows && col < H) a.ybuf[(size_t)s_pair[row] * H + col] = 0.0f;
-      }
-    }
-    if (tid == 0) atomicOr(&a.ctrl[kCtrlError], 1);
+    tile_missing<STB>(a, t, s_pair);
     return;
   }
   tile_rows<FMT, MODE, STB>(a, proj_slot(PW, slot), I, n0, rows, lds, s_pair, s_w, s_bias, Xs);
+}
+
+// ---------------------------------------------------------------- scaled-MFMA tiles
+// The routed experts of MXFP4 and FP8 (128 x 128 blocks) layers: the same
+// tile on v_mfma_scale_f32_16x16x128_f8f6f4 with the decode path's operand
+// layouts (ftm_moe.hip).  The weights go in as stored, straight from the
+// buffer loads (e4m3, or e2m1 with e8m0 as scale_b); the activations as their
+// two-term e4m3 split (kMxChunk bytes per row and 128 K: the input by token
+// from the router launch, h by pair from stage A's epilogue).  One K step is
+// one MFMA pair per 16 x 16 block, so FP8's block scale multiplies the pair's
+// sums and no second accumulator set is held.
+//
+// The activation rows are requested two K steps ahead, by direct buffer->LDS
+// copies into a ring of three stages (buffer copies, not the global ones:
+// those count as FLAT accesses, after which the compiler waits for every load
+// in flight before it uses any), the weights one step ahead into one of two
+// register sets.
+constexpr int kXRow = 256;                           // hi and lo terms of a row and step
+constexpr int kXStage = kTM * kXRow + kTM * 16;      // + the rows' scale bytes, 16 a row
+constexpr int kXStages = 3;
+constexpr int kXbSteps = 4;  // k_gemm_mxb_f8: K of at most this many steps, a stage for each
+
+template <int FMT>
+struct MxW {
+  u32x4 w[4][FMT == FTM_FMT_MXFP4 ? 1 : 2];
+  uint32_t s[4];  // MXFP4: the lane's e8m0 byte of block nj; FP8: [0] / [2], the halves' fp32 block scales
+};
+
+// This thread's activation sources: byte offsets (BIG: addresses) of the rows
+// its copies read.  Copy i of a wave covers rows 16 wave + 4 i + lane / 16
+// (16-byte pieces, swizzled), its last one the scale bytes of rows 16 wave +
+// lane / 4.
+struct MxRows {
+  uint64_t p[5];
+};
+
+// Wait until at most NW + NA n vector-memory operations are in flight (n < 4).
+template <int NW, int NA>
+__device__ __forceinline__ void wait_n(int n) {
+  if (n == 3) wait_vm<NW + 3 * NA>();
+  else if (n == 2) wait_vm<NW + 2 * NA>();
+  else if (n == 1) wait_vm<NW + NA>();
+  else wait_vm<NW>();
+}
+
+// One K step of a wave: 16 MI activation rows of the LDS stage st against its
+// 64 weight rows, into acc.
+template <int FMT, int MI>
+__device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, f32x4 (&acc)[MI][4]) {
+  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK;
+  constexpr int NL = F8 ? 2 : 1;
+  const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
+  i32x8 bw[4];
+  int sb[4];
+#pragma unroll
+  for (int nj = 0; nj < 4; ++nj) {
+    const u32x4 r0 = cur.w[nj][0];
+    if constexpr (F8) {
+      const u32x4 r1 = cur.w[nj][NL - 1];
+      bw[nj] = (i32x8){(int)r0.x, (int)r0.y, (int)r0.z, (int)r0.w, (int)r1.x, (int)r1.y, (int)r1.z, (int)r1.w};
+      sb[nj] = 127;
+    } else {
+      bw[nj] = (i32x8){(int)r0.x, (int)r0.y, (int)r0.z, (int)r0.w, 0, 0, 0, 0};
+      sb[nj] = (int)cur.s[nj];
+    }
+  }
+  // each term of a row block is read from LDS during the MFMAs of the term
+  // before it, and FP8's products of block mi are scaled into acc during
+  // block mi + 1's
+  struct Term {
+    u32x4 a, b;
+  };
+  auto term = [&](int mi, int lo) {
+    const char* cb = st + (16 * mi + m) * kXRow;
+    Term t;
+    t.a = *(const u32x4*)(cb + 16 * ((8 * lo + g) ^ m));
+    t.b = *(const u32x4*)(cb + 16 * ((8 * lo + 4 + g) ^ m));
+    return t;
+  };
+  auto scales = [&](int mi) { return (uint32_t)*(const uint16_t*)(st + kTM * kXRow + 16 * (16 * mi + m) + 2 * g); };
+  f32x4 tq[2][4];
+  auto fold = [&](int mi) {
+    if constexpr (F8) {
+#pragma unroll
+      for (int nj = 0; nj < 4; ++nj) acc[mi][nj] += tq[mi & 1][nj] * __uint_as_float(cur.s[nj & 2]);
+    }
+  };
+  constexpr int kB = F8 ? 0 : 4;  // B format: e4m3 or e2m1
+  auto mma = [&](int mi, const Term& t, int scale, bool first) {
+    const i32x8 av = {(int)t.a.x, (int)t.a.y, (int)t.a.z, (int)t.a.w, (int)t.b.x, (int)t.b.y, (int)t.b.z, (int)t.b.w};
+#pragma unroll
+    for (int nj = 0; nj < 4; ++nj) {
+      f32x4& d = F8 ? tq[mi & 1][nj] : acc[mi][nj];
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bw[nj], F8 && first ? z : d, 0, kB, 0, scale, 0, sb[nj]);
+    }
+  };
+  Term hi = term(0, 0);
+  uint32_t sc = scales(0);
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi) {
+    const Term lo = term(mi, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(mi, hi, (int)(sc & 0xffu), true);
+    const int slo = (int)(sc >> 8);
+    __builtin_amdgcn_sched_barrier(0);
+    if (mi + 1 < MI) {
+      hi = term(mi + 1, 0);
+      sc = scales(mi + 1);
+    }
+    if (mi > 0) fold(mi - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(mi, lo, slo, false);
+  }
+  fold(MI - 1);
+}
+
+template <int FMT, int MI, bool BIG, bool SHORT>
+__device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2], const char* abase, uint32_t abytes,
+                                         const MxRows& rows, char* lds, f32x4 (&acc)[MI][4]) {
+  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK;
+  constexpr int NL = F8 ? 2 : 1;
+  constexpr int NA = 5, NW = 4 * NL + (F8 ? 2 : 4);  // copies / loads a step
+  typedef __attribute__((address_space(1))) const void* GPtr;
+  typedef __attribute__((address_space(3))) void* LPtr;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4, m = lane & 15;
+  const int K = W.K, N = W.N;
+  const int nsteps = (K + 127) / 128;
+  const Rsrc ares = make_rsrc(abase, abytes);
+  uint32_t aoff[NA];
+#pragma unroll
+  for (int i = 0; i < NA; ++i) aoff[i] = (uint32_t)rows.p[i];
+  auto issue_a = [&](int kb, int slot) {
+    const uint32_t so = (uint32_t)(kb < nsteps ? kb : nsteps - 1) * (uint32_t)kMxChunk;
+    char* st = lds + slot * kXStage;
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      char* dst = i < 4 ? st + (16 * wave + 4 * i) * kXRow : st + kTM * kXRow + 256 * wave;
+      if constexpr (BIG) {
+        if (i < 4) __builtin_amdgcn_global_load_lds((GPtr)(rows.p[i] + so), (LPtr)dst, 16, 0, 0);
+        else __builtin_amdgcn_global_load_lds((GPtr)(rows.p[i] + so), (LPtr)dst, 4, 0, 0);
+      } else {
+        if (i < 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (LPtr)dst, 16, (int)aoff[i], (int)so, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (LPtr)dst, 4, (int)aoff[i], (int)so, 0, 0);
+      }
+    }
+  };
+
+  const uint32_t rb = F8 ? (uint32_t)K : (uint32_t)K / 2;
+  const int nkb = K / 128;
+  const Rsrc wres = make_rsrc(W.w, rb * (uint32_t)N);
+  const Rsrc sres = make_rsrc(W.s, F8 ? 4u * (uint32_t)((N + 127) / 128) * (uint32_t)nkb : (uint32_t)N * (uint32_t)(K / 32));
+  uint32_t woff[4];
+#pragma unroll
+  for (int nj = 0; nj < 4; ++nj) {
+    const int row = tile_row<FMT>(base, nj, m);
+    woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
+  }
+  auto load_w = [&](int kb, MxW<FMT>& t) {
+    const int k0 = F8 ? kb * 128 : kb * 128 + 32 * g;  // FP8: K is whole steps
+    const uint32_t so = k0 < K ? 4u * (uint32_t)kb : kOOB;
+    const uint32_t ko = k0 < K ? (uint32_t)kb * (F8 ? 128u : 64u) : kOOB;
+    if constexpr (F8) {
+#pragma unroll
+      for (int h = 0; h < 4; h += 2) t.s[h] = bload4(sres, 4u * (uint32_t)(base[h >> 1] / 128 * nkb) + so);
+    } else {
+      // the e8m0 byte of a 16-byte piece sits at a sixteenth of its offset
+      // (rows past N: past the scales' end as well)
+#pragma unroll
+      for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload1(sres, (woff[nj] >> 4) + so);
+    }
+#pragma unroll
+    for (int nj = 0; nj < 4; ++nj)
+#pragma unroll
+      for (int i = 0; i < NL; ++i) t.w[nj][i] = bload16(wres, woff[nj] + ko + 64u * (uint32_t)i);
+  };
+
+  MxW<FMT> w0, w1;
+  if constexpr (SHORT) {
+    // at most kXbSteps steps: every stage's copies go out at once, each step
+    // waits for its own
+    issue_a(0, 0);
+    load_w(0, w0);
+#pragma unroll
+    for (int kb = 1; kb < kXbSteps; ++kb) issue_a(kb, kb);
+#pragma unroll
+    for (int kb = 0; kb < kXbSteps; ++kb) {
+      if (kb < nsteps) {
+        const MxW<FMT>& cur = kb & 1 ? w1 : w0;
+        // younger than stage kb's copies: this step's weights, the later stages' copies
+        wait_n<NW, NA>(kXbSteps - 1 - kb);
+        asm volatile("s_barrier" ::: "memory");
+        if (kb + 1 < kXbSteps) load_w(kb + 1, kb & 1 ? w0 : w1);
+        __builtin_amdgcn_sched_barrier(0);
+        mx_step<FMT, MI>(lds + kb * kXStage, cur, acc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  } else {
+    auto step = [&](int kb, int slot, const MxW<FMT>& cur, MxW<FMT>& nxt) {
+      // the copies of stage kb have landed (younger: this step's weights, the
+      // copies of stage kb + 1), then every wave's have, and every wave is
+      // done reading stage kb - 1
+      wait_vm<NW + NA>();
+      asm volatile("s_barrier" ::: "memory");
+      issue_a(kb + 2, slot == 0 ? 2 : slot - 1);
+      load_w(kb + 1, nxt);
+      __builtin_amdgcn_sched_barrier(0);
+      mx_step<FMT, MI>(lds + slot * kXStage, cur, acc);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    issue_a(0, 0);
+    load_w(0, w0);
+    issue_a(1, 1);
+    int slot = 0;
+    auto next = [&] { slot = slot == 2 ? 0 : slot + 1; };
+    if constexpr (F8) {
+      // an odd last step of its own: with a branch round the second step of a
+      // pair the compiler waits for this step's weights before it requests the
+      // next ones (MXFP4 has no registers for the third copy of the step)
+      int kb = 0;
+      for (; kb + 1 < nsteps; kb += 2) {
+        step(kb, slot, w0, w1);
+        next();
+        step(kb + 1, slot, w1, w0);
+        next();
+      }
+      if (kb < nsteps) step(kb, slot, w0, w1);
+    } else {
+      for (int kb = 0; kb < nsteps; kb += 2) {
+        step(kb, slot, w0, w1);
+        next();
+        if (kb + 1 < nsteps) step(kb + 1, slot, w1, w0);
+        next();
+      }
+    }
+  }
+  // the copies past the last step have landed and every wave is done with the ring
+  wait_vm<0>();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+template <bool STB, bool BIG>
+__device__ __forceinline__ MxRows mx_rows(const LayerArgs& a, int rows, const int* s_pair) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const uint32_t arb = (uint32_t)mx_row_bytes(STB ? a.Imax : a.L.hidden);
+  const char* abase = (const char*)(STB ? a.hq : a.xq);
+  // padding rows repeat the first (their outputs are dropped)
+  MxRows ar;
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int r = 16 * wave + (i < 4 ? 4 * i + (lane >> 4) : lane >> 2);
+    const int pr = s_pair[r < rows ? r : 0];
+    const uint64_t off = (uint64_t)(STB ? pr : pr / a.KP) * arb +
+                         (i < 4 ? 16 * ((lane & 15) ^ (r & 15)) : 256 + 4 * (lane & 3));
+    ar.p[i] = BIG ? (uint64_t)(uintptr_t)abase + off : off;
+  }
+  return ar;
+}
+
+template <int FMT, int MI, bool STB, bool BIG, bool SHORT>
+__device__ __forceinline__ void mx_run(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
+                                       const int* s_pair, const float* s_w, const float* s_bias) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int m = lane & 15;
+  const int KP = a.KP, H = a.L.hidden;
+  const uint32_t arb = (uint32_t)mx_row_bytes(STB ? a.Imax : H);
+  const char* abase = (const char*)(STB ? a.hq : a.xq);
+  const MxRows ar = mx_rows<STB, BIG>(a, rows, s_pair);
+  const uint32_t abytes = BIG ? 0u : (uint32_t)(STB ? a.T * KP : a.T) * arb;
+  const int base[2] = {n0 + (STB ? 64 : 32) * wave, STB ? n0 + 64 * wave + 32 : Iu + n0 + 32 * wave};
+  f32x4 acc[MI][4];
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  mx_kloop<FMT, MI, BIG, SHORT>(W, base, abase, abytes, ar, lds, acc);
+
+  const int lb[2] = {(STB ? 64 : 32) * wave, STB ? 64 * wave + 32 : kTN / 2 + 32 * wave};
+  float bf[4];
+#pragma unroll
+  for (int nj = 0; nj < 4; ++nj) bf[nj] = s_bias[tile_row<FMT>(lb, nj, m)];
+  if constexpr (STB) {
+    tile_store_y<FMT, MI>(a, W, base, bf, rows, s_pair, s_w, acc);
+  } else {
+    // h = bf16(act(gate) up) to LDS rows of 128 channels, then split into
+    // e4m3 hi + lo, 8 channels a thread and one 32-channel block a quad of
+    // lanes (channels past I are zeros: the tile is one whole chunk)
+    tile_stage_h<FMT, MI>(a, n0, bf, lds, acc);
+    const size_t hrow = (size_t)mx_row_bytes(a.Imax);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int row = 16 * i + (tid >> 4), pc = tid & 15;
+      u32x4 v = *(const u32x4*)(lds + row * kTHPitch + 16 * pc);
+      if (n0 + 8 * pc >= Iu) v = (u32x4){0u, 0u, 0u, 0u};
+      const MxPiece q = mx_piece(v);
+      if (row < rows) {
+        uint8_t* o = a.hq + (size_t)s_pair[row] * hrow + (size_t)(n0 / 128) * kMxChunk;
+        *(u32x2*)(o + 8 * pc) = q.hi;
+        *(u32x2*)(o + 128 + 8 * pc) = q.lo;
+        if ((pc & 3) == 0) *(uint16_t*)(o + 256 + (pc >> 1)) = (uint16_t)q.sc;
+      }
+    }
+  }
+}
+
+template <int FMT, bool STB, bool BIG, bool SHORT>
+__device__ __forceinline__ void mx_tile(const LayerArgs& a, int ring) {
+  char* lds = ftm_tile_lds;
+  int* s_pair = (int*)(lds + ring);
+  float* s_w = (float*)(s_pair + kTM);
+  float* s_bias = s_w + kTM;
+  const TileItem t = tile_item<STB>(a);
+  if (t.rows <= 0) return;
+  tile_tables<STB>(a, t, s_pair, s_w, s_bias);
+  const int H = a.L.hidden, I = a.L.inter, Is = a.L.shared_inter;
+  if (t.shared) {
+    const ProjSlot W = STB ? shared_view(a.L.shared_w2, H, Is) : shared_view(a.L.shared_w13, 2 * Is, H);
+    tile_rows<FTM_FMT_BF16, kScaleNone, STB>(a, W, Is, t.n0, t.rows, lds, s_pair, s_w, s_bias, nullptr);
+    return;
+  }
+  const ftm_proj& PW = STB ? a.L.w2 : a.L.w13;
+  if (t.slot < 0 || t.slot >= PW.num_slots) {
+    tile_missing<STB>(a, t, s_pair);
+    return;
+  }
+  const ProjSlot W = proj_slot(PW, t.slot);
+  if (t.rows > 32) mx_run<FMT, 4, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
+  else mx_run<FMT, 2, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
+}
+
+template <int FMT, bool STB, bool BIG>
+__global__ __launch_bounds__(kBlock, FMT == FTM_FMT_MXFP4 ? 3 : 2) void k_gemm_mx(const LayerArgs a) {
+  mx_tile<FMT, STB, BIG, false>(a, kXStages * kXStage);
+}
+
+// FP8 stage B with K = I of at most kXbSteps steps (the layer of 256 experts
+// of 512): an LDS stage for every step, so no copy is issued past the last.
+// Products, scales and epilogue are k_gemm_mx's, in the same order: the
+// output is the same bits.
+__global__ __launch_bounds__(kBlock, 2) void k_gemm_mxb_f8(const LayerArgs a) {
+  mx_tile<FTM_FMT_FP8_BLOCK, true, false, true>(a, kXbSteps * kXStage);
 }
 
 // ---------------------------------------------------------------- launch
@@ -565,28 +971,86 @@ bool tile_gptq_ok(const ftm_moe_layer& L) {
   return tile_lds<FTM_FMT_GPTQ_INT4>(L, false) <= 160u * 1024u && tile_lds<FTM_FMT_GPTQ_INT4>(L, true) <= 160u * 1024u;
 }
 
-template <int FMT, int MODE, bool STB>
-static void launch_tile_t(const LayerArgs& a, hipStream_t st) {
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_tile<FMT, MODE, STB>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr = true;
-  }
+// Items of one stage, an upper bound: every routed expert's last M tile may
+// be partly filled.
+template <bool STB>
+static unsigned tile_items(const LayerArgs& a) {
   const ftm_moe_layer& L = a.L;
   const long pairs = (long)a.T * L.topk;
   const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
   const int I = L.inter, Is = L.shared_inter, H = L.hidden;
-  const long ntn = STB ? (H + kTN - 1) / kTN : (I + kTN / 2 - 1) / (kTN / 2);
-  const long nts = Is == 0 ? 0 : STB ? ntn : (Is + kTN / 2 - 1) / (kTN / 2);
-  const long items = (pairs / kTM + maxU) * ntn + (long)((a.T + kTM - 1) / kTM) * nts;
-  hipLaunchKernelGGL((k_tile<FMT, MODE, STB>), dim3((unsigned)items), dim3(kBlock), tile_lds<FMT>(L, STB), st, a,
-                     tile_ring<FMT>(Is > 0));
+  constexpr long tn = STB ? kTN : kTN / 2;
+  const long ntn = ((STB ? H : I) + tn - 1) / tn, nts = Is == 0 ? 0 : ((STB ? H : Is) + tn - 1) / tn;
+  return (unsigned)((pairs / kTM + maxU) * ntn + (long)((a.T + kTM - 1) / kTM) * nts);
+}
+
+template <class K>
+static void tile_attr(K* kernel, bool& done) {
+  if (!done) {
+    // a failure here surfaces as the launch error that follows
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              160 * 1024);
+    done = true;
+  }
+}
+
+template <int FMT, int MODE, bool STB>
+static void launch_tile_t(const LayerArgs& a, hipStream_t st) {
+  static bool attr = false;
+  tile_attr(&k_tile<FMT, MODE, STB>, attr);
+  hipLaunchKernelGGL((k_tile<FMT, MODE, STB>), dim3(tile_items<STB>(a)), dim3(kBlock), tile_lds<FMT>(a.L, STB), st, a,
+                     tile_ring<FMT>(a.L.shared_inter > 0));
 }
 
 void launch_tile_gptq(const LayerArgs& a, hipStream_t st, int which) {
   if (which & 1) launch_tile_t<FTM_FMT_GPTQ_INT4, kScale128, false>(a, st);
   if (which & 2) launch_tile_t<FTM_FMT_GPTQ_INT4, kScale128, true>(a, st);
+}
+
+template <int FMT, bool STB, bool BIG>
+static void launch_mx_t(const LayerArgs& a, hipStream_t st) {
+  static bool attr = false;
+  tile_attr(&k_gemm_mx<FMT, STB, BIG>, attr);
+  constexpr int kRing = kXStages * kXStage;
+  static_assert(kRing >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
+  hipLaunchKernelGGL((k_gemm_mx<FMT, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock),
+                     (size_t)kRing + (size_t)kTM * 8u + (size_t)kTN * 4u, st, a);
+}
+
+// BIG: activation rows past what one buffer descriptor's 32-bit offsets span.
+template <int FMT, bool STB>
+static void launch_mx_s(const LayerArgs& a, hipStream_t st) {
+  const double rows = STB ? (double)a.T * a.KP : (double)a.T;
+  if (rows * (double)mx_row_bytes(STB ? a.Imax : a.L.hidden) < 4294967296.0) launch_mx_t<FMT, STB, false>(a, st);
+  else launch_mx_t<FMT, STB, true>(a, st);
+}
+
+// k_gemm_mxb_f8's layers; FTM_PROJ_RING_B asks for k_gemm_mx.
+bool tile_mxb_ok(const ftm_moe_layer& L, int T) {
+  const int KP = L.topk + (L.shared_inter > 0 ? 1 : 0);
+  const int imax = L.inter > L.shared_inter ? L.inter : L.shared_inter;
+  return L.w2.fmt == FTM_FMT_FP8_BLOCK && (L.w2.flags & FTM_PROJ_RING_B) == 0 && L.inter % 128 == 0 &&
+         L.inter <= 128 * kXbSteps && (double)T * KP * mx_row_bytes(imax) < 4294967296.0;
+}
+
+static void launch_mxb(const LayerArgs& a, hipStream_t st) {
+  static bool attr = false;
+  tile_attr(&k_gemm_mxb_f8, attr);
+  hipLaunchKernelGGL(k_gemm_mxb_f8, dim3(tile_items<true>(a)), dim3(kBlock),
+                     (size_t)kXbSteps * kXStage + (size_t)kTM * 8u + (size_t)kTN * 4u, st, a);
+}
+
+void launch_tile_mx(const LayerArgs& a, hipStream_t st, int which) {
+  const bool f8 = a.L.w13.fmt == FTM_FMT_FP8_BLOCK;
+  if (which & 1) {
+    if (f8) launch_mx_s<FTM_FMT_FP8_BLOCK, false>(a, st);
+    else launch_mx_s<FTM_FMT_MXFP4, false>(a, st);
+  }
+  if (which & 2) {
+    if (f8 && tile_mxb_ok(a.L, a.T)) launch_mxb(a, st);
+    else if (f8) launch_mx_s<FTM_FMT_FP8_BLOCK, true>(a, st);
+    else launch_mx_s<FTM_FMT_MXFP4, true>(a, st);
+  }
 }
 
 }  // namespace ftm

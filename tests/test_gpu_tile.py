@@ -68,7 +68,7 @@ def test_gptq_tiles_match_oracle(gpu, T, H, I, shared, group):
     assert layer.stage_kernel(T, nat.STAGE_W2) == "k_tile"
 
 
-@pytest.mark.parametrize("name", ["c2_gptq"])
+@pytest.mark.parametrize("name", ["c2_gptq", "c3_fp8", "c4_mxfp4"])
 def test_tiles_with_uneven_experts(gpu, name):
     """Experts of 1, 15, 16, 17, 32, 33, 64, 65 and 129 rows, some of none."""
     T, E, k = 144, 16, 4
