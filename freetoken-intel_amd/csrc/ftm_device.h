@@ -232,18 +232,19 @@ __device__ __forceinline__ u32x4 fp8x8_to_bf16(uint32_t w0, uint32_t w1) {
 }
 
 // 8 offset-binary int8 bytes (value = byte - 128, compressed-tensors
-// pack-quantized, int8_packed_linear.py:74-93) -> 8 exact bf16 values.
-__device__ __forceinline__ uint32_t u8pair_to_bf16(uint32_t w, int hi) {
-  uint32_t b0 = (w >> (16 * hi)) & 0xffu, b1 = (w >> (16 * hi + 8)) & 0xffu;
-  return pack_bf16x2((float)b0 - 128.0f, (float)b1 - 128.0f);
+// pack-quantized, int8_packed_linear.py:74-93) -> 8 exact bf16 values: the
+// sign bits flipped, each signed byte converted in place (an SDWA convert) and
+// the upper halves of the floats paired (|v| <= 128 fits bf16's significand).
+__device__ __forceinline__ u32x2 i8x4_to_bf16(uint32_t w) {
+  const uint32_t a = w ^ 0x80808080u;
+  const float f0 = (float)(int8_t)a, f1 = (float)(int8_t)(a >> 8);
+  const float f2 = (float)(int8_t)(a >> 16), f3 = (float)((int)a >> 24);
+  return (u32x2){__builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u),
+                 __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u)};
 }
 __device__ __forceinline__ u32x4 i8x8_to_bf16(uint32_t w0, uint32_t w1) {
-  u32x4 r;
-  r.x = u8pair_to_bf16(w0, 0);
-  r.y = u8pair_to_bf16(w0, 1);
-  r.z = u8pair_to_bf16(w1, 0);
-  r.w = u8pair_to_bf16(w1, 1);
-  return r;
+  const u32x2 a = i8x4_to_bf16(w0), b = i8x4_to_bf16(w1);
+  return (u32x4){a.x, a.y, b.x, b.y};
 }
 
 // 8 e2m1 nibbles (one dword, low nibble = even element) scaled by the block's

@@ -1,14 +1,17 @@
-// ftm_gemm.hip -- the MoE expert stages above the token crossover: grouped,
-// LDS-tiled GEMMs on bf16 MFMA (v_mfma_f32_16x16x32_bf16).
+// ftm_gemm.hip -- the dispatch of the expert stages above the token crossover,
+// and the LDS-tiled bf16-MFMA GEMMs (v_mfma_f32_16x16x32_bf16) for the layers
+// the register-fed tiles (ftm_tile.hip) do not take: FP8 blocks other than
+// 128 x 128 with fp32 scales, FP8 with H or I not a multiple of 128, INT8 with
+// 64-wide groups.
 //
 // Below the crossover every expert sees a handful of tokens and the stages are
 // weight-streaming GEMVs (ftm_moe.hip).  Above it (prefill) each expert's
 // weights are reused by many tokens, so a tile of 64 tokens x 64 channels
 // loads its weights once per K step into LDS, decoded to bf16 exactly (FP8
-// e4m3 and INT8 codes are exact in bf16, MXFP4 e2m1 times its power-of-two
-// scale is exact), and four waves run 16x16x32 MFMAs out of LDS.  FP8 block
-// and INT8 group scales multiply the fp32 partial sums of each quantisation
-// group, as in the GEMV path, so both paths share one numerical contract.
+// e4m3 and INT8 codes are exact in bf16), and four waves run 16x16x32 MFMAs
+// out of LDS.  FP8 block and INT8 group scales multiply the fp32 partial sums
+// of each quantisation group, as in the GEMV path, so both paths share one
+// numerical contract.
 //
 // Tiles: the routed experts' token lists are cut into 64-row M tiles
 // (ascending compact expert index u), then the shared expert's tokens.  Stage
@@ -32,11 +35,11 @@ constexpr int kGemmMinRows = 16;
 // Weight bytes per element and 16-byte pieces per tile row per K step.
 template <int WFMT>
 struct GemmW {
-  static constexpr int kPieces = WFMT == FTM_FMT_BF16 ? 8 : WFMT == FTM_FMT_MXFP4 ? 2 : 4;
+  static constexpr int kPieces = WFMT == FTM_FMT_BF16 ? 8 : 4;
   static constexpr int kElems = kGK / kPieces;  // elements per piece
   static constexpr bool kPostScale = WFMT == FTM_FMT_FP8_BLOCK || WFMT == FTM_FMT_INT8_PACKED;
   __device__ static uint32_t row_bytes(int K) {
-    return WFMT == FTM_FMT_BF16 ? 2u * (uint32_t)K : WFMT == FTM_FMT_MXFP4 ? (uint32_t)K / 2 : (uint32_t)K;
+    return WFMT == FTM_FMT_BF16 ? 2u * (uint32_t)K : (uint32_t)K;
   }
 };
 
@@ -159,16 +162,6 @@ __device__ __forceinline__ void gemm_tile(const ProjSlot& W, int c0, int Iu, Rsr
     const int r = grow(wtr[i]);
     woff[i] = (c < R::kWPieces && r < W.N) ? (uint32_t)r * rb + (uint32_t)wpc[i] * 16u : kOOB;
   }
-  Rsrc sres = wres;  // MXFP4 e8m0 scales: one byte per (row, 32 elements)
-  uint32_t moff[R::kWLoads];
-  if constexpr (WFMT == FTM_FMT_MXFP4) {
-    sres = make_rsrc(W.s, (uint32_t)W.N * (uint32_t)(K / 32));
-#pragma unroll
-    for (int i = 0; i < R::kWLoads; ++i) {
-      const int r = grow(wtr[i]);
-      moff[i] = woff[i] != kOOB ? (uint32_t)(r * (K / 32) + wpc[i]) : kOOB;
-    }
-  }
   // post-scale sources: FP8 block rows (uniform per column block), INT8 rows (per lane)
   const int lpg = G::kPostScale ? W.group / kGK : 1;
   int srow[NB];
@@ -179,15 +172,10 @@ __device__ __forceinline__ void gemm_tile(const ProjSlot& W, int c0, int Iu, Rsr
   if constexpr (WFMT == FTM_FMT_INT8_PACKED) i8res = make_rsrc(W.s, (uint32_t)(W.N * (K / W.group)) * sesz);
 
   u32x4 rw[R::kWLoads], ra[2];
-  uint32_t rs[R::kWLoads];
   auto issue = [&](int kb) {
     const uint32_t kbyte = (uint32_t)kb * (uint32_t)(kGK * (WFMT == FTM_FMT_BF16 ? 2 : 1));
-    const uint32_t kbw = WFMT == FTM_FMT_MXFP4 ? kbyte / 2 : kbyte;
 #pragma unroll
-    for (int i = 0; i < R::kWLoads; ++i) {
-      rw[i] = bload16(wres, woff[i] != kOOB ? woff[i] + kbw : kOOB);
-      if constexpr (WFMT == FTM_FMT_MXFP4) rs[i] = bload1(sres, moff[i] != kOOB ? moff[i] + (uint32_t)(2 * kb) : kOOB);
-    }
+    for (int i = 0; i < R::kWLoads; ++i) rw[i] = bload16(wres, woff[i] != kOOB ? woff[i] + kbyte : kOOB);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int piece = (tid + kBlock * i) & 7;
@@ -212,12 +200,6 @@ __device__ __forceinline__ void gemm_tile(const ProjSlot& W, int c0, int Iu, Rsr
       } else if constexpr (WFMT == FTM_FMT_INT8_PACKED) {
         *(u32x4*)dst = i8x8_to_bf16(rw[i].x, rw[i].y);
         *(u32x4*)(dst + 8) = i8x8_to_bf16(rw[i].z, rw[i].w);
-      } else if constexpr (WFMT == FTM_FMT_MXFP4) {
-        const float sc = e8m0_to_f32(rs[i]);
-        *(u32x4*)dst = fp4x8_to_bf16(rw[i].x, sc);
-        *(u32x4*)(dst + 8) = fp4x8_to_bf16(rw[i].y, sc);
-        *(u32x4*)(dst + 16) = fp4x8_to_bf16(rw[i].z, sc);
-        *(u32x4*)(dst + 24) = fp4x8_to_bf16(rw[i].w, sc);
       } else {
         *(u32x4*)dst = rw[i];
       }
@@ -286,7 +268,7 @@ __device__ __forceinline__ void gemm_tile(const ProjSlot& W, int c0, int Iu, Rsr
 }
 
 // ---------------------------------------------------------------- LDS ring tiles (stage A)
-// The stage A tiles for FP8 / INT8 / MXFP4 / bf16 weights, fed by a ring of up to
+// The stage A tiles for FP8 / INT8 / bf16 weights, fed by a ring of up to
 // four LDS stages that direct global-to-LDS copies (global_load_lds, 16 B per
 // lane) fill three K steps ahead of the MFMAs.  Activations (bf16) and the raw
 // weight bytes both land in LDS undecoded; a wave decodes its own weight rows
@@ -301,7 +283,7 @@ __device__ __forceinline__ void gemm_tile(const ProjSlot& W, int c0, int Iu, Rsr
 // Raw weight bytes per row per K step and rows per 1 KiB copy.
 template <int WFMT>
 struct RingW {
-  static constexpr int kRowBytes = WFMT == FTM_FMT_BF16 ? 2 * kGK : WFMT == FTM_FMT_MXFP4 ? kGK / 2 : kGK;
+  static constexpr int kRowBytes = WFMT == FTM_FMT_BF16 ? 2 * kGK : kGK;
   static constexpr int kRowsPerCopy = 1024 / kRowBytes;
 };
 // Ring bytes per workgroup: 64 KiB (FP8/INT8: 4 stages, bf16: 2).  The
@@ -324,7 +306,6 @@ struct RingPlan {
 
 __device__ __forceinline__ int ring_fa(int r) { return (r ^ (r >> 3)) & 7; }         // 8 pieces per row
 __device__ __forceinline__ int ring_fw(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }  // 4 pieces per row
-__device__ __forceinline__ int ring_fm(int r) { return (r >> 3) & 1; }                // 2 pieces per row (MXFP4)
 
 // Wait until at most `stages` ring stages of this wave's copies are in flight.
 template <int LOADS, int MAXS>
@@ -379,9 +360,6 @@ __device__ __forceinline__ void gemm_tile_ring(const ProjSlot& W, int c0, int Iu
     if constexpr (WFMT == FTM_FMT_BF16) {
       r = 8 * j + (lane >> 3);
       piece = (lane & 7) ^ ring_fa(r);
-    } else if constexpr (WFMT == FTM_FMT_MXFP4) {
-      r = 32 * j + (lane >> 1);
-      piece = (lane & 1) ^ ring_fm(r);
     } else {
       r = 16 * j + (lane >> 2);
       piece = (lane & 3) ^ ring_fw(r);
@@ -404,24 +382,9 @@ __device__ __forceinline__ void gemm_tile_ring(const ProjSlot& W, int c0, int Iu
   // half, INT8: one row per tile row), loads issued before the ring prologue
   const int ngroups = kPost ? (K + W.group - 1) / W.group : 0;
   constexpr int kScaleRows = WFMT == FTM_FMT_INT8_PACKED ? NWR : NWR / 64;
-  constexpr int kScalePer = WFMT == FTM_FMT_INT8_PACKED || WFMT == FTM_FMT_MXFP4
-                                ? (kRingScaleBytes / 4 + kBlock - 1) / kBlock : 1;
+  constexpr int kScalePer = WFMT == FTM_FMT_INT8_PACKED ? (kRingScaleBytes / 4 + kBlock - 1) / kBlock : 1;
   uint32_t sw[kScalePer];
   uint32_t sidx[kScalePer];
-  // MXFP4: the e8m0 bytes [NWR rows][K / 32], copied as words; each 64-row
-  // half of the tile is one contiguous run of 64 * K / 32 bytes
-  const int kgb = K / 32;                 // scale bytes per row
-  const int mwords = 64 * kgb / 4;        // words per 64-row half
-  if constexpr (WFMT == FTM_FMT_MXFP4) {
-    const Rsrc mres = make_rsrc(W.s, (uint32_t)W.N * (uint32_t)kgb);
-#pragma unroll
-    for (int q = 0; q < kScalePer; ++q) {
-      const int e = tid + kBlock * q;
-      const int half = e / mwords, wi = e - half * mwords;
-      const bool ok = e < (NWR / 64) * mwords;
-      sw[q] = bload4(mres, ok ? (uint32_t)(grow(64 * half) * kgb + 4 * wi) : kOOB);
-    }
-  }
   if constexpr (kPost) {
     const uint32_t sesz = W.s_dt == FTM_DT_F32 ? 4u : 2u;
     const int nsc = kScaleRows * ngroups;
@@ -439,14 +402,6 @@ __device__ __forceinline__ void gemm_tile_ring(const ProjSlot& W, int c0, int Iu
   }
   const int pro = nsteps < S - 1 ? nsteps : S - 1;
   for (int kb = 0; kb < pro; ++kb) issue(kb, kb);
-  if constexpr (WFMT == FTM_FMT_MXFP4) {
-    wait_ring<P::kLoads, S - 1>(pro);
-#pragma unroll
-    for (int q = 0; q < kScalePer; ++q) {
-      const int e = tid + kBlock * q;
-      if (e < (NWR / 64) * mwords) ((uint32_t*)sS)[e] = sw[q];
-    }
-  }
   if constexpr (kPost) {
     wait_ring<P::kLoads, S - 1>(pro);
 #pragma unroll
@@ -477,12 +432,6 @@ __device__ __forceinline__ void gemm_tile_ring(const ProjSlot& W, int c0, int Iu
       if constexpr (WFMT == FTM_FMT_BF16) {
         b0[nj] = *(const u32x4*)(row + 16 * ((2 * g4) ^ ring_fa(wrr[nj])));
         b1[nj] = *(const u32x4*)(row + 16 * ((2 * g4 + 1) ^ ring_fa(wrr[nj])));
-      } else if constexpr (WFMT == FTM_FMT_MXFP4) {
-        // 16 e2m1 codes (K 16 g .. 16 g + 15), one 32-wide e8m0 group
-        const u32x2 raw = *(const u32x2*)(row + 16 * ((g4 >> 1) ^ ring_fm(wrr[nj])) + 8 * (g4 & 1));
-        const float sc = e8m0_to_f32(((const uint8_t*)sS)[wrr[nj] * kgb + 2 * kb + (g4 >> 1)]);
-        b0[nj] = fp4x8_to_bf16(raw.x, sc);
-        b1[nj] = fp4x8_to_bf16(raw.y, sc);
       } else {
         const u32x4 raw = *(const u32x4*)(row + 16 * (g4 ^ ring_fw(wrr[nj])));
         if constexpr (WFMT == FTM_FMT_FP8_BLOCK) {
@@ -670,7 +619,7 @@ template <int WFMT>
 __device__ __forceinline__ void ring_a(const LayerArgs& a, const ProjSlot& W, int Iu, int c0, int m0, int cnt,
                                        const int32_t* list, int shared_col, char* lds) {
   const int lpg = ring_lpg(WFMT, W.group, W.K);
-  if constexpr (WFMT == FTM_FMT_BF16 || WFMT == FTM_FMT_MXFP4) {  // no group post-scale
+  if constexpr (WFMT == FTM_FMT_BF16) {  // no group post-scale
     gemm_a_ring_body<WFMT, 0>(a, W, Iu, c0, m0, cnt, list, shared_col, lds);
   } else if constexpr (WFMT == FTM_FMT_FP8_BLOCK) {
     if (lpg == 2) gemm_a_ring_body<WFMT, 2>(a, W, Iu, c0, m0, cnt, list, shared_col, lds);
@@ -682,13 +631,12 @@ __device__ __forceinline__ void ring_a(const LayerArgs& a, const ProjSlot& W, in
   }
 }
 
-// SONLY: the shared expert's items only (its routed experts run elsewhere)
-template <int FMT, bool RING, bool SONLY = false>
+template <int FMT, bool RING>
 __device__ __forceinline__ void gemm_a_item(const LayerArgs& a, int item, uint16_t* sA, uint16_t* sB) {
   const int I = a.L.inter, Is = a.L.shared_inter;
   const int nRouted = a.ctrl[kCtrlNRouted];
   const int ntn = I / 64;
-  const int routed_items = SONLY ? 0 : gemm_routed_mtiles(a, nRouted) * ntn;
+  const int routed_items = gemm_routed_mtiles(a, nRouted) * ntn;
   if (item < routed_items) {
     const GemmTile t = gemm_find_tile(a, item / ntn, nRouted, false);
     if (t.u < 0) return;
@@ -726,9 +674,9 @@ extern __shared__ __attribute__((aligned(16))) uint16_t ftm_ring_lds[];
 
 // The ring tiles (dynamic LDS: ring + the layer's tile scales), items in
 // XCD-aware order.
-template <int FMT, bool SONLY = false>
+template <int FMT>
 __global__ __launch_bounds__(kBlock) void k_gemm_a_ring(const LayerArgs a) {
-  gemm_a_item<FMT, true, SONLY>(a, xcd_item(blockIdx.x, gridDim.x), ftm_ring_lds, nullptr);
+  gemm_a_item<FMT, true>(a, xcd_item(blockIdx.x, gridDim.x), ftm_ring_lds, nullptr);
 }
 
 // ---------------------------------------------------------------- stage B (w2 -> slot buffer)
@@ -785,12 +733,12 @@ __device__ void gemm_b_body(const LayerArgs& a, const ProjSlot& W, int n0, int m
     }
 }
 
-template <int FMT, bool SONLY = false>
+template <int FMT>
 __device__ __forceinline__ void gemm_b_item(const LayerArgs& a, int item, uint16_t* sA, uint16_t* sB) {
   const int H = a.L.hidden, Is = a.L.shared_inter;
   const int nRouted = a.ctrl[kCtrlNRouted];
   const int ntn = H / 64;
-  const int routed_items = SONLY ? 0 : gemm_routed_mtiles(a, nRouted) * ntn;
+  const int routed_items = gemm_routed_mtiles(a, nRouted) * ntn;
   if (item < routed_items) {
     const GemmTile t = gemm_find_tile(a, item / ntn, nRouted, false);
     if (t.u < 0) return;
@@ -818,11 +766,11 @@ __device__ __forceinline__ void gemm_b_item(const LayerArgs& a, int item, uint16
   }
 }
 
-template <int FMT, bool SONLY = false>
+template <int FMT>
 __global__ __launch_bounds__(kBlock) void k_gemm_b(const LayerArgs a) {
   __shared__ __attribute__((aligned(16))) uint16_t sA[2 * kGM * kGPitch];
   __shared__ __attribute__((aligned(16))) uint16_t sB[2 * 64 * kGPitch];
-  gemm_b_item<FMT, SONLY>(a, blockIdx.x, sA, sB);
+  gemm_b_item<FMT>(a, blockIdx.x, sA, sB);
 }
 
 // ---------------------------------------------------------------- launch
@@ -845,11 +793,9 @@ bool gemm_path_ok(const ftm_moe_layer& L, int T) {
 }
 
 // Whether the ring tiles take this layer: weights whose tile scales fit the
-// LDS scale area (INT8: one fp32 per tile row and group; MXFP4: one e8m0 byte
-// per tile row and 32 K).
+// LDS scale area (INT8: one fp32 per tile row and group).
 static bool ring_ok(const ftm_moe_layer& L) {
   const int f = L.w13.fmt;
-  if (f == FTM_FMT_MXFP4 && 128 * (L.hidden / 32) > kRingScaleBytes) return false;  // e8m0 bytes of the tile
   if (f == FTM_FMT_INT8_PACKED || f == FTM_FMT_FP8_BLOCK) {
     const long g13 = (L.hidden + L.w13.group - 1) / L.w13.group;
     if (f == FTM_FMT_INT8_PACKED && 128 * g13 * 4 > kRingScaleBytes) return false;
@@ -861,7 +807,6 @@ static bool ring_ok(const ftm_moe_layer& L) {
 // Dynamic LDS of the ring kernels for this layer: ring + tile scales.
 static size_t ring_lds_a(const ftm_moe_layer& L) {
   const int f = L.w13.fmt;
-  if (f == FTM_FMT_MXFP4) return (size_t)kRingA + 128u * (size_t)(L.hidden / 32);
   const int g = (L.hidden + L.w13.group - 1) / (L.w13.group > 0 ? L.w13.group : 1);
   const int rows = f == FTM_FMT_FP8_BLOCK ? 2 : f == FTM_FMT_INT8_PACKED ? 128 : 0;
   return (size_t)kRingA + (size_t)rows * g * 4;
@@ -869,47 +814,38 @@ static size_t ring_lds_a(const ftm_moe_layer& L) {
 bool mx_gemm_ok(const ftm_moe_layer& L) { return mx_fmt(L); }
 
 const char* gemm_a_kernel_name(const ftm_moe_layer& L) {
-  return L.w13.fmt == FTM_FMT_GPTQ_INT4 ? "k_tile" : mx_gemm_ok(L) ? "k_gemm_mx" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
+  return mx_gemm_ok(L) ? "k_gemm_mx" : tile_bf16_ok(L) ? "k_tile" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
 }
 
-template <int FMT, bool SONLY = false>
+template <int FMT>
 static void ring_lds_attr() {
   static bool done = false;  // once per instantiation (setting it twice is harmless)
   if (!done) {
     // a failure here surfaces as the launch error that follows
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_a_ring<FMT, SONLY>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_a_ring<FMT>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, kRingA + kRingScaleBytes);
     done = true;
   }
 }
 
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T) {
-  if (L.w13.fmt == FTM_FMT_GPTQ_INT4) return "k_tile";
+  if (tile_bf16_ok(L)) return "k_tile";
   if (!mx_gemm_ok(L)) return "k_gemm_b";
   return tile_mxb_ok(L, T) ? "k_gemm_mxb_f8" : "k_gemm_mx";
 }
 
 template <int FMT>
-static void launch_gemm_t(const LayerArgs& a, hipStream_t st, int which, bool xq_ready) {
+static void launch_gemm_t(const LayerArgs& a, hipStream_t st, int which) {
   const ftm_moe_layer& L = a.L;
   const long pairs = (long)a.T * L.topk;
   const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
-  if constexpr (FMT == FTM_FMT_MXFP4 || FMT == FTM_FMT_FP8_BLOCK) {
-    if (mx_gemm_ok(L)) {
-      // both stages on the scaled-MFMA tiles: stage A over the quantised
-      // input, writing h quantised the same way for stage B
-      if ((which & 1) && !xq_ready) launch_quant_mx(a.x, a.T, L.hidden, a.xq, st);
-      launch_tile_mx(a, st, which);
-      return;
-    }
-  }
   const long mt_routed = pairs / kGM + maxU + 1;
   const long mt_shared = L.shared_inter > 0 ? (a.T + kGM - 1) / kGM : 0;
   const long items_a = mt_routed * (L.inter / 64) + mt_shared * (L.shared_inter > 0 ? L.shared_inter / 64 : 0);
   const long items_b = (mt_routed + mt_shared) * (L.hidden / 64);
   // Stage A on the ring tiles where they apply (measured on MI355X, C3 FP8:
   // w13 285 us against 343 at T=2048, 179 against 239 at T=512; C1 INT8 T=1024:
-  // 29 against 42; C4 MXFP4 T=4096: 1045 against 1415).  Stage B keeps the register-staged tiles: with K = I its
+  // 29 against 42).  Stage B keeps the register-staged tiles: with K = I its
   // tiles are 8 K steps long and 4 workgroups per CU beat the deeper ring
   // (C3 T=2048 w2 259 us against 377).
   const bool ring = ring_ok(L);
@@ -927,13 +863,18 @@ static void launch_gemm_t(const LayerArgs& a, hipStream_t st, int which, bool xq
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready) {
   const LayerArgs a = make_args(L, x, out, T, ws, wl);
-  switch (L.w13.fmt) {
-    case FTM_FMT_GPTQ_INT4: launch_tile_gptq(a, st, which); break;
-    case FTM_FMT_FP8_BLOCK: launch_gemm_t<FTM_FMT_FP8_BLOCK>(a, st, which, xq_ready); break;
-    case FTM_FMT_INT8_PACKED: launch_gemm_t<FTM_FMT_INT8_PACKED>(a, st, which, xq_ready); break;
-    case FTM_FMT_MXFP4: launch_gemm_t<FTM_FMT_MXFP4>(a, st, which, xq_ready); break;
-    default: launch_gemm_t<FTM_FMT_BF16>(a, st, which, xq_ready); break;
+  if (mx_gemm_ok(L)) {
+    // stage A over the quantised input, writing h quantised the same way for stage B
+    if ((which & 1) && !xq_ready) launch_quant_mx(x, T, L.hidden, a.xq, st);
+    launch_tile_mx(a, st, which);
+    return;
   }
+  if (tile_bf16_ok(L)) {
+    launch_tile_bf16(a, st, which);
+    return;
+  }
+  if (L.w13.fmt == FTM_FMT_FP8_BLOCK) launch_gemm_t<FTM_FMT_FP8_BLOCK>(a, st, which);
+  else launch_gemm_t<FTM_FMT_INT8_PACKED>(a, st, which);
 }
 
 }  // namespace ftm

@@ -73,12 +73,18 @@ constexpr int kMaxColTiles = FTM_WS_CTRL_BYTES / 4 - kCtrlTileCnt;
 // size are zeros).
 constexpr int kMxChunk = 272;
 __host__ __device__ inline int mx_row_bytes(int H) { return (H + 127) / 128 * kMxChunk; }
-// Weight formats the scaled-MFMA stages take (bf16 activations): MXFP4, and
-// FP8 e4m3 with 128 x 128 blocks (the block scale applied to each K step's
+// An internal flag of w13 (ftm_proj.flags): no tiles, so no quantised copies in
+// the workspace (ftm_moe_forward_noalloc, where they would not fit its scratch).
+constexpr int kProjNoTiles = 1 << 30;
+bool tile_gptq_ok(const ftm_moe_layer& L);  // GPTQ layers the scaled-MFMA tiles take (ftm_tile.hip)
+bool gemm_path_ok(const ftm_moe_layer& L, int T);
+// Weight formats the scaled-MFMA stages take (bf16 activations): MXFP4, GPTQ
+// with 128-wide groups, and FP8 e4m3 with 128 x 128 blocks (the block scale applied to each K step's
 // partial sums).
 inline bool mx_fmt(const ftm_moe_layer& L) {
   if (L.act_dtype != FTM_DT_BF16) return false;
   if (L.w13.fmt == FTM_FMT_MXFP4) return true;
+  if (L.w13.fmt == FTM_FMT_GPTQ_INT4) return tile_gptq_ok(L);
   return L.w13.fmt == FTM_FMT_FP8_BLOCK && L.w13.group == 128 && L.w2.group == 128 &&
          L.w13.s_dtype == FTM_DT_F32 && L.w2.s_dtype == FTM_DT_F32 && L.hidden % 128 == 0 && L.inter % 128 == 0;
 }
@@ -110,8 +116,9 @@ inline WsLayout ws_layout(const ftm_moe_layer& L, int T) {
   w.hbuf = o;   o = align_up(o + act * Tt * w.KP * w.Imax, 256);
   w.ybuf = o;   o = align_up(o + 4 * Tt * w.KP * (size_t)L.hidden, 256);
   // layers the scaled-MFMA stages take: the input and h quantised (kMxChunk
-  // layout, by token and by pair)
-  const bool mx = mx_fmt(L);
+  // layout, by token and by pair); GPTQ: above the crossover only (its decode
+  // stages read the bf16 input)
+  const bool mx = mx_fmt(L) && (L.w13.fmt != FTM_FMT_GPTQ_INT4 || gemm_path_ok(L, T));
   w.hq = o;     o = align_up(o + (mx ? Tt * w.KP * (size_t)mx_row_bytes(w.Imax) : 0), 256);
   w.xq = o;     o = align_up(o + (mx ? Tt * (size_t)mx_row_bytes(L.hidden) : 0), 256);
   w.total = o;
@@ -146,13 +153,12 @@ bool mx_stage_a(const ftm_moe_layer& L, int T);
 bool mx_input(const ftm_moe_layer& L, int T);
 // Prefill side of the crossover (ftm_gemm.hip): whether the tiled GEMM stages
 // take this layer at T tokens, and their launch (which: bit 0 = w13, bit 1 = w2).
-bool gemm_path_ok(const ftm_moe_layer& L, int T);
 const char* gemm_a_kernel_name(const ftm_moe_layer& L);  // the stage A tile kernel the layer takes
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T);  // the stage B tile kernel at T tokens
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready = false);
-// GPTQ layers whose expert stages the register-fed tiles take (ftm_tile.hip).
-bool tile_gptq_ok(const ftm_moe_layer& L);
+// INT8 and bf16 layers the bf16 tiles take above the crossover (ftm_tile.hip).
+bool tile_bf16_ok(const ftm_moe_layer& L);
 // FP8 stage B above the crossover on k_gemm_mxb_f8 (else k_gemm_mx).
 bool tile_mxb_ok(const ftm_moe_layer& L, int T);
 // MXFP4 stage A on the scaled-MFMA tiles (k_gemm_a_mx) above the crossover.

@@ -63,11 +63,11 @@ inline LayerArgs make_args(const ftm_moe_layer& L, const void* x, void* out, int
   return a;
 }
 
-// The expert stages of a GPTQ layer on the register-fed tiles (ftm_tile.hip);
-// which: bit 0 = w13, bit 1 = w2.
-void launch_tile_gptq(const LayerArgs& a, hipStream_t st, int which);
-// ... and of an MXFP4 or FP8 (128 x 128 blocks) layer on the scaled MFMAs, over the quantised input.
+// The expert stages above the crossover on the register-fed tiles
+// (ftm_tile.hip; which: bit 0 = w13, bit 1 = w2): the scaled-MFMA ones over
+// the quantised input (mx_fmt layers), the bf16 ones (tile_bf16_ok).
 void launch_tile_mx(const LayerArgs& a, hipStream_t st, int which);
+void launch_tile_bf16(const LayerArgs& a, hipStream_t st, int which);
 
 // Pair slot p of row m of an expert's token list (the shared expert has no
 // list: its rows are the tokens, p = m*KP + shared_col), or -1 past cnt.

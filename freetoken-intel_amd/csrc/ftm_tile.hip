@@ -29,21 +29,20 @@ namespace ftm {
 constexpr int kTM = 64;        // rows (pairs) per tile
 constexpr int kTN = 256;       // weight rows per tile
 constexpr int kTHPitch = 128 * 2 + 16;  // bytes of a staged h row (stage A's epilogue, 128 channels)
-constexpr int kTStages = 2;    // activation stages in LDS
+constexpr int kTStages = 3;    // activation stages in LDS
 
-// How group scales enter: none (bf16; MXFP4's ride in the decode), one group
-// over K (applied after the loop), one per K step of 128, one per 64.
-enum { kScaleNone = 0, kScaleOne = 1, kScale128 = 2, kScale64 = 3 };
+// How group scales enter: none (bf16), one group over K (applied after the
+// loop), one per K step of 128.
+enum { kScaleNone = 0, kScaleOne = 1, kScale128 = 2 };
 
 template <int FMT>
 struct TileFmt {
-  static constexpr int kKS = FMT == FTM_FMT_BF16 ? 64 : 128;                        // K per step
-  static constexpr int kNL = FMT == FTM_FMT_MXFP4 ? 1 : 2;                          // 16-byte loads per row and step
-  static constexpr int kARow = 2 * kKS;                                             // activation bytes per row and step
+  static constexpr int kKS = FMT == FTM_FMT_BF16 ? 64 : 128;  // K per step
+  static constexpr int kSub = kKS / 32;                       // MFMA sub-steps
+  static constexpr int kARow = 2 * kKS;                       // activation bytes per row and step
   static constexpr int kStage = kTM * kARow;
-  static constexpr int kACopies = kStage / 1024 / 4;                                // 16-byte pieces per thread and step
+  static constexpr int kACopies = kStage / 1024 / 4;          // 1 KiB copies per wave and step
   static constexpr int kRing = kTStages * kStage > kTM * kTHPitch ? kTStages * kStage : kTM * kTHPitch;
-  static constexpr bool kPost = FMT == FTM_FMT_FP8_BLOCK || FMT == FTM_FMT_INT8_PACKED || FMT == FTM_FMT_GPTQ_INT4;
 };
 
 // Activation slot swizzle: slot s of row r holds 16-byte piece s ^ tile_fa(r)
@@ -57,34 +56,8 @@ __device__ __forceinline__ int tile_fa(int r) {
 // column m, of a wave whose first rows are base[0] (nj 0, 1) and base[1] (2,
 // 3): two neighbouring rows a lane (GPTQ: one 8-byte load of two columns), so
 // that a lane's results are neighbours too.
-template <int FMT>
 __device__ __forceinline__ int tile_row(const int (&base)[2], int nj, int m) {
   return base[nj >> 1] + 2 * m + (nj & 1);
-}
-
-// One step's packed weights of a wave and the raw words of its scales.
-template <int FMT>
-struct TileW {
-  u32x4 w[4][TileFmt<FMT>::kNL];
-  uint32_t s[2][4];  // FP8: [half-step][0 / 2]; INT8: [half-step][nj]; MXFP4: [0][nj], the lane's e8m0 byte
-};
-template <>
-struct TileW<FTM_FMT_GPTQ_INT4> {
-  u32x2 w[2][4];  // [half][q]: the words of columns 2m, 2m + 1 at K 32 q + 8 g
-  uint32_t s[2];  // [half]: both columns' 16-bit scales
-};
-
-// Eight nibbles (low first) -> bf16 values q in natural order.
-__device__ __forceinline__ u32x4 gptq_word_natural(uint32_t w) {
-  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;  // q0 q2 q4 q6 / q1 q3 q5 q7
-  const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x05010400u);     // q0 q1 q2 q3
-  const uint32_t b = __builtin_amdgcn_perm(hi, lo, 0x07030602u);     // q4 q5 q6 q7
-  u32x4 r;
-  r.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)a, 512.0f, false));
-  r.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)a, 512.0f, true));
-  r.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)b, 512.0f, false));
-  r.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)b, 512.0f, true));
-  return r;
 }
 
 // 16-bit scale word `hi` (0 / 1) of a pair -> its value (branch-free).
@@ -94,261 +67,217 @@ __device__ __forceinline__ float half_word(uint32_t w, int hi, int dt) {
   return dt == FTM_DT_F16 ? f : b;
 }
 
-// The K loop: acc += A (16 MI rows) . W^T over the whole K.
-//   arow[i]: start of the activation row of this thread's piece i
-//   lds: two activation stages; Xs: GPTQ row sums [kTM][K / 128 + 1]
+// Activation sources of a wave's copies: byte offsets into the buffer (BIG:
+// addresses).
+template <int N>
+struct TileSrc {
+  uint64_t p[N];
+};
+
+// The K loop of the bf16 tiles: acc += A (16 MI rows) . W^T over the whole K.
 // Every step issues the same loads (past the last step through clamped or
-// out-of-range offsets), so the compiler's counted waits are exact.
-template <int FMT, int MODE, int MI>
-__device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[2],
-                                           const char* const (&arow)[TileFmt<FMT>::kACopies], char* lds, float* Xs,
-                                           f32x4 (&acc)[MI][4]) {
+// out-of-range offsets), so the counted waits are exact.
+template <int FMT, int MODE, int MI, bool BIG>
+__device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[2], const char* abase, uint32_t abytes,
+                                           const TileSrc<TileFmt<FMT>::kACopies>& src, char* lds, f32x4 (&acc)[MI][4]) {
   using F = TileFmt<FMT>;
-  constexpr bool GQ = FMT == FTM_FMT_GPTQ_INT4;
-  constexpr bool POST = MODE == kScale128 || MODE == kScale64;  // partial sums per step (or half step)
-  constexpr int KS = F::kKS;
+  constexpr bool I8 = FMT == FTM_FMT_INT8_PACKED;
+  constexpr int KS = F::kKS, NA = F::kACopies;
+  constexpr int NW = 8 + (MODE == kScale128 ? 4 : 0);  // weight and scale loads a step
+  typedef __attribute__((address_space(1))) const void* GPtr;
+  typedef __attribute__((address_space(3))) void* LPtr;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, m = lane & 15;
   const int K = W.K, N = W.N;
   const int nsteps = (K + KS - 1) / KS;
 
-  // ---- activations: 16-byte pieces of the step's rows, one step ahead in
-  // registers, then to LDS.  A piece past K re-reads one of the row's first
-  // 64 elements (multiplied by zero weights, or skipped).
-  constexpr int NA = F::kACopies, kPer = F::kARow / 16;
-  // piece i is row (kBlock / kPer) i + tid / kPer: the swizzle is the same for every i
-  const uint32_t aslot = (uint32_t)((tid / kPer) * F::kARow + 16 * ((tid % kPer) ^ tile_fa<FMT>(tid / kPer)));
-  auto load_a = [&](int kb, u32x4 (&t)[NA]) {
-    uint32_t off = (uint32_t)(kb < nsteps ? kb : nsteps - 1) * (uint32_t)F::kARow + 16u * (uint32_t)(tid % kPer);
-    if (KS == 128) off = off < 2u * (uint32_t)K ? off : off & 127u;
+  // a last half step's copies read past the row (another row, or zeros past
+  // the buffer): nothing uses them
+  const Rsrc ares = make_rsrc(abase, abytes);
+  auto issue_a = [&](int kb, int slot) {
+    const uint32_t ko = (uint32_t)(kb < nsteps ? kb : nsteps - 1) * (uint32_t)F::kARow;
 #pragma unroll
-    for (int i = 0; i < NA; ++i) t[i] = *(const u32x4*)(arow[i] + off);
-  };
-  auto store_a = [&](const u32x4 (&t)[NA], char* st) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) *(u32x4*)(st + aslot + i * (kBlock / kPer) * F::kARow) = t[i];
+    for (int i = 0; i < NA; ++i) {
+      char* dst = lds + slot * F::kStage + 1024 * (wave * NA + i);
+      if constexpr (BIG) {
+        // the piece's K must exist: an address has no range check
+        const uint32_t pc = (uint32_t)((lane % (F::kARow / 16)) ^ tile_fa<FMT>((64 * (wave * NA + i) + lane) / (F::kARow / 16)));
+        const uint32_t over = KS == 128 && ko + 16u * pc >= 2u * (uint32_t)K ? 128u : 0u;
+        __builtin_amdgcn_global_load_lds((GPtr)(src.p[i] + ko - over), (LPtr)dst, 16, 0, 0);
+      } else {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ares, (LPtr)dst, 16, (int)((uint32_t)src.p[i] + ko), 0, 0, 0);
+      }
+    }
   };
 
-  // ---- weights and scales
-  const uint32_t rb = FMT == FTM_FMT_BF16 ? 2u * (uint32_t)K : FMT == FTM_FMT_MXFP4 ? (uint32_t)K / 2 : (uint32_t)K;
-  const Rsrc wres = make_rsrc(W.w, GQ ? (uint32_t)(K / 8) * (uint32_t)N * 4u : rb * (uint32_t)N);
+  struct Wgt {
+    u32x4 w[4][2];
+    uint32_t s[4];
+  };
+  const uint32_t rb = I8 ? (uint32_t)K : 2u * (uint32_t)K;
+  const Rsrc wres = make_rsrc(W.w, rb * (uint32_t)N);
   const uint32_t sesz = W.s_dt == FTM_DT_F32 ? 4u : 2u;
-  const int ngrp = F::kPost ? (K + W.group - 1) / W.group : 0;
-  const Rsrc sres = make_rsrc(W.s, FMT == FTM_FMT_FP8_BLOCK ? (uint32_t)(((N + W.group - 1) / W.group) * ngrp) * sesz
-                              : FMT == FTM_FMT_MXFP4        ? (uint32_t)N * (uint32_t)(K / 32)
-                              : F::kPost                    ? (uint32_t)(N * ngrp) * sesz
-                                                            : 0u);
-  uint32_t woff[4], soff[4];
+  const int ngrp = I8 ? K / W.group : 0;
+  const Rsrc sres = make_rsrc(W.s, (uint32_t)(N * ngrp) * sesz);
+  uint32_t woff[4];
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) {
-    const int row = tile_row<FMT>(base, nj, m);
-    soff[nj] = kOOB;
-    if constexpr (GQ) {  // nj 0 and 2: the halves
-      woff[nj] = row < N ? ((uint32_t)g * (uint32_t)N + (uint32_t)row) * 4u : kOOB;
-      soff[nj] = row < N ? 2u * (uint32_t)row : kOOB;
-    } else {
-      woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
-      if constexpr (FMT == FTM_FMT_FP8_BLOCK) soff[nj] = sesz * (uint32_t)((base[nj >> 1] / W.group) * ngrp);
-      if constexpr (FMT == FTM_FMT_INT8_PACKED) soff[nj] = row < N ? sesz * (uint32_t)(row * ngrp) : kOOB;
-      if constexpr (FMT == FTM_FMT_MXFP4)
-        soff[nj] = row < N ? (uint32_t)row * (uint32_t)(K / 32) + (uint32_t)g : kOOB;
-    }
+    const int row = tile_row(base, nj, m);
+    woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
   }
-  // piece i of step kb's weights: 64 bytes of each row (GPTQ: half i)
-  auto load_w = [&](int kb, int i, TileW<FMT>& t) {
-    if constexpr (GQ) {
-      const uint32_t o = woff[2 * i] + (kb < nsteps ? (uint32_t)kb * 64u * (uint32_t)N : kOOB);
+  // index of the scale of block nj in step kb (rows past N: past the end)
+  auto sidx = [&](int kb, int nj) {
+    return (uint32_t)(tile_row(base, nj, m) * ngrp) + (MODE == kScaleOne ? 0u : (uint32_t)(kb * 128 / W.group));
+  };
+  auto load_s = [&](int kb, Wgt& t) {
+    if constexpr (MODE == kScale128) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        t.w[i][q] = __builtin_amdgcn_raw_buffer_load_b64(wres, o, 16u * (uint32_t)N * (uint32_t)q, 0);
+      for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload4(sres, (sesz * sidx(kb < nsteps ? kb : 0, nj)) & ~3u);
+    }
+  };
+  auto load_w = [&](int kb, int i, Wgt& t) {  // 64 bytes of each row
+    const uint32_t ko = kb * KS + (I8 ? 64 : 32) * i < K ? (uint32_t)kb * 128u + 64u * (uint32_t)i : kOOB;
+#pragma unroll
+    for (int nj = 0; nj < 4; ++nj) t.w[nj][i] = bload16(wres, woff[nj] + ko);
+  };
+
+  // kScale128 holds one register set beside its partial sums: cur and nxt are
+  // the same, a piece is requested again as soon as its last MFMA has read it
+  auto step = [&](int kb, int slot, Wgt& cur, Wgt& nxt) {
+    // the copies of stage kb have landed (younger: this step's weights, the
+    // copies of stage kb + 1), then every wave's have, and every wave is done
+    // reading stage kb - 1
+    wait_vm<NW + NA>();
+    asm volatile("s_barrier" ::: "memory");
+    issue_a(kb + 2, slot == 0 ? 2 : slot - 1);
+    uint32_t sw[4];
+    if constexpr (MODE == kScale128) {
+#pragma unroll
+      for (int nj = 0; nj < 4; ++nj) sw[nj] = cur.s[nj];
+      load_s(kb + 1, nxt);
     } else {
-      constexpr uint32_t kStep = FMT == FTM_FMT_MXFP4 ? 64u : 128u;
-      const int k0 = FMT == FTM_FMT_MXFP4 ? kb * KS + 32 * g : FMT == FTM_FMT_BF16 ? kb * KS + 32 * i : kb * KS + 64 * i;
-      const uint32_t ko = k0 < K ? (uint32_t)kb * kStep + 64u * (uint32_t)i : kOOB;
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj) t.w[nj][i] = bload16(wres, woff[nj] + ko);
+      load_w(kb + 1, 0, nxt);
+      load_w(kb + 1, 1, nxt);
     }
-  };
-  // byte offset of the scale of half-step i of step kb within its row
-  auto sgrp = [&](int kb, int i) { return sesz * (uint32_t)((kb * 128 + 64 * i) / W.group); };
-  auto load_s = [&](int kb, TileW<FMT>& t) {
-    if constexpr (GQ) {
-      const uint32_t go = kb < nsteps ? 2u * (uint32_t)(kb * 128 / W.group) * (uint32_t)N : kOOB;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) t.s[h] = bload4(sres, soff[2 * h] + go);
-    } else if constexpr (FMT == FTM_FMT_MXFP4) {
-      const uint32_t go = kb * KS + 32 * g < K ? 4u * (uint32_t)kb : kOOB;
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj) t.s[0][nj] = bload1(sres, soff[nj] + go);
-    } else if constexpr (POST) {
-#pragma unroll
-      for (int i = 0; i < (MODE == kScale64 ? 2 : 1); ++i) {
-        const uint32_t go = kb * KS + 64 * i < K ? sgrp(kb, i) : kOOB;
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj)
-          if (FMT == FTM_FMT_INT8_PACKED || (nj & 1) == 0) t.s[i][nj] = bload4(sres, (soff[nj] + go) & ~3u);
-      }
-    }
-  };
-
-  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-  auto afrag = [&](const char* st, int blk, int piece) {
-    const int r = 16 * blk + m;
-    return *(const u32x4*)(st + r * F::kARow + 16 * (piece ^ tile_fa<FMT>(r)));
-  };
-
-  // One K step: its weights in cur, the next step's loads into nxt and ra
-  // first, so that they are in flight during the MFMAs.
-  auto step = [&](int kb, const TileW<FMT>& cur, TileW<FMT>& nxt) {
-    // stage kb is in LDS for every wave, and every wave is done with kb - 1
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    u32x4 ra[NA];
-    load_a(kb + 1, ra);
-    load_s(kb + 1, nxt);
-#pragma unroll
-    for (int i = 0; i < F::kNL; ++i) load_w(kb + 1, i, nxt);
     __builtin_amdgcn_sched_barrier(0);
-    const char* st = lds + (kb & 1) * F::kStage;
-    f32x4 p[MI][4], x = {0.f, 0.f, 0.f, 0.f};
+    const char* st = lds + slot * F::kStage;
+    f32x4 p[MODE == kScale128 ? MI : 1][4];
 #pragma unroll
-    for (int mi = 0; mi < MI; ++mi)
+    for (auto& r : p)
 #pragma unroll
-      for (int nj = 0; nj < 4; ++nj) p[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    f32x4(&d)[MI][4] = POST ? p : acc;
-    // one 32-wide sub-step: B operands bq against activation piece `piece` of every row
-    auto mma = [&](int piece, const u32x4(&bq)[4]) {
+      for (int nj = 0; nj < 4; ++nj) r[nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // sub-step q's operand: activation piece 4 q + g (INT8: 8 (q / 2) + 2 g +
+    // q % 2, the 16 K of a lane's weight bytes); read during the MFMAs of the
+    // sub-step before
+    auto frag = [&](int q, u32x4(&a)[MI]) {
+      const int piece = I8 ? 8 * (q >> 1) + 2 * g + (q & 1) : 4 * q + g;
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) {
-        const u32x4 af = afrag(st, mi, piece);
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj) d[mi][nj] = mfma_bf16(af, bq[nj], d[mi][nj]);
+        const int r = 16 * mi + m;
+        a[mi] = *(const u32x4*)(st + r * F::kARow + 16 * (piece ^ tile_fa<FMT>(r)));
       }
-      if constexpr (GQ) x = mfma_bf16(afrag(st, wave, piece), ones, x);
     };
-    // the partial sums of the step (kScale64: of half-step i) join acc
-    auto fold = [&](int i, const auto& t) {
+    auto mma = [&](int q, const u32x4(&a)[MI]) {
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) {
-        const int sj = FMT == FTM_FMT_INT8_PACKED ? nj : nj & 2;
-        const float s = decode_scalar_word(t.s[i][sj], (soff[sj] + sgrp(kb, i)) / sesz, W.s_dt);
+        u32x4 b;
+        if constexpr (I8) {
+          const u32x4 r = cur.w[nj][q >> 1];
+          b = i8x8_to_bf16(q & 1 ? r.z : r.x, q & 1 ? r.w : r.y);
+        } else {
+          b = cur.w[nj][q];
+        }
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) {
-          acc[mi][nj] += p[mi][nj] * s;
-          p[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          f32x4& d = MODE == kScale128 ? p[mi][nj] : acc[mi][nj];
+          d = mfma_bf16(a[mi], b, d);
         }
       }
     };
-    if constexpr (GQ) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        u32x4 bq[4];
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj)
-          bq[nj] = gptq_word_natural((nj & 1) ? cur.w[nj >> 1][q].y : cur.w[nj >> 1][q].x);
-        mma(4 * q + g, bq);
+    u32x4 a0[MI], a1[MI];
+    frag(0, a0);
+    if constexpr (MODE == kScale128) {
+      frag(1, a1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(0, a0);
+      frag(2, a0);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(1, a1);
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(kb + 1, 0, nxt);
+      if (kb * 128 + 64 < K) {
+        frag(3, a1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(2, a0);
+        mma(3, a1);
       }
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj) {
-        const float s = half_word(cur.s[nj >> 1], nj & 1, W.s_dt);
-#pragma unroll
-        for (int mi = 0; mi < MI; ++mi) acc[mi][nj] += p[mi][nj] * s;
-      }
-      if (m == 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Xs[(16 * wave + 4 * g + r) * (nsteps + 1) + kb] = x[r];
-      }
-    } else if constexpr (FMT == FTM_FMT_MXFP4) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        u32x4 bq[4];
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj) {
-          const u32x4 r = cur.w[nj][0];
-          bq[nj] = fp4x8_to_bf16(q == 0 ? r.x : q == 1 ? r.y : q == 2 ? r.z : r.w, e8m0_to_f32(cur.s[0][nj]));
-        }
-        mma(4 * g + q, bq);
-      }
-    } else if constexpr (FMT == FTM_FMT_BF16) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        u32x4 bq[4];
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj) bq[nj] = cur.w[nj][i];
-        mma(4 * i + g, bq);
+      __builtin_amdgcn_sched_barrier(0);
+      load_w(kb + 1, 1, nxt);
+    } else if constexpr (I8) {
+      // INT8: K may end in a half step, whose zero bytes would decode to -128
+      frag(1, a1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(0, a0);
+      frag(2, a0);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(1, a1);
+      if (kb * 128 + 64 < K) {
+        frag(3, a1);
+        __builtin_amdgcn_sched_barrier(0);
+        mma(2, a0);
+        mma(3, a1);
       }
     } else {
+      frag(1, a1);
+      __builtin_amdgcn_sched_barrier(0);
+      mma(0, a0);
+      mma(1, a1);
+    }
+    if constexpr (MODE == kScale128) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (i == 0 || kb * 128 + 64 < K) {
+      for (int nj = 0; nj < 4; ++nj) {
+        const float sv = decode_scalar_word(sw[nj], sidx(kb, nj), W.s_dt);
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            u32x4 bq[4];
-#pragma unroll
-            for (int nj = 0; nj < 4; ++nj) {
-              const u32x4 r = cur.w[nj][i];
-              bq[nj] = FMT == FTM_FMT_FP8_BLOCK ? fp8x8_to_bf16(h ? r.z : r.x, h ? r.w : r.y)
-                                                : i8x8_to_bf16(h ? r.z : r.x, h ? r.w : r.y);
-            }
-            mma(8 * i + 2 * g + h, bq);
-          }
-          if (MODE == kScale64) fold(i, cur);
-        }
+        for (int mi = 0; mi < MI; ++mi) acc[mi][nj] += p[mi][nj] * sv;
       }
-      if (MODE == kScale128) fold(0, cur);
     }
     __builtin_amdgcn_sched_barrier(0);
-    store_a(ra, lds + ((kb + 1) & 1) * F::kStage);
   };
 
-  TileW<FMT> w0, w1;
-  {
-    u32x4 ra[NA];
-    load_a(0, ra);
-    load_s(0, w0);
-#pragma unroll
-    for (int i = 0; i < F::kNL; ++i) load_w(0, i, w0);
-    store_a(ra, lds);
-  }
-  for (int kb = 0; kb < nsteps; kb += 2) {
-    step(kb, w0, w1);
-    if (kb + 1 < nsteps) step(kb + 1, w1, w0);
+  Wgt w0, w1;
+  issue_a(0, 0);
+  load_s(0, w0);
+  load_w(0, 0, w0);
+  load_w(0, 1, w0);
+  issue_a(1, 1);
+  int slot = 0;
+  auto next = [&] { slot = slot == 2 ? 0 : slot + 1; };
+  if constexpr (MODE == kScale128) {
+    for (int kb = 0; kb < nsteps; ++kb) {
+      step(kb, slot, w0, w0);
+      next();
+    }
+  } else {
+    for (int kb = 0; kb < nsteps; kb += 2) {
+      step(kb, slot, w0, w1);
+      next();
+      if (kb + 1 < nsteps) step(kb + 1, slot, w1, w0);
+      next();
+    }
   }
   if constexpr (MODE == kScaleOne) {
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) {
-      const float s = decode_scalar_word(bload4(sres, soff[nj] & ~3u), soff[nj] / sesz, W.s_dt);
+      const uint32_t idx = sidx(0, nj);
+      const float sv = decode_scalar_word(bload4(sres, (sesz * idx) & ~3u), idx, W.s_dt);
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi) acc[mi][nj] *= s;
+      for (int mi = 0; mi < MI; ++mi) acc[mi][nj] *= sv;
     }
   }
-  // every wave is done with the stages and (GPTQ) has written its row sums
+  // the copies past the last step have landed and every wave is done with the ring
+  wait_vm<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  if constexpr (GQ) {
-    // acc -= X . (s (z + 1)): groups 4 t + g of row m / column (nj, m)
-    const Rsrc zres = make_rsrc(W.z, (uint32_t)ngrp * (uint32_t)(N / 8) * 4u);
-    for (int t = 0; t < nsteps; t += 4) {
-      const int kb = t + g;
-      const bool in = kb < nsteps;
-      const uint32_t grp = (uint32_t)(kb * 128 / W.group);
-      float c[4];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const bool ok = in && soff[2 * h] != kOOB;
-        const uint32_t row = soff[2 * h] >> 1;
-        const uint32_t sw = bload4(sres, ok ? 2u * grp * (uint32_t)N + soff[2 * h] : kOOB);
-        const uint32_t zw = bload4(zres, ok ? 4u * (grp * (uint32_t)(N / 8) + row / 8u) : kOOB) >> (4u * (row & 7u));
-        c[2 * h] = -half_word(sw, 0, W.s_dt) * (float)((zw & 15u) + 1u);
-        c[2 * h + 1] = -half_word(sw, 1, W.s_dt) * (float)(((zw >> 4) & 15u) + 1u);
-      }
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi) {
-        const float xa = in ? Xs[(16 * mi + m) * (nsteps + 1) + kb] : 0.0f;
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, c[nj], acc[mi][nj], 0, 0, 0);
-      }
-    }
-  }
 }
 
 // h = act(gate) * up for one 16 x 16 block pair, with the activation fixed at
@@ -405,43 +334,45 @@ __device__ __forceinline__ void tile_store_y(const LayerArgs& a, const ProjSlot&
         const float w = s_w[row];
 #pragma unroll
         for (int nj = 0; nj < 4; nj += 2) {  // N is a multiple of 64: both columns of a lane or none
-          const int col = tile_row<FMT>(base, nj, m);
+          const int col = tile_row(base, nj, m);
           if (col < W.N) *(f32x2*)(y + col) = (f32x2){(acc[mi][nj][r] + bf[nj]) * w, (acc[mi][nj + 1][r] + bf[nj + 1]) * w};
         }
       }
     }
 }
 
-template <int FMT, int MODE, int MI, bool STB>
+template <int FMT, int MODE, int MI, bool STB, bool BIG>
 __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                         const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
+                                         const int* s_pair, const float* s_w, const float* s_bias) {
   using F = TileFmt<FMT>;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, m = lane & 15;
+  const int m = lane & 15;
   const int KP = a.KP, H = a.L.hidden;
-  const size_t arb = STB ? (size_t)a.Imax * 2u : (size_t)H * 2u;
+  const uint32_t arb = 2u * (uint32_t)(STB ? a.Imax : H);
   const char* abase = STB ? a.hbuf : (const char*)a.x;
-  const char* arow[F::kACopies];
+  TileSrc<F::kACopies> src;
 #pragma unroll
   for (int i = 0; i < F::kACopies; ++i) {
     constexpr int kPer = F::kARow / 16;
-    const int r = (kBlock / kPer) * i + tid / kPer;
+    const int r = (64 * (wave * F::kACopies + i) + lane) / kPer;
     const int pr = s_pair[r < rows ? r : 0];  // padding rows repeat the first (their outputs are dropped)
-    arow[i] = abase + (size_t)(STB ? pr : pr / KP) * arb;
+    const uint64_t off = (uint64_t)(STB ? pr : pr / KP) * arb + 16 * ((lane % kPer) ^ tile_fa<FMT>(r));
+    src.p[i] = BIG ? (uint64_t)(uintptr_t)abase + off : off;
   }
+  const uint32_t abytes = BIG ? 0u : (uint32_t)(STB ? a.T * KP : a.T) * arb;
   const int base[2] = {n0 + (STB ? 64 : 32) * wave, STB ? n0 + 64 * wave + 32 : Iu + n0 + 32 * wave};
   f32x4 acc[MI][4];
 #pragma unroll
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  tile_kloop<FMT, MODE, MI>(W, base, arow, lds, Xs, acc);
+  tile_kloop<FMT, MODE, MI, BIG>(W, base, abase, abytes, src, lds, acc);
 
   const int lb[2] = {(STB ? 64 : 32) * wave, STB ? 64 * wave + 32 : kTN / 2 + 32 * wave};
   float bf[4];
 #pragma unroll
-  for (int nj = 0; nj < 4; ++nj) bf[nj] = s_bias[tile_row<FMT>(lb, nj, m)];
+  for (int nj = 0; nj < 4; ++nj) bf[nj] = s_bias[tile_row(lb, nj, m)];
   if constexpr (STB) {
     tile_store_y<FMT, MI>(a, W, base, bf, rows, s_pair, s_w, acc);
   } else {
@@ -456,21 +387,14 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
 }
 
 // The tile on the instantiation for its number of 16-row blocks.
-template <int FMT, int MODE, bool STB>
+template <int FMT, int MODE, bool STB, bool BIG>
 __device__ __forceinline__ void tile_rows(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                          const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
-  if (rows > 32) tile_run<FMT, MODE, 4, STB>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias, Xs);
-  else tile_run<FMT, MODE, 2, STB>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias, Xs);
+                                          const int* s_pair, const float* s_w, const float* s_bias) {
+  if (rows > 32) tile_run<FMT, MODE, 4, STB, BIG>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias);
+  else tile_run<FMT, MODE, 2, STB, BIG>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias);
 }
 
 extern __shared__ __attribute__((aligned(16))) char ftm_tile_lds[];
-
-// Dynamic LDS: activation stages, the tile's pairs, router weights and biases, GPTQ row sums.
-template <int FMT>
-constexpr int tile_ring(bool shared) {
-  return shared && TileFmt<FTM_FMT_BF16>::kRing > TileFmt<FMT>::kRing ? TileFmt<FTM_FMT_BF16>::kRing
-                                                                      : TileFmt<FMT>::kRing;
-}
 
 // One item: a tile of 64 rows x 128 channels (stage A) or 256 columns (B).
 // Items run expert by expert (ascending compact index), within an expert over
@@ -582,29 +506,27 @@ __device__ __forceinline__ void tile_missing(const LayerArgs& a, const TileItem&
   if (threadIdx.x == 0) atomicOr(&a.ctrl[kCtrlError], 1);
 }
 
-template <int FMT, int MODE, bool STB>
-__global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a, int ring) {
+template <int FMT, int MODE, bool STB, bool BIG>
+__global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a) {
   char* lds = ftm_tile_lds;
-  int* s_pair = (int*)(lds + ring);
+  int* s_pair = (int*)(lds + TileFmt<FMT>::kRing);
   float* s_w = (float*)(s_pair + kTM);
   float* s_bias = s_w + kTM;
-  float* Xs = s_bias + kTN;
   const TileItem t = tile_item<STB>(a);
   if (t.rows <= 0) return;
   tile_tables<STB>(a, t, s_pair, s_w, s_bias);
   const int H = a.L.hidden, I = a.L.inter, Is = a.L.shared_inter;
-  const int n0 = t.n0, rows = t.rows, slot = t.slot;
   if (t.shared) {
     const ProjSlot W = STB ? shared_view(a.L.shared_w2, H, Is) : shared_view(a.L.shared_w13, 2 * Is, H);
-    tile_rows<FTM_FMT_BF16, kScaleNone, STB>(a, W, Is, n0, rows, lds, s_pair, s_w, s_bias, Xs);
+    tile_rows<FTM_FMT_BF16, kScaleNone, STB, BIG>(a, W, Is, t.n0, t.rows, lds, s_pair, s_w, s_bias);
     return;
   }
   const ftm_proj& PW = STB ? a.L.w2 : a.L.w13;
-  if (slot < 0 || slot >= PW.num_slots) {
+  if (t.slot < 0 || t.slot >= PW.num_slots) {
     tile_missing<STB>(a, t, s_pair);
     return;
   }
-  tile_rows<FMT, MODE, STB>(a, proj_slot(PW, slot), I, n0, rows, lds, s_pair, s_w, s_bias, Xs);
+  tile_rows<FMT, MODE, STB, BIG>(a, proj_slot(PW, t.slot), I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
 }
 
 // ---------------------------------------------------------------- scaled-MFMA tiles
@@ -633,13 +555,15 @@ struct MxW {
   uint32_t s[4];  // MXFP4: the lane's e8m0 byte of block nj; FP8: [0] / [2], the halves' fp32 block scales
 };
 
-// This thread's activation sources: byte offsets (BIG: addresses) of the rows
-// its copies read.  Copy i of a wave covers rows 16 wave + 4 i + lane / 16
-// (16-byte pieces, swizzled), its last one the scale bytes of rows 16 wave +
-// lane / 4.
-struct MxRows {
-  uint64_t p[5];
+template <>
+struct MxW<FTM_FMT_GPTQ_INT4> {
+  u32x2 w[2][4];  // [half][i]: columns 2m, 2m + 1; words of K 16 g, 16 g + 8, 64 + 16 g, 72 + 16 g
+  uint32_t s[2];  // [half]: both columns' 16-bit scales
 };
+
+// Copy i of a wave covers rows 16 wave + 4 i + lane / 16 (16-byte pieces,
+// swizzled), its last one the scale bytes of rows 16 wave + lane / 4.
+using MxRows = TileSrc<5>;
 
 // Wait until at most NW + NA n vector-memory operations are in flight (n < 4).
 template <int NW, int NA>
@@ -651,22 +575,33 @@ __device__ __forceinline__ void wait_n(int n) {
 }
 
 // One K step of a wave: 16 MI activation rows of the LDS stage st against its
-// 64 weight rows, into acc.
+// 64 weight rows, into acc.  GPTQ: x = the sums of row block `wave` over the step.
 template <int FMT, int MI>
-__device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, f32x4 (&acc)[MI][4]) {
-  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK;
-  constexpr int NL = F8 ? 2 : 1;
+__device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, int s_dt, f32x4 (&acc)[MI][4], f32x4& x) {
+  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK, GQ = FMT == FTM_FMT_GPTQ_INT4;
+  constexpr bool POST = F8 || GQ;  // the step's products are scaled into acc
   const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
   i32x8 bw[4];
   int sb[4];
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) {
-    const u32x4 r0 = cur.w[nj][0];
-    if constexpr (F8) {
-      const u32x4 r1 = cur.w[nj][NL - 1];
+    if constexpr (GQ) {
+      // a nibble, zero-extended to a byte, is the e4m3 code of q 2^-9 (0..15
+      // are the subnormals and the first binade): scale_b = 2^9 makes it q
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t w = (nj & 1) ? cur.w[nj >> 1][i].y : cur.w[nj >> 1][i].x;
+        const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;       // q0 q2 q4 q6 / q1 q3 q5 q7
+        bw[nj][2 * i] = (int)__builtin_amdgcn_perm(hi, lo, 0x05010400u);      // q0 q1 q2 q3
+        bw[nj][2 * i + 1] = (int)__builtin_amdgcn_perm(hi, lo, 0x07030602u);  // q4 q5 q6 q7
+      }
+      sb[nj] = 127 + 9;
+    } else if constexpr (F8) {
+      const u32x4 r0 = cur.w[nj][0], r1 = cur.w[nj][1];
       bw[nj] = (i32x8){(int)r0.x, (int)r0.y, (int)r0.z, (int)r0.w, (int)r1.x, (int)r1.y, (int)r1.z, (int)r1.w};
       sb[nj] = 127;
     } else {
+      const u32x4 r0 = cur.w[nj][0];
       bw[nj] = (i32x8){(int)r0.x, (int)r0.y, (int)r0.z, (int)r0.w, 0, 0, 0, 0};
       sb[nj] = (int)cur.s[nj];
     }
@@ -687,21 +622,38 @@ __device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, f32
   auto scales = [&](int mi) { return (uint32_t)*(const uint16_t*)(st + kTM * kXRow + 16 * (16 * mi + m) + 2 * g); };
   f32x4 tq[2][4];
   auto fold = [&](int mi) {
-    if constexpr (F8) {
+    if constexpr (POST) {
 #pragma unroll
-      for (int nj = 0; nj < 4; ++nj) acc[mi][nj] += tq[mi & 1][nj] * __uint_as_float(cur.s[nj & 2]);
+      for (int nj = 0; nj < 4; ++nj) {
+        float s;
+        if constexpr (GQ) s = half_word(cur.s[nj >> 1], nj & 1, s_dt);
+        else s = __uint_as_float(cur.s[nj & 2]);
+        acc[mi][nj] += tq[mi & 1][nj] * s;
+      }
     }
   };
-  constexpr int kB = F8 ? 0 : 4;  // B format: e4m3 or e2m1
+  constexpr int kB = POST ? 0 : 4;  // B format: e4m3 or e2m1
   auto mma = [&](int mi, const Term& t, int scale, bool first) {
     const i32x8 av = {(int)t.a.x, (int)t.a.y, (int)t.a.z, (int)t.a.w, (int)t.b.x, (int)t.b.y, (int)t.b.z, (int)t.b.w};
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) {
-      f32x4& d = F8 ? tq[mi & 1][nj] : acc[mi][nj];
+      f32x4& d = POST ? tq[mi & 1][nj] : acc[mi][nj];
       const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bw[nj], F8 && first ? z : d, 0, kB, 0, scale, 0, sb[nj]);
+      d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bw[nj], POST && first ? z : d, 0, kB, 0, scale, 0, sb[nj]);
     }
   };
+  if constexpr (GQ) {
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const Term h = term(wave, 0), l = term(wave, 1);
+    const uint32_t xs = scales(wave);
+    const int one = 0x38383838;  // e4m3 1.0
+    const i32x8 ones = {one, one, one, one, one, one, one, one};
+    const i32x8 hv = {(int)h.a.x, (int)h.a.y, (int)h.a.z, (int)h.a.w, (int)h.b.x, (int)h.b.y, (int)h.b.z, (int)h.b.w};
+    const i32x8 lv = {(int)l.a.x, (int)l.a.y, (int)l.a.z, (int)l.a.w, (int)l.b.x, (int)l.b.y, (int)l.b.z, (int)l.b.w};
+    x = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(hv, ones, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0,
+                                                         (int)(xs & 0xffu), 0, 127);
+    x = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(lv, ones, x, 0, 0, 0, (int)(xs >> 8), 0, 127);
+  }
   Term hi = term(0, 0);
   uint32_t sc = scales(0);
 #pragma unroll
@@ -724,10 +676,9 @@ __device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, f32
 
 template <int FMT, int MI, bool BIG, bool SHORT>
 __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2], const char* abase, uint32_t abytes,
-                                         const MxRows& rows, char* lds, f32x4 (&acc)[MI][4]) {
-  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK;
-  constexpr int NL = F8 ? 2 : 1;
-  constexpr int NA = 5, NW = 4 * NL + (F8 ? 2 : 4);  // copies / loads a step
+                                         const MxRows& rows, char* lds, float* Xs, f32x4 (&acc)[MI][4]) {
+  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK, GQ = FMT == FTM_FMT_GPTQ_INT4;
+  constexpr int NA = 5, NW = F8 || GQ ? 10 : 8;  // copies / loads a step
   typedef __attribute__((address_space(1))) const void* GPtr;
   typedef __attribute__((address_space(3))) void* LPtr;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -757,31 +708,67 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
 
   const uint32_t rb = F8 ? (uint32_t)K : (uint32_t)K / 2;
   const int nkb = K / 128;
+  const int ngrp = GQ ? K / W.group : 0;
   const Rsrc wres = make_rsrc(W.w, rb * (uint32_t)N);
-  const Rsrc sres = make_rsrc(W.s, F8 ? 4u * (uint32_t)((N + 127) / 128) * (uint32_t)nkb : (uint32_t)N * (uint32_t)(K / 32));
-  uint32_t woff[4];
+  const Rsrc sres = make_rsrc(W.s, F8 ? 4u * (uint32_t)((N + 127) / 128) * (uint32_t)nkb
+                              : GQ ? 2u * (uint32_t)ngrp * (uint32_t)N
+                                   : (uint32_t)N * (uint32_t)(K / 32));
+  uint32_t woff[GQ ? 2 : 4];
+  if constexpr (GQ) {  // the halves' first columns, word row 2 g
 #pragma unroll
-  for (int nj = 0; nj < 4; ++nj) {
-    const int row = tile_row<FMT>(base, nj, m);
-    woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
+    for (int h = 0; h < 2; ++h) {
+      const int row = tile_row(base, 2 * h, m);
+      woff[h] = row < N ? 4u * (uint32_t)(2 * g * N + row) : kOOB;
+    }
+  } else {
+#pragma unroll
+    for (int nj = 0; nj < 4; ++nj) {
+      const int row = tile_row(base, nj, m);
+      woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
+    }
   }
   auto load_w = [&](int kb, MxW<FMT>& t) {
-    const int k0 = F8 ? kb * 128 : kb * 128 + 32 * g;  // FP8: K is whole steps
-    const uint32_t so = k0 < K ? 4u * (uint32_t)kb : kOOB;
-    const uint32_t ko = k0 < K ? (uint32_t)kb * (F8 ? 128u : 64u) : kOOB;
-    if constexpr (F8) {
+    if constexpr (GQ) {
+      const uint32_t go = kb < nsteps ? 2u * (uint32_t)(kb * 128 / W.group) * (uint32_t)N : kOOB;
+      const uint32_t ko = kb < nsteps ? (uint32_t)kb * 64u * (uint32_t)N : kOOB;
 #pragma unroll
-      for (int h = 0; h < 4; h += 2) t.s[h] = bload4(sres, 4u * (uint32_t)(base[h >> 1] / 128 * nkb) + so);
+      for (int h = 0; h < 2; ++h) t.s[h] = bload4(sres, 2u * (uint32_t)tile_row(base, 2 * h, m) + go);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          t.w[h][i] = __builtin_amdgcn_raw_buffer_load_b64(wres, woff[h] + ko,
+                                                           4u * (uint32_t)N * (uint32_t)((i & 1) + 8 * (i >> 1)), 0);
     } else {
-      // the e8m0 byte of a 16-byte piece sits at a sixteenth of its offset
-      // (rows past N: past the scales' end as well)
+      const int k0 = F8 ? kb * 128 : kb * 128 + 32 * g;  // FP8: K is whole steps
+      const uint32_t so = k0 < K ? 4u * (uint32_t)kb : kOOB;
+      const uint32_t ko = k0 < K ? (uint32_t)kb * (F8 ? 128u : 64u) : kOOB;
+      if constexpr (F8) {
 #pragma unroll
-      for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload1(sres, (woff[nj] >> 4) + so);
+        for (int h = 0; h < 4; h += 2) t.s[h] = bload4(sres, 4u * (uint32_t)(base[h >> 1] / 128 * nkb) + so);
+      } else {
+        // the e8m0 byte of a 16-byte piece sits at a sixteenth of its offset
+        // (rows past N: past the scales' end as well)
+#pragma unroll
+        for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload1(sres, (woff[nj] >> 4) + so);
+      }
+#pragma unroll
+      for (int nj = 0; nj < 4; ++nj)
+#pragma unroll
+        for (int i = 0; i < (F8 ? 2 : 1); ++i) t.w[nj][i] = bload16(wres, woff[nj] + ko + 64u * (uint32_t)i);
     }
+  };
+  // GPTQ: the row sums of step kb (the same in every column)
+  auto put_x = [&](int kb, f32x4 x) {
+    if constexpr (GQ) {
+      // the sums exist before the branch: the compiler has sunk their MFMAs
+      // (and the operand moves, which then skip the masked lanes) into it
+      asm volatile("" : "+v"(x));
+      if (m == 0) {
 #pragma unroll
-    for (int nj = 0; nj < 4; ++nj)
-#pragma unroll
-      for (int i = 0; i < NL; ++i) t.w[nj][i] = bload16(wres, woff[nj] + ko + 64u * (uint32_t)i);
+        for (int r = 0; r < 4; ++r) Xs[(16 * wave + 4 * g + r) * (nsteps + 1) + kb] = x[r];
+      }
+    }
   };
 
   MxW<FMT> w0, w1;
@@ -801,7 +788,8 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
         asm volatile("s_barrier" ::: "memory");
         if (kb + 1 < kXbSteps) load_w(kb + 1, kb & 1 ? w0 : w1);
         __builtin_amdgcn_sched_barrier(0);
-        mx_step<FMT, MI>(lds + kb * kXStage, cur, acc);
+        f32x4 x;
+        mx_step<FMT, MI>(lds + kb * kXStage, cur, W.s_dt, acc, x);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -815,7 +803,9 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
       issue_a(kb + 2, slot == 0 ? 2 : slot - 1);
       load_w(kb + 1, nxt);
       __builtin_amdgcn_sched_barrier(0);
-      mx_step<FMT, MI>(lds + slot * kXStage, cur, acc);
+      f32x4 x;
+      mx_step<FMT, MI>(lds + slot * kXStage, cur, W.s_dt, acc, x);
+      put_x(kb, x);
       __builtin_amdgcn_sched_barrier(0);
     };
     issue_a(0, 0);
@@ -847,6 +837,32 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
   // the copies past the last step have landed and every wave is done with the ring
   wait_vm<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (GQ) {
+    // the zero points: acc -= X . (s (z + 1)), steps t + g of row m / column (nj, m)
+    const Rsrc zres = make_rsrc(W.z, (uint32_t)ngrp * (uint32_t)(N / 8) * 4u);
+    for (int t = 0; t < nsteps; t += 4) {
+      const int kb = t + g;
+      const bool in = kb < nsteps;
+      const uint32_t grp = (uint32_t)(kb * 128 / W.group);
+      float c[4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t row = (uint32_t)tile_row(base, 2 * h, m);
+        const bool ok = in && row < (uint32_t)N;
+        const uint32_t sw = bload4(sres, ok ? 2u * (grp * (uint32_t)N + row) : kOOB);
+        const uint32_t zw = bload4(zres, ok ? 4u * (grp * (uint32_t)(N / 8) + row / 8u) : kOOB) >> (4u * (row & 7u));
+        c[2 * h] = -half_word(sw, 0, W.s_dt) * (float)((zw & 15u) + 1u);
+        c[2 * h + 1] = -half_word(sw, 1, W.s_dt) * (float)(((zw >> 4) & 15u) + 1u);
+      }
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi) {
+        const float xa = in ? Xs[(16 * mi + m) * (nsteps + 1) + kb] : 0.0f;
+#pragma unroll
+        for (int nj = 0; nj < 4; ++nj)
+          acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, c[nj], acc[mi][nj], 0, 0, 0);
+      }
+    }
+  }
 }
 
 template <bool STB, bool BIG>
@@ -870,7 +886,7 @@ __device__ __forceinline__ MxRows mx_rows(const LayerArgs& a, int rows, const in
 
 template <int FMT, int MI, bool STB, bool BIG, bool SHORT>
 __device__ __forceinline__ void mx_run(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                       const int* s_pair, const float* s_w, const float* s_bias) {
+                                       const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15;
@@ -885,12 +901,12 @@ __device__ __forceinline__ void mx_run(const LayerArgs& a, const ProjSlot& W, in
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  mx_kloop<FMT, MI, BIG, SHORT>(W, base, abase, abytes, ar, lds, acc);
+  mx_kloop<FMT, MI, BIG, SHORT>(W, base, abase, abytes, ar, lds, Xs, acc);
 
   const int lb[2] = {(STB ? 64 : 32) * wave, STB ? 64 * wave + 32 : kTN / 2 + 32 * wave};
   float bf[4];
 #pragma unroll
-  for (int nj = 0; nj < 4; ++nj) bf[nj] = s_bias[tile_row<FMT>(lb, nj, m)];
+  for (int nj = 0; nj < 4; ++nj) bf[nj] = s_bias[tile_row(lb, nj, m)];
   if constexpr (STB) {
     tile_store_y<FMT, MI>(a, W, base, bf, rows, s_pair, s_w, acc);
   } else {
@@ -927,7 +943,7 @@ __device__ __forceinline__ void mx_tile(const LayerArgs& a, int ring) {
   const int H = a.L.hidden, I = a.L.inter, Is = a.L.shared_inter;
   if (t.shared) {
     const ProjSlot W = STB ? shared_view(a.L.shared_w2, H, Is) : shared_view(a.L.shared_w13, 2 * Is, H);
-    tile_rows<FTM_FMT_BF16, kScaleNone, STB>(a, W, Is, t.n0, t.rows, lds, s_pair, s_w, s_bias, nullptr);
+    tile_rows<FTM_FMT_BF16, kScaleNone, STB, BIG>(a, W, Is, t.n0, t.rows, lds, s_pair, s_w, s_bias);
     return;
   }
   const ftm_proj& PW = STB ? a.L.w2 : a.L.w13;
@@ -936,8 +952,9 @@ __device__ __forceinline__ void mx_tile(const LayerArgs& a, int ring) {
     return;
   }
   const ProjSlot W = proj_slot(PW, t.slot);
-  if (t.rows > 32) mx_run<FMT, 4, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
-  else mx_run<FMT, 2, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
+  float* Xs = s_bias + kTN;
+  if (t.rows > 32) mx_run<FMT, 4, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias, Xs);
+  else mx_run<FMT, 2, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias, Xs);
 }
 
 template <int FMT, bool STB, bool BIG>
@@ -954,21 +971,29 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_mxb_f8(const LayerArgs a) {
 }
 
 // ---------------------------------------------------------------- launch
-// Dynamic LDS of one projection's tiles.
-template <int FMT>
-static size_t tile_lds(const ftm_moe_layer& L, bool stb) {
-  const int K = stb ? L.inter : L.hidden;
-  const size_t x = FMT == FTM_FMT_GPTQ_INT4 ? (size_t)kTM * (size_t)((K + 127) / 128 + 1) * 4u : 0u;
-  return (size_t)tile_ring<FMT>(L.shared_inter > 0) + (size_t)kTM * 8u + (size_t)kTN * 4u + x;
+// Dynamic LDS of one projection's scaled-MFMA tiles: activation stages, the
+// tile's pairs, router weights and biases, GPTQ row sums.
+static size_t mx_lds(const ftm_moe_layer& L, bool stb) {
+  const size_t x = L.w13.fmt == FTM_FMT_GPTQ_INT4 ? (size_t)kTM * (size_t)((stb ? L.inter : L.hidden) / 128 + 1) * 4u : 0u;
+  return (size_t)kXStages * kXStage + (size_t)kTM * 8u + (size_t)kTN * 4u + x;
 }
 
 // GPTQ layers the tiles take: 128-wide groups (or multiples), 16-bit scales,
 // whole K steps, and row sums that fit the LDS beside the ring.
 bool tile_gptq_ok(const ftm_moe_layer& L) {
-  if (L.w13.fmt != FTM_FMT_GPTQ_INT4 || L.act_dtype != FTM_DT_BF16) return false;
-  if (L.w13.group % 128 != 0 || L.w2.group % 128 != 0 || L.hidden % 128 != 0 || L.inter % 128 != 0) return false;
+  if (L.w13.fmt != FTM_FMT_GPTQ_INT4 || L.act_dtype != FTM_DT_BF16 || (L.w13.flags & kProjNoTiles) != 0) return false;
+  if (L.w13.group <= 0 || L.w2.group <= 0 || L.w13.group % 128 != 0 || L.w2.group % 128 != 0) return false;
+  if (L.hidden % 128 != 0 || L.inter % 128 != 0 || L.hidden % L.w13.group != 0 || L.inter % L.w2.group != 0) return false;
   if (L.w13.s_dtype == FTM_DT_F32 || L.w2.s_dtype == FTM_DT_F32) return false;
-  return tile_lds<FTM_FMT_GPTQ_INT4>(L, false) <= 160u * 1024u && tile_lds<FTM_FMT_GPTQ_INT4>(L, true) <= 160u * 1024u;
+  return mx_lds(L, false) <= 160u * 1024u && mx_lds(L, true) <= 160u * 1024u;
+}
+
+// INT8 and bf16 layers the bf16 tiles take: INT8 groups of whole K steps, or one over K.
+bool tile_bf16_ok(const ftm_moe_layer& L) {
+  if (L.act_dtype != FTM_DT_BF16) return false;
+  if (L.w13.fmt == FTM_FMT_BF16) return true;
+  auto ok = [](const ftm_proj& P) { return P.group == P.K || (P.group % 128 == 0 && P.group > 0); };
+  return L.w13.fmt == FTM_FMT_INT8_PACKED && ok(L.w13) && ok(L.w2);
 }
 
 // Items of one stage, an upper bound: every routed expert's last M tile may
@@ -994,35 +1019,52 @@ static void tile_attr(K* kernel, bool& done) {
   }
 }
 
-template <int FMT, int MODE, bool STB>
-static void launch_tile_t(const LayerArgs& a, hipStream_t st) {
-  static bool attr = false;
-  tile_attr(&k_tile<FMT, MODE, STB>, attr);
-  hipLaunchKernelGGL((k_tile<FMT, MODE, STB>), dim3(tile_items<STB>(a)), dim3(kBlock), tile_lds<FMT>(a.L, STB), st, a,
-                     tile_ring<FMT>(a.L.shared_inter > 0));
+// BIG: activation rows past what one buffer descriptor's 32-bit offsets span.
+static bool tile_big(const LayerArgs& a, bool stb, size_t row_bytes) {
+  return (stb ? (double)a.T * a.KP : (double)a.T) * (double)row_bytes >= 4294967296.0;
 }
 
-void launch_tile_gptq(const LayerArgs& a, hipStream_t st, int which) {
-  if (which & 1) launch_tile_t<FTM_FMT_GPTQ_INT4, kScale128, false>(a, st);
-  if (which & 2) launch_tile_t<FTM_FMT_GPTQ_INT4, kScale128, true>(a, st);
+template <int FMT, int MODE, bool STB, bool BIG>
+static void launch_tile_t(const LayerArgs& a, hipStream_t st) {
+  static bool attr = false;
+  tile_attr(&k_tile<FMT, MODE, STB, BIG>, attr);
+  static_assert(TileFmt<FMT>::kRing >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
+  hipLaunchKernelGGL((k_tile<FMT, MODE, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock),
+                     (size_t)TileFmt<FMT>::kRing + (size_t)kTM * 8u + (size_t)kTN * 4u, st, a);
+}
+
+template <int FMT, int MODE, bool STB>
+static void launch_tile_s(const LayerArgs& a, hipStream_t st) {
+  if (tile_big(a, STB, 2u * (size_t)(STB ? a.Imax : a.L.hidden))) launch_tile_t<FMT, MODE, STB, true>(a, st);
+  else launch_tile_t<FMT, MODE, STB, false>(a, st);
+}
+
+void launch_tile_bf16(const LayerArgs& a, hipStream_t st, int which) {
+  const bool i8 = a.L.w13.fmt == FTM_FMT_INT8_PACKED;
+  if (which & 1) {
+    if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, false>(a, st);
+    else if (a.L.w13.group == a.L.w13.K) launch_tile_s<FTM_FMT_INT8_PACKED, kScaleOne, false>(a, st);
+    else launch_tile_s<FTM_FMT_INT8_PACKED, kScale128, false>(a, st);
+  }
+  if (which & 2) {
+    if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, true>(a, st);
+    else if (a.L.w2.group == a.L.w2.K) launch_tile_s<FTM_FMT_INT8_PACKED, kScaleOne, true>(a, st);
+    else launch_tile_s<FTM_FMT_INT8_PACKED, kScale128, true>(a, st);
+  }
 }
 
 template <int FMT, bool STB, bool BIG>
 static void launch_mx_t(const LayerArgs& a, hipStream_t st) {
   static bool attr = false;
   tile_attr(&k_gemm_mx<FMT, STB, BIG>, attr);
-  constexpr int kRing = kXStages * kXStage;
-  static_assert(kRing >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
-  hipLaunchKernelGGL((k_gemm_mx<FMT, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock),
-                     (size_t)kRing + (size_t)kTM * 8u + (size_t)kTN * 4u, st, a);
+  static_assert(kXStages * kXStage >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
+  hipLaunchKernelGGL((k_gemm_mx<FMT, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock), mx_lds(a.L, STB), st, a);
 }
 
-// BIG: activation rows past what one buffer descriptor's 32-bit offsets span.
 template <int FMT, bool STB>
 static void launch_mx_s(const LayerArgs& a, hipStream_t st) {
-  const double rows = STB ? (double)a.T * a.KP : (double)a.T;
-  if (rows * (double)mx_row_bytes(STB ? a.Imax : a.L.hidden) < 4294967296.0) launch_mx_t<FMT, STB, false>(a, st);
-  else launch_mx_t<FMT, STB, true>(a, st);
+  if (tile_big(a, STB, (size_t)mx_row_bytes(STB ? a.Imax : a.L.hidden))) launch_mx_t<FMT, STB, true>(a, st);
+  else launch_mx_t<FMT, STB, false>(a, st);
 }
 
 // k_gemm_mxb_f8's layers; FTM_PROJ_RING_B asks for k_gemm_mx.
@@ -1041,14 +1083,16 @@ static void launch_mxb(const LayerArgs& a, hipStream_t st) {
 }
 
 void launch_tile_mx(const LayerArgs& a, hipStream_t st, int which) {
-  const bool f8 = a.L.w13.fmt == FTM_FMT_FP8_BLOCK;
+  const int f = a.L.w13.fmt;
   if (which & 1) {
-    if (f8) launch_mx_s<FTM_FMT_FP8_BLOCK, false>(a, st);
+    if (f == FTM_FMT_FP8_BLOCK) launch_mx_s<FTM_FMT_FP8_BLOCK, false>(a, st);
+    else if (f == FTM_FMT_GPTQ_INT4) launch_mx_s<FTM_FMT_GPTQ_INT4, false>(a, st);
     else launch_mx_s<FTM_FMT_MXFP4, false>(a, st);
   }
   if (which & 2) {
-    if (f8 && tile_mxb_ok(a.L, a.T)) launch_mxb(a, st);
-    else if (f8) launch_mx_s<FTM_FMT_FP8_BLOCK, true>(a, st);
+    if (f == FTM_FMT_FP8_BLOCK && tile_mxb_ok(a.L, a.T)) launch_mxb(a, st);
+    else if (f == FTM_FMT_FP8_BLOCK) launch_mx_s<FTM_FMT_FP8_BLOCK, true>(a, st);
+    else if (f == FTM_FMT_GPTQ_INT4) launch_mx_s<FTM_FMT_GPTQ_INT4, true>(a, st);
     else launch_mx_s<FTM_FMT_MXFP4, true>(a, st);
   }
 }

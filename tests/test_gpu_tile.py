@@ -64,14 +64,26 @@ def test_gptq_tiles_match_oracle(gpu, T, H, I, shared, group):
         z = syn.bank[n]
         syn.bank[n] = torch.randint(-2**31, 2**31 - 1, z.shape, generator=g, dtype=torch.int64).to(torch.int32)
     layer = _check(syn, gpu)
+    assert layer.stage_kernel(T, nat.STAGE_W13) == "k_gemm_mx"
+    assert layer.stage_kernel(T, nat.STAGE_W2) == "k_gemm_mx"
+
+
+@pytest.mark.parametrize("T,H,I,shared,groups", [(64, 256, 128, 0, 1), (130, 320, 192, 0, 1), (100, 512, 256, 128, 2),
+                                                 (75, 384, 256, 0, 1)])
+def test_int8_tiles_match_oracle(gpu, T, H, I, shared, groups):
+    """INT8 per channel and with K groups of 256 / 128, K ending in a half
+    step (H = 320, I = 192), channels and columns that end inside a tile."""
+    cfg = replace(S.SMALL["c1_int8"], H=H, I=I, shared_inter=shared, int8_num_groups=groups)
+    layer = _check(S.generate(cfg, T=T, seed=T + H), gpu)
     assert layer.stage_kernel(T, nat.STAGE_W13) == "k_tile"
     assert layer.stage_kernel(T, nat.STAGE_W2) == "k_tile"
 
 
-@pytest.mark.parametrize("name", ["c2_gptq", "c3_fp8", "c4_mxfp4"])
+@pytest.mark.parametrize("name", ["c1_int8", "c2_gptq", "c3_fp8", "c4_mxfp4", "bf16"])
 def test_tiles_with_uneven_experts(gpu, name):
     """Experts of 1, 15, 16, 17, 32, 33, 64, 65 and 129 rows, some of none."""
     T, E, k = 144, 16, 4
-    syn = S.generate(replace(S.SMALL[name], E=E, k=k), T=T, seed=9)
+    cfg = replace(S.SMALL["c1_int8"], fmt="bf16") if name == "bf16" else S.SMALL[name]
+    syn = S.generate(replace(cfg, E=E, k=k), T=T, seed=9)
     ids, w = _skewed(T, E, k, [1, 15, 16, 17, 0, 32, 33, 64, 65, 129, 0, 48], 3)
     _check(syn, gpu, ids, w)
