@@ -26,11 +26,23 @@ namespace ftm {
 constexpr int kGM = 64;            // tokens per tile
 constexpr int kGK = 64;            // K per step
 constexpr int kGPitch = kGK + 8;   // LDS row pitch in bf16 (144 B: rows do not share a bank period)
-// Crossover, in average tokens per routed expert.  Measured on MI355X (C3 FP8
-// and C4 MXFP4 layers): the tiles win from 16 on (C3 T=512: 466 us against
-// 723 us on the GEMVs; C4 T=128: 360 us against 380 us) and lose at 8 and
-// below (C4 T=64: 341 us against 236 us; C4 T=32: 333 us against 193 us).
+// Crossover, in average tokens per routed expert: 16 where the tiles' grid is
+// small (a tile's latency is then the stage's: 16 INT8 experts of 512 take
+// 26.6 us on the GEMV stages against 34.6 at 8 tokens per expert, 50 against
+// 37 at 16) and for MXFP4 (its token-resident stages win below).
 constexpr int kGemmMinRows = 16;
+// Register-fed tiles that cover the chip (at least kGemmWideItems stage-A
+// tiles, one per CU) read the weights once at a higher rate than the GEMV
+// stages, which read them again for every few tokens.  Measured on MI355X (us
+// per layer, GEMV stages / tiles): GPTQ 128 experts of 768 at 2 / 3 / 8 tokens
+// per expert 103 / 124 / 136 against 101 / 104 / 110; 64 INT8 experts of 1024
+// at 2 / 8 132 / 172 against 112 / 123; 64 FP8 experts of 1024 at 3 / 12 162 /
+// 237 against 128 / 143; bf16 at 2 / 3 220 / 253 against 241 / 248.
+constexpr int kGemmMinRowsWide = 3;
+constexpr int kGemmWideItems = 256;
+// The lean FP8 shape's own stages hold on longer: 2 / 3 / 4 / 6 / 8 tokens per
+// expert 149 / 175 / 199 / 237 / 270 us against 168 / 188 / 190 / 201 / 205.
+constexpr int kGemmMinRowsLean = 9;
 
 // Weight bytes per element and 16-byte pieces per tile row per K step.
 template <int WFMT>
@@ -784,12 +796,15 @@ bool gemm_path_ok(const ftm_moe_layer& L, int T) {
       (L.w13.group % kGK != 0 || L.w2.group % kGK != 0))
     return false;
   if (L.apply_router_weight_on_input) return false;
-  // above the crossover: on average at least kGemmMinRows tokens per routed
+  // above the crossover: on average at least that many tokens per routed
   // expert (MXFP4: more than that, up to which its scaled-MFMA decode path wins)
   const long pairs = (long)T * L.topk;
   const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
   if (f == FTM_FMT_MXFP4 && T <= kXlMaxTMx) return pairs > (long)kGemmMinRows * maxU;
-  return pairs >= (long)kGemmMinRows * maxU;
+  long rows = kGemmMinRows;
+  if (f != FTM_FMT_MXFP4 && (mx_gemm_ok(L) || tile_bf16_ok(L)) && maxU * ((L.inter + 127) / 128) >= kGemmWideItems)
+    rows = lean_shape(L) ? kGemmMinRowsLean : kGemmMinRowsWide;
+  return pairs >= rows * maxU;
 }
 
 // Whether the ring tiles take this layer: weights whose tile scales fit the

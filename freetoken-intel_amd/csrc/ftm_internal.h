@@ -169,15 +169,15 @@ void launch_quant_mx(const void* x, int T, int H, uint8_t* xq, hipStream_t st);
 // range per wave in stage A), I = 512 (one 8-load window per wave in stage
 // B), fp32 block-128 scales, no projection biases, bf16 activations and a
 // shared expert (if any) of the routed width, below the GEMM crossover.
-inline bool lean_ok(const ftm_moe_layer& L, int T) {
+inline bool lean_shape(const ftm_moe_layer& L) {
   const ftm_proj &A = L.w13, &B = L.w2;
   if (A.fmt != FTM_FMT_FP8_BLOCK || L.act_dtype != FTM_DT_BF16) return false;
   if (A.group != 128 || B.group != 128 || A.s_dtype != FTM_DT_F32 || B.s_dtype != FTM_DT_F32) return false;
   if (A.bias != nullptr || B.bias != nullptr) return false;
   if (L.hidden != 2048 || L.inter != 512) return false;
-  if (L.shared_inter != 0 && L.shared_inter != L.inter) return false;
-  return !gemm_path_ok(L, T);
+  return L.shared_inter == 0 || L.shared_inter == L.inter;
 }
+inline bool lean_ok(const ftm_moe_layer& L, int T) { return lean_shape(L) && !gemm_path_ok(L, T); }
 
 // Small decode batches on the lean kernels: stage A routes the T <=
 // kLeanRouteMaxT tokens in every workgroup (one wave per token) instead of

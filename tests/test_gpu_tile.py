@@ -87,3 +87,15 @@ def test_tiles_with_uneven_experts(gpu, name):
     syn = S.generate(replace(cfg, E=E, k=k), T=T, seed=9)
     ids, w = _skewed(T, E, k, [1, 15, 16, 17, 0, 32, 33, 64, 65, 129, 0, 48], 3)
     _check(syn, gpu, ids, w)
+
+
+@pytest.mark.parametrize("fmt", ["c1_int8", "c2_gptq", "c3_fp8", "bf16"])
+@pytest.mark.parametrize("T", [47, 48])
+def test_tiles_of_few_rows(gpu, fmt, T):
+    """64 experts of 512 channels cover the chip: tiles from 3 tokens per
+    expert (48 tokens, top-4) on, most of a row block empty; the GEMV stages
+    below."""
+    cfg = replace(S.SMALL["c1_int8"], fmt="bf16") if fmt == "bf16" else S.SMALL[fmt]
+    layer = _check(S.generate(replace(cfg, E=64, k=4, H=256, I=512, shared_inter=0), T=T, seed=T), gpu)
+    tile = {"c1_int8": "k_tile", "bf16": "k_tile", "c2_gptq": "k_gemm_mx", "c3_fp8": "k_gemm_mx"}[fmt]
+    assert (layer.stage_kernel(T, nat.STAGE_W13) == tile) == (T >= 48)
