@@ -126,13 +126,14 @@ inline WsLayout ws_layout(const ftm_moe_layer& L, int T) {
 }
 
 // ---- launchers (ftm_moe.hip); all return hipError_t of the launch
-// quant: also quantise the input for the MXFP4 stage A (mx_stage_a) in the
-// same launch; the expert stages are then launched with xq_ready.
+// quant / x: also quantise the input for the expert stages that read it so
+// (mx_input), in the router's launch or, for the batches of k_topk_blk, in the
+// top-k's; the expert stages are then launched with xq_ready.
 hipError_t launch_router(const ftm_moe_layer& L, const void* x, int T, int row_begin, int row_end, char* ws,
                          const WsLayout& wl, hipStream_t st, bool quant = false);
 hipError_t launch_topk(const ftm_moe_layer& L, int T, const void* logits_in, int logits_dt,
                        const int32_t* ids_in, const float* w_in, int32_t* ids_out, float* w_out,
-                       float* logits_out, char* ws, const WsLayout& wl, hipStream_t st);
+                       float* logits_out, char* ws, const WsLayout& wl, hipStream_t st, const void* x = nullptr);
 // The caller's routing outputs of ftm_moe_forward (each may be null).
 struct RouteOut {
   int32_t* ids;
@@ -141,7 +142,7 @@ struct RouteOut {
 };
 // ro: route inside the expert stages where lean_route_ok allows it (the caller
 // then launches no top-k); which: bit 0 = stage A, bit 1 = stage B, bit 2 = combine;
-// xq_ready: the router launch has quantised the input (launch_router's quant).
+// xq_ready: the routing launches have quantised the input (launch_router, launch_topk).
 hipError_t launch_experts(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws,
                           const WsLayout& wl, hipStream_t st, int which = 7, const RouteOut* ro = nullptr,
                           bool xq_ready = false);

@@ -90,6 +90,7 @@ __global__ __launch_bounds__(kBlock) void k_quant_mx(const uint16_t* __restrict_
 // any fma, with buffer loads that read zeros past the end, so one wave has
 // 20 x 16 B per lane in flight.  Chunks past H are masked by a select.
 constexpr int kRouterTPW = 4;  // tokens per wave
+constexpr int kTopkBlkMinT = 256;  // from here on k_topk_blk, which then carries the input quantisation
 constexpr int kRouterSteps = 4;  // 512-element chunk steps per load group
 
 // Logits of row r for tokens tb + ts i (i < NT), by one wave, NS chunk steps
@@ -199,6 +200,27 @@ constexpr int kRouterMinT = 64;  // from here on k_router_rows (x re-reads domin
 constexpr double kRouterRowsMinElems = 40e6;
 __host__ __forceinline__ bool router_by_rows(int rows, int T, int H) {
   return T >= kRouterMinT && (double)rows * T * H > kRouterRowsMinElems;
+}
+
+// From here on k_router_mm, unless a third and more of its rows would be
+// padding.  k_router_rows against k_router_mm (us): C3 T=256 / 512 / 1024 /
+// 2048 / 4096 11.5 / 17.7 / 28.8 / 51.5 / 95.5 against 14.9 / 15.4 / 16.7 /
+// 32.4 / 58.5; C2 T=512 / 1024 / 4096 10.0 / 15.2 / 49.3 against 14.6 / 14.5 /
+// 31.7; C4 T=2048 / 4096 13.7 / 23.9 against 18.9 / 20.3; 16 rows of 1024,
+// T=4096 6.6 against 9.4.
+constexpr double kRouterMmMinElems = 250e6;
+constexpr int kRmT = 32;  // tokens and rows of a k_router_mm tile
+
+// Rows that k_router_mm leaves to its waves' own chains (router_row_tile), one
+// row and token at a time: a few past a whole tile (the shared gate's), while
+// that is at most two per wave.
+__host__ __device__ __forceinline__ int router_mm_rest(int rows) {
+  const int tiles = rows / kRmT, rest = rows % kRmT;
+  return 2 * rest <= tiles ? rest : 0;
+}
+__host__ __forceinline__ bool router_by_mm(int rows, int T, int H) {
+  const int padded = (rows - router_mm_rest(rows) + kRmT - 1) / kRmT * kRmT;
+  return T >= kTopkBlkMinT && (double)rows * T * H > kRouterMmMinElems && 3 * rows >= 2 * padded;
 }
 
 // One level of the transposing butterfly: lanes with bit M set keep values
@@ -317,6 +339,116 @@ __global__ __launch_bounds__(kBlock) void k_router_rows(const LayerArgs a, int r
     return;
   }
   router_rows_tile(a, row_begin + blockIdx.x * kRouterRB, row_end, blockIdx.y * 4 * kRouterTPW + wave * kRouterTPW);
+}
+
+// Prefill: the same sums on the fp32 matrix cores.  v_mfma_f32_32x32x1 adds one
+// product to each of 2 x 32 x 32 accumulators with one rounding (an fma), so a
+// wave that keeps one accumulator block per chain l and feeds it the chain's
+// elements in order has k_router's bits, and the two blocks of an instruction
+// are the chains l and l + 32, the butterfly's first pairing.
+// A workgroup takes 32 tokens x 32 rows; wave w has the chains l = w (mod 8):
+// pairings 16 and 8 are between its own accumulators, 4, 2 and 1 between the
+// waves, through LDS.  512 elements of the 64 rows are staged at a time by
+// buffer -> LDS copies, one row each, the next stage's under this one's MFMAs;
+// 16-byte pieces lie at position piece ^ row (low five bits), so that the 32
+// rows' reads of one piece fall on different banks.
+// Bound by the fp32 MFMA rate (131 TF measured, 2 us per stage and workgroup,
+// one workgroup per CU): C3 T=2048 (512 workgroups, two rounds) 32.4 us, 67
+// TF, where k_router_rows takes 51.5 on the vector ALUs.
+constexpr int kRmWaves = 8;
+constexpr int kRmStage = 2 * kRmT * 1024;
+constexpr int kRmLds = 2 * kRmStage;
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
+__global__ __launch_bounds__(64 * kRmWaves) void k_router_mm(const LayerArgs a, int row_begin, int row_end) {
+  extern __shared__ __attribute__((aligned(16))) char rm_lds[];
+  typedef __attribute__((address_space(3))) void* LPtr;
+  const int E = a.L.num_experts, H = a.L.hidden, T = a.T;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rows = row_end - row_begin, rest = router_mm_rest(rows);
+  const int ntt = (T + kRmT - 1) / kRmT, nrt = (rows - rest + kRmT - 1) / kRmT;
+  const int rt = (int)blockIdx.x / ntt;  // consecutive workgroups (XCDs) take different tokens
+  const int t0 = ((int)blockIdx.x - rt * ntt) * kRmT, r0 = row_begin + rt * kRmT, rend = row_end - rest;
+  const int nq = (H + 511) / 512;
+
+  // stage rows 0..31: tokens, 32..63: gate rows; wave w copies rows 8 w .. 8 w + 7
+  auto issue = [&](int q) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int row = 8 * wave + i;
+      const int t = t0 + row, r = r0 + row - kRmT;
+      const char* base = row < kRmT ? (const char*)a.x + (size_t)t * H * 2
+                                    : r < E ? (const char*)a.L.gate_w + (size_t)r * H * 2 : (const char*)a.L.shared_gate;
+      const bool ok = row < kRmT ? t < T : r < rend;
+      const Rsrc res = make_rsrc(base, ok ? (uint32_t)H * 2u : 0u);
+      char* dst = rm_lds + (q & 1) * kRmStage + 1024 * row;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (LPtr)dst, 16, (int)(1024u * (uint32_t)q + 16u * (uint32_t)(lane ^ (row & 31))),
+                                               0, 0, 0);
+    }
+  };
+  issue(0);
+  for (int j = rt * kRmWaves + wave; j < rest * kRmT; j += nrt * kRmWaves) {
+    const int t = t0 + j % kRmT;
+    if (t < T) router_row_tile<false, 1>(a, rend + j / kRmT, t);
+  }
+
+  f32x32 acc[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p)
+#pragma unroll
+    for (int j = 0; j < 32; ++j) acc[p][j] = 0.0f;
+  const int m = lane & 31;
+  for (int q = 0; q < nq; ++q) {
+    wait_vm<0>();    // this wave's copies have landed ...
+    __syncthreads();  // ... and all waves'; the other stage is read up
+    if (q + 1 < nq) issue(q + 1);
+    const char* st = rm_lds + (q & 1) * kRmStage + 1024 * m;
+    u32x4 xv[4], gv[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int pos = (wave + 8 * p + 32 * (lane >> 5)) ^ m;
+      xv[p] = *(const u32x4*)(st + 16 * pos);
+      gv[p] = *(const u32x4*)(st + 1024 * kRmT + 16 * pos);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const uint32_t xw = xv[p][e / 2], gw = gv[p][e / 2];
+        const float xf = __uint_as_float(e & 1 ? xw & 0xffff0000u : xw << 16);
+        const float gf = __uint_as_float(e & 1 ? gw & 0xffff0000u : gw << 16);
+        acc[p] = __builtin_amdgcn_mfma_f32_32x32x1f32(xf, gf, acc[p], 0, 0, 0);
+      }
+  }
+
+  float u[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    float f[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) f[p] = acc[p][j] + acc[p][16 + j];  // 32
+    u[j] = (f[0] + f[2]) + (f[1] + f[3]);                           // 16, 8
+  }
+  float* red = (float*)rm_lds;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; ++j) red[wave * 1024 + j * 64 + lane] = u[j];
+  __syncthreads();
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int idx = tid + 64 * kRmWaves * h, j = idx >> 6;
+    float v[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) v[w] = red[w * 1024 + idx];
+    const float tot = ((v[0] + v[4]) + (v[2] + v[6])) + ((v[1] + v[5]) + (v[3] + v[7]));  // 4, 2, 1
+    const int t = t0 + 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3), r = r0 + m;
+    if (t < T && r < rend) {
+      float z = tot;
+      if (r < E && a.L.gate_b != nullptr) z = tot + bf16_to_f32(((const uint16_t*)a.L.gate_b)[r]);
+      a.logits[(size_t)t * (E + 1) + r] = round_to(z, a.L.act_dtype);
+    }
+  }
 }
 
 // ============================================================== top-k + grouping
@@ -878,7 +1010,6 @@ __global__ __launch_bounds__(kBlock) void k_topk(const LayerArgs a, const void* 
 constexpr int kTopkBlkWaves = 16;
 constexpr int kTopkBlkMaxWG = 128;
 constexpr int kTopkBlkSlots = 8192;  // LDS pair slots per workgroup
-constexpr int kTopkBlkMinT = 256;    // from here on k_topk_blk
 
 __host__ __device__ __forceinline__ int topk_blk_grid(int T, int k) {
   int g = (T + kTopkBlkWaves - 1) / kTopkBlkWaves;
@@ -893,7 +1024,14 @@ template <int MODE, int NV>
 __global__ __launch_bounds__(64 * kTopkBlkWaves) void k_topk_blk(const LayerArgs a, const void* logits_in,
                                                                  int logits_dt, const int32_t* ids_in,
                                                                  const float* w_in, int32_t* ids_out,
-                                                                 float* w_out, float* logits_out) {
+                                                                 float* w_out, float* logits_out, int nwg) {
+  // The input's quantisation, on the CUs that the routing leaves free: C3 T=2048
+  // 11.9 -> 12.6 us here, where it took 6.5 us more in the router's launch (C2
+  // T=4096 32, C4 T=4096 12), whose grid keeps every CU busy.
+  if ((int)blockIdx.x >= nwg) {
+    quant_mx_piece((const uint16_t*)a.x, a.T, a.L.hidden, a.xq, ((int)blockIdx.x - nwg) * 64 * kTopkBlkWaves + threadIdx.x);
+    return;
+  }
   __shared__ int32_t s_cnt[kMaxExperts];    // local pair count, then the reserved base, per expert
   __shared__ int32_t s_slot[kTopkBlkSlots];  // expert | local position << 9 per pair slot, -1: none
   __shared__ int s_last;
@@ -902,7 +1040,7 @@ __global__ __launch_bounds__(64 * kTopkBlkWaves) void k_topk_blk(const LayerArgs
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   for (int e = threadIdx.x; e < E; e += 64 * kTopkBlkWaves) s_cnt[e] = 0;
   __syncthreads();
-  const int stride = kTopkBlkWaves * (int)gridDim.x;
+  const int stride = kTopkBlkWaves * nwg;
   int li = wave;  // local token index: slot base li * k
   // router path: the next token's logits load while this one is routed
   const bool pre = logits_in == nullptr && ids_in == nullptr;
@@ -966,7 +1104,7 @@ __global__ __launch_bounds__(64 * kTopkBlkWaves) void k_topk_blk(const LayerArgs
   // would write back or invalidate the whole L2 of the XCD).
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  if (threadIdx.x == 0) s_last = (atomicAdd(&a.ctrl[kCtrlArriveTopk], 1) == (int)gridDim.x - 1);
+  if (threadIdx.x == 0) s_last = (atomicAdd(&a.ctrl[kCtrlArriveTopk], 1) == nwg - 1);
   __syncthreads();
   if (!s_last) return;
   compact_experts<kTopkBlkWaves>(a, gcnt, true, s_wsum);
@@ -3548,9 +3686,16 @@ hipError_t launch_router(const ftm_moe_layer& L, const void* x, int T, int row_b
   const int tpb = one ? 4 : 4 * kRouterTPW;
   const int ty = (T + tpb - 1) / tpb;
   // quantisation blocks spread over the grid's token-block rows (ceil(nq / ty) columns)
-  const int nq = quant && mx_input(L, T) ? (quant_mx_threads(T, L.hidden) + kBlock - 1) / kBlock : 0;
+  const int nq = quant && T < kTopkBlkMinT && mx_input(L, T) ? (quant_mx_threads(T, L.hidden) + kBlock - 1) / kBlock : 0;
   const int qx = (nq + ty - 1) / ty;
-  if (router_by_rows(row_end - row_begin, T, L.hidden))
+  if (router_by_mm(row_end - row_begin, T, L.hidden)) {
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_router_mm),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kRmLds);
+    if (attr != hipSuccess) return attr;
+    const int rows = row_end - row_begin;
+    hipLaunchKernelGGL(k_router_mm, dim3((rows - router_mm_rest(rows) + kRmT - 1) / kRmT * ((T + kRmT - 1) / kRmT)),
+                       dim3(64 * kRmWaves), kRmLds, st, a, row_begin, row_end);
+  } else if (router_by_rows(row_end - row_begin, T, L.hidden))
     hipLaunchKernelGGL(k_router_rows, dim3((row_end - row_begin + kRouterRB - 1) / kRouterRB + qx, ty),
                        dim3(kBlock), 0, st, a, row_begin, row_end);
   else if (one)
@@ -3599,18 +3744,21 @@ hipError_t launch_route_topk(const ftm_moe_layer& L, const void* x, int T, int32
 
 hipError_t launch_topk(const ftm_moe_layer& L, int T, const void* logits_in, int logits_dt,
                        const int32_t* ids_in, const float* w_in, int32_t* ids_out, float* w_out,
-                       float* logits_out, char* ws, const WsLayout& wl, hipStream_t st) {
-  const LayerArgs a = make_args(L, nullptr, nullptr, T, ws, wl);
+                       float* logits_out, char* ws, const WsLayout& wl, hipStream_t st, const void* x) {
+  const LayerArgs a = make_args(L, x, nullptr, T, ws, wl);
   const bool one = T <= kTopk1MaxT, blk = T >= kTopkBlkMinT;
   const dim3 grid(one ? 1 : (T + 3) / 4), block(one ? 64 * kTopk1Waves : kBlock);
-  const dim3 gblk(topk_blk_grid(T, L.topk)), bblk(64 * kTopkBlkWaves);
+  const int nwg = topk_blk_grid(T, L.topk);
+  const int nq = x != nullptr && blk && mx_input(L, T)
+                     ? (quant_mx_threads(T, L.hidden) + 64 * kTopkBlkWaves - 1) / (64 * kTopkBlkWaves) : 0;
+  const dim3 gblk(nwg + nq), bblk(64 * kTopkBlkWaves);
 #define FTM_TOPK_LAUNCH(M, NV)                                                                                 \
   if (one)                                                                                                     \
     hipLaunchKernelGGL((k_topk1<M, NV>), grid, block, 0, st, a, logits_in, logits_dt, ids_in, w_in, ids_out,    \
                        w_out, logits_out);                                                                     \
   else if (blk)                                                                                                \
     hipLaunchKernelGGL((k_topk_blk<M, NV>), gblk, bblk, 0, st, a, logits_in, logits_dt, ids_in, w_in,           \
-                       ids_out, w_out, logits_out);                                                            \
+                       ids_out, w_out, logits_out, nwg);                                                       \
   else                                                                                                         \
     hipLaunchKernelGGL((k_topk<M, NV>), grid, block, 0, st, a, logits_in, logits_dt, ids_in, w_in, ids_out,     \
                        w_out, logits_out);
@@ -4145,10 +4293,12 @@ static const char* expert_kernel_name_dt(const ftm_moe_layer& L, int T, int stag
 }
 
 const char* stage_kernel_name(const ftm_moe_layer& L, int T, int stage) {
+  const int rows = L.num_experts + (L.shared_inter > 0 ? 1 : 0);
   switch (stage) {
     case FTM_STAGE_ROUTER:
       if (route_topk_fused(L, T)) return "k_route_topk1";
-      return router_by_rows(L.num_experts + (L.shared_inter > 0 ? 1 : 0), T, L.hidden) ? "k_router_rows" : "k_router";
+      if (router_by_mm(rows, T, L.hidden)) return "k_router_mm";
+      return router_by_rows(rows, T, L.hidden) ? "k_router_rows" : "k_router";
     case FTM_STAGE_TOPK:
       if (route_a_ok(L, T) || route_topk_fused(L, T)) return "";  // routed inside stage A / the router
       return T <= kTopk1MaxT ? "k_topk1" : T >= kTopkBlkMinT ? "k_topk_blk" : "k_topk";

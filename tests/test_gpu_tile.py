@@ -99,3 +99,44 @@ def test_tiles_of_few_rows(gpu, fmt, T):
     layer = _check(S.generate(replace(cfg, E=64, k=4, H=256, I=512, shared_inter=0), T=T, seed=T), gpu)
     tile = {"c1_int8": "k_tile", "bf16": "k_tile", "c2_gptq": "k_gemm_mx", "c3_fp8": "k_gemm_mx"}[fmt]
     assert (layer.stage_kernel(T, nat.STAGE_W13) == tile) == (T >= 48)
+
+
+@pytest.mark.parametrize("E,shared,H,T", [
+    (256, True, 2048, 481),   # the shared gate's row beside whole tiles, a token block of one
+    (60, False, 2880, 1480),  # rows padded to a tile, a last stage of 320 elements
+    (62, True, 1024, 3890),   # the shared gate's row inside a padded tile
+    (290, True, 320, 2720),   # one partial stage, 291 rows: three past the tiles
+])
+def test_router_mm_bit_exact(gpu, E, shared, H, T):
+    """The prefill router on the fp32 matrix cores keeps the fma chains and
+    the butterfly that the oracle replays."""
+    from ftmoe.banks import Proj
+    from ftmoe.layer import MoeLayer
+
+    I, k = 16, 4
+    rng = np.random.RandomState(E + T)
+    bits = lambda v: O.f32_to_bf16_bits(v.astype(np.float32))  # noqa: E731
+    dev = lambda b: torch.from_numpy(b.view(np.int16)).view(torch.bfloat16).to(gpu)  # noqa: E731
+    gate, x = bits(rng.randn(E, H) * 0.05), bits(rng.randn(T, H))
+    sgate, s13, s2 = bits(rng.randn(1, H) * 0.05), bits(rng.randn(2 * I, H) * 0.05), bits(rng.randn(H, I))
+    shd = {"w13": dev(s13), "w2": dev(s2), "gate": dev(sgate)} if shared else None
+    w13 = Proj("bf16", torch.zeros(E, 2 * I, H, dtype=torch.bfloat16, device=gpu), 2 * I, H)
+    w2 = Proj("bf16", torch.zeros(E, H, I, dtype=torch.bfloat16, device=gpu), H, I)
+    layer = MoeLayer(w13=w13, w2=w2, num_experts=E, hidden=H, inter=I, topk=k, gate_w=dev(gate), shared=shd,
+                     act_dtype=torch.bfloat16)
+    assert layer.stage_kernel(T, nat.STAGE_ROUTER) == "k_router_mm"
+    out, ids, w, logits = layer.forward(dev(x), return_routing=True)
+    torch.cuda.synchronize()
+    ref = O.router_logits(x, gate)
+    rid, rw = O.route(ref, k, "softmax_topk", True)
+    np.testing.assert_array_equal(to_f32(logits), ref)
+    np.testing.assert_array_equal(ids.cpu().numpy(), rid)
+    np.testing.assert_array_equal(w.cpu().numpy(), rw)
+    if shared:  # zero banks: the output is the shared expert's, times its gate
+        f = lambda b: torch.from_numpy(b.view(np.int16)).view(torch.bfloat16).double()  # noqa: E731
+        gu = f(x) @ f(s13).t()
+        h = (torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]).bfloat16().double()
+        want = (h @ f(s2).t()) * torch.sigmoid((f(x) @ f(sgate).t()).bfloat16().double())
+        assert rel_rms(to_f32(out), want.numpy()) < 2 * REL_RMS  # the gate's own rounding as well
+    else:
+        assert torch.count_nonzero(out) == 0
