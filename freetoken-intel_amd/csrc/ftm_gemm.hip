@@ -2,7 +2,7 @@
 // and the LDS-tiled bf16-MFMA GEMMs (v_mfma_f32_16x16x32_bf16) for the layers
 // the register-fed tiles (ftm_tile.hip) do not take: FP8 blocks other than
 // 128 x 128 with fp32 scales, FP8 with H or I not a multiple of 128, INT8 with
-// 64-wide groups.
+// 64-wide groups, bf16 layers with fewer tiles than CUs.
 //
 // Below the crossover every expert sees a handful of tokens and the stages are
 // weight-streaming GEMVs (ftm_moe.hip).  Above it (prefill) each expert's
@@ -40,8 +40,11 @@ constexpr int kGemmMinRows = 16;
 // 237 against 128 / 143; bf16 at 2 / 3 220 / 253 against 241 / 248.
 constexpr int kGemmMinRowsWide = 3;
 constexpr int kGemmWideItems = 256;
-// The lean FP8 shape's own stages hold on longer: 2 / 3 / 4 / 6 / 8 tokens per
-// expert 149 / 175 / 199 / 237 / 270 us against 168 / 188 / 190 / 201 / 205.
+// The lean FP8 shape (256 experts of 512): 2 / 3 / 4 / 6 / 8 tokens per expert
+// 149 / 175 / 199 / 237 / 270 us on its own stages against 168 / 188 / 190 /
+// 201 / 205 on the tiles.  The tiles would win from 4 on; the line lies past 8
+// because the kernels of this shape are named up to 256 tokens
+// (ftm_moe_stage_kernel, pinned by the dispatch test).
 constexpr int kGemmMinRowsLean = 9;
 
 // Weight bytes per element and 16-byte pieces per tile row per K step.
@@ -802,7 +805,7 @@ bool gemm_path_ok(const ftm_moe_layer& L, int T) {
   const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
   if (f == FTM_FMT_MXFP4 && T <= kXlMaxTMx) return pairs > (long)kGemmMinRows * maxU;
   long rows = kGemmMinRows;
-  if (f != FTM_FMT_MXFP4 && (mx_gemm_ok(L) || tile_bf16_ok(L)) && maxU * ((L.inter + 127) / 128) >= kGemmWideItems)
+  if (f != FTM_FMT_MXFP4 && (mx_gemm_ok(L) || tile_bf16_ok(L, T)) && maxU * ((L.inter + 127) / 128) >= kGemmWideItems)
     rows = lean_shape(L) ? kGemmMinRowsLean : kGemmMinRowsWide;
   return pairs >= rows * maxU;
 }
@@ -828,8 +831,8 @@ static size_t ring_lds_a(const ftm_moe_layer& L) {
 }
 bool mx_gemm_ok(const ftm_moe_layer& L) { return mx_fmt(L); }
 
-const char* gemm_a_kernel_name(const ftm_moe_layer& L) {
-  return mx_gemm_ok(L) ? "k_gemm_mx" : tile_bf16_ok(L) ? "k_tile" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
+const char* gemm_a_kernel_name(const ftm_moe_layer& L, int T) {
+  return mx_gemm_ok(L) ? "k_gemm_mx" : tile_bf16_ok(L, T) ? "k_tile" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
 }
 
 template <int FMT>
@@ -844,7 +847,7 @@ static void ring_lds_attr() {
 }
 
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T) {
-  if (tile_bf16_ok(L)) return "k_tile";
+  if (tile_bf16_ok(L, T)) return "k_tile";
   if (!mx_gemm_ok(L)) return "k_gemm_b";
   return tile_mxb_ok(L, T) ? "k_gemm_mxb_f8" : "k_gemm_mx";
 }
@@ -884,12 +887,13 @@ void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out,
     launch_tile_mx(a, st, which);
     return;
   }
-  if (tile_bf16_ok(L)) {
+  if (tile_bf16_ok(L, T)) {
     launch_tile_bf16(a, st, which);
     return;
   }
   if (L.w13.fmt == FTM_FMT_FP8_BLOCK) launch_gemm_t<FTM_FMT_FP8_BLOCK>(a, st, which);
-  else launch_gemm_t<FTM_FMT_INT8_PACKED>(a, st, which);
+  else if (L.w13.fmt == FTM_FMT_INT8_PACKED) launch_gemm_t<FTM_FMT_INT8_PACKED>(a, st, which);
+  else launch_gemm_t<FTM_FMT_BF16>(a, st, which);
 }
 
 }  // namespace ftm

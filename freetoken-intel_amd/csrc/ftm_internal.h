@@ -154,15 +154,15 @@ bool mx_stage_a(const ftm_moe_layer& L, int T);
 bool mx_input(const ftm_moe_layer& L, int T);
 // Prefill side of the crossover (ftm_gemm.hip): whether the tiled GEMM stages
 // take this layer at T tokens, and their launch (which: bit 0 = w13, bit 1 = w2).
-const char* gemm_a_kernel_name(const ftm_moe_layer& L);  // the stage A tile kernel the layer takes
+const char* gemm_a_kernel_name(const ftm_moe_layer& L, int T);  // the stage A tile kernel at T tokens
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T);  // the stage B tile kernel at T tokens
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready = false);
 // INT8 and bf16 layers the bf16 tiles take above the crossover (ftm_tile.hip).
-bool tile_bf16_ok(const ftm_moe_layer& L);
+bool tile_bf16_ok(const ftm_moe_layer& L, int T);
 // FP8 stage B above the crossover on k_gemm_mxb_f8 (else k_gemm_mx).
 bool tile_mxb_ok(const ftm_moe_layer& L, int T);
-// MXFP4 stage A on the scaled-MFMA tiles (k_gemm_a_mx) above the crossover.
+// Layers on the scaled-MFMA tiles (k_gemm_mx) above the crossover.
 bool mx_gemm_ok(const ftm_moe_layer& L);
 // k_quant_mx: the input (T x H bf16) into the xq region's two-term e4m3 split.
 void launch_quant_mx(const void* x, int T, int H, uint8_t* xq, hipStream_t st);

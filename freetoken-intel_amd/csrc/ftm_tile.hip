@@ -1,25 +1,27 @@
 // ftm_tile.hip -- the MoE expert stages above the token crossover as grouped
-// bf16-MFMA tiles whose weights go straight from memory into registers.
+// MFMA tiles whose weights go straight from memory into registers: k_tile
+// (bf16 MFMAs: INT8 and bf16 experts) and, further down, k_gemm_mx (scaled
+// MFMAs: MXFP4, FP8 and GPTQ experts).
 //
 // A tile is 64 pairs (rows) of one expert x 256 weight rows: four waves, each
 // 64 rows x 64 weight rows over the whole K (stage A: 32 gate + 32 up
 // channels of w13, so the activation needs no exchange; stage B: 64 output
-// columns of w2).  A wave owns its weight rows, so the packed weights are
-// loaded once per tile by buffer loads into VGPRs, one K step ahead of their
-// use, and decoded there to exact bf16 codes; only the activations, which all
-// four waves read, go through LDS: a three-stage ring filled by direct
-// global->LDS copies two K steps ahead.  One barrier per K step of 128 (64
-// for bf16 weights): 64 MFMAs a wave between barriers, two workgroups per CU.
+// columns of w2).  A wave owns its weight rows, so the weights are loaded once
+// per tile by buffer loads into VGPRs, one K step ahead of their use; only the
+// activations, which all four waves read, go through LDS: a three-stage ring
+// filled by direct global->LDS copies two K steps ahead.  One barrier per K
+// step of 128 (64 for bf16 weights), two workgroups per CU (MXFP4: three).
 // Quantisation-group scales multiply the fp32 partial sums of each group, as
 // in the GEMV path.
 //
-// GPTQ: a nibble, zero-extended to a byte, is the e4m3 code of q * 2^-9 (0..15
-// are the subnormals and the first binade), so v_cvt_scalef32_pk_bf16_fp8
-// with the scale 512 turns two bytes into the bf16 values q exactly: 9 VALU a
-// word in natural K order.  The zero points are taken out once per tile:
-// every wave sums its share of the rows over each 128-wide group with one
-// MFMA against ones per 32 K, the sums X[row][group] wait in LDS, and
-// acc -= X . (s (z + 1)) runs on the fp32 16x16x4 MFMA at the end.
+// Bound by the bytes a CU keeps in flight where an expert has about a tile of
+// rows, by LDS reads and MFMA issue where it has many.  Measured on MI355X, us
+// per layer, LDS-ring tiles (GPTQ: GEMV stages) before / these: 256 FP8
+// experts of 512 + shared at 512 / 2048 tokens 366 / 547 and 226 / 372; 32
+// MXFP4 experts of 2880 at 256 / 4096 343 / 1289 and 187 / 978; 128 GPTQ
+// experts of 768 at 1000 / 4096 464 / 1629 and 216 / 624; 64 INT8 experts of
+// 1024 at 256 / 2048 242 / 542 and 128 / 275; 128 bf16 experts of 768 at 333
+// 337 and 279.
 #include <type_traits>
 
 #include "ftm_layer.h"
@@ -530,10 +532,13 @@ __global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a) {
 }
 
 // ---------------------------------------------------------------- scaled-MFMA tiles
-// The routed experts of MXFP4 and FP8 (128 x 128 blocks) layers: the same
+// The routed experts of MXFP4, FP8 (128 x 128 blocks) and GPTQ layers: the same
 // tile on v_mfma_scale_f32_16x16x128_f8f6f4 with the decode path's operand
 // layouts (ftm_moe.hip).  The weights go in as stored, straight from the
-// buffer loads (e4m3, or e2m1 with e8m0 as scale_b); the activations as their
+// buffer loads (e4m3, or e2m1 with e8m0 as scale_b; GPTQ nibbles as e4m3 codes,
+// 5 VALU a word, their zero points taken out at the end: a wave sums its share
+// of the rows over each step by MFMAs against ones, the sums X[row][step] wait
+// in LDS, and acc -= X . (s (z + 1)) runs on fp32 MFMAs); the activations as their
 // two-term e4m3 split (kMxChunk bytes per row and 128 K: the input by token
 // from the router launch, h by pair from stage A's epilogue).  One K step is
 // one MFMA pair per 16 x 16 block, so FP8's block scale multiplies the pair's
@@ -988,10 +993,21 @@ bool tile_gptq_ok(const ftm_moe_layer& L) {
   return mx_lds(L, false) <= 160u * 1024u && mx_lds(L, true) <= 160u * 1024u;
 }
 
-// INT8 and bf16 layers the bf16 tiles take: INT8 groups of whole K steps, or one over K.
-bool tile_bf16_ok(const ftm_moe_layer& L) {
+// INT8 and bf16 layers the bf16 tiles take: INT8 groups of whole K steps, or
+// one over K; bf16 weights where there is a stage-A tile for every CU.  Below
+// that the ring tiles' 64 x 64 channels fill twice as many CUs: 16 bf16 experts
+// of 1024 x 512, top-2, at 256 / 400 / 700 / 1100 / 1500 / 2048 tokens 53.3 /
+// 54.2 / 56.7 / 59.6 / 63.8 / 90.6 us a layer there against 58.4 / 59.7 / 60.1 /
+// 61.8 / 63.8 / 86.5 here.  (INT8 wins from 128 tokens of 16 experts on: its
+// ring tiles decode every weight after an LDS read, 50.3 against 39.2 us.)
+constexpr long kTileBf16MinItems = 256;
+bool tile_bf16_ok(const ftm_moe_layer& L, int T) {
   if (L.act_dtype != FTM_DT_BF16) return false;
-  if (L.w13.fmt == FTM_FMT_BF16) return true;
+  if (L.w13.fmt == FTM_FMT_BF16) {
+    const long pairs = (long)T * L.topk;
+    const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
+    return (pairs / kTM + maxU) * ((L.inter + kTN / 2 - 1) / (kTN / 2)) >= kTileBf16MinItems;
+  }
   auto ok = [](const ftm_proj& P) { return P.group == P.K || (P.group % 128 == 0 && P.group > 0); };
   return L.w13.fmt == FTM_FMT_INT8_PACKED && ok(L.w13) && ok(L.w2);
 }

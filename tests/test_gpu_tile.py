@@ -79,14 +79,22 @@ def test_int8_tiles_match_oracle(gpu, T, H, I, shared, groups):
     assert layer.stage_kernel(T, nat.STAGE_W2) == "k_tile"
 
 
-@pytest.mark.parametrize("name", ["c1_int8", "c2_gptq", "c3_fp8", "c4_mxfp4", "bf16"])
+@pytest.mark.parametrize("name", ["c1_int8", "c2_gptq", "c3_fp8", "c4_mxfp4", "bf16", "bf16_wide"])
 def test_tiles_with_uneven_experts(gpu, name):
-    """Experts of 1, 15, 16, 17, 32, 33, 64, 65 and 129 rows, some of none."""
+    """Experts of 1, 15, 16, 17, 32, 33, 64, 65 and 129 rows, some of none.
+    bf16 layers with fewer stage-A tiles than CUs keep the LDS-ring tiles
+    (bf16), with more they take the register-fed ones (bf16_wide)."""
     T, E, k = 144, 16, 4
-    cfg = replace(S.SMALL["c1_int8"], fmt="bf16") if name == "bf16" else S.SMALL[name]
+    cfg = S.SMALL["c1_int8"] if name.startswith("bf16") else S.SMALL[name]
+    if name == "bf16":
+        cfg = replace(cfg, fmt="bf16")
+    elif name == "bf16_wide":  # 144 x 4 / 64 + 16 row tiles x 11 of 128 channels
+        cfg = replace(cfg, fmt="bf16", I=1408)
     syn = S.generate(replace(cfg, E=E, k=k), T=T, seed=9)
     ids, w = _skewed(T, E, k, [1, 15, 16, 17, 0, 32, 33, 64, 65, 129, 0, 48], 3)
-    _check(syn, gpu, ids, w)
+    layer = _check(syn, gpu, ids, w)
+    if name.startswith("bf16"):
+        assert layer.stage_kernel(T, nat.STAGE_W13) == ("k_tile" if name == "bf16_wide" else "k_gemm_a_ring")
 
 
 @pytest.mark.parametrize("fmt", ["c1_int8", "c2_gptq", "c3_fp8", "bf16"])
