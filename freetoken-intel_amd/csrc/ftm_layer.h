@@ -1,6 +1,6 @@
 // ftm_layer.h -- the per-call argument block of the layer kernels and the small
-// device helpers shared by the decode kernels (ftm_moe.hip) and the tiled
-// prefill GEMMs (ftm_gemm.hip).
+// device helpers shared by the decode kernels (ftm_moe.hip) and the prefill
+// tiles (ftm_tile.hip, ftm_gemm.hip).
 #pragma once
 
 #include <math.h>
