@@ -246,3 +246,34 @@ def test_fp8_e5m2_linear_matches_dequant_then_matmul(gpu, m, k, n):
     # the reference's dequant (fp8_block_linear.py:48-91): fp32(w) times its block's scale
     dense = w.float() * torch.repeat_interleave(torch.repeat_interleave(s, 128, 0), 128, 1)[:n, :k]
     _check(got, x, dense.numpy(), 2e-3, 2e-2)
+
+
+@pytest.mark.parametrize("m", [1, 16, 33])
+@pytest.mark.parametrize("fmt,k,n", [("fp8", 128, 64), ("fp8", 384, 200), ("fp8", 640, 72), ("int8", 64, 40),
+                                     ("int8", 448, 136), ("mxfp4", 32, 24), ("mxfp4", 416, 72)])
+def test_linear_k_split(gpu, fmt, k, n, m):
+    """K split over a workgroup's four waves: waves without a range (one or two
+    wave-loads of K), ranges that begin and end inside a scale group, a last
+    wave-load partly past K, rows and columns past a block.  fp32 activations
+    enter as two bf16 terms (2^-17 of each product) and the fp32 sums lose at
+    most 2^-24 a step."""
+    g = torch.Generator().manual_seed(k + n)
+    w = torch.randn(n, k, generator=g) * 0.1
+    x = torch.randn(m, k, generator=g)
+    if fmt == "fp8":
+        wq, s = quant.quantize_block_fp8(w, block=128)
+        got = fused_fp8_linear(x.to(gpu), wq.to(gpu), s.to(gpu), block=128)
+        wd = O.dequantize_block_fp8(np_(wq), s.numpy(), 128)
+    elif fmt == "int8":
+        s = (w.abs().amax(dim=1, keepdim=True) / 127.0).clamp_min(1e-12)
+        q = (w / s).round().clamp(-127, 127)
+        wq = (q + 128).to(torch.uint8).contiguous().view(torch.int32)
+        got = fused_int8_linear(x.to(gpu), wq.to(gpu), s.to(gpu), k=k)
+        wd = q.double().numpy() * s.double().numpy()
+    else:
+        b, s = quant.quantize_mxfp4_blocks(w)
+        got = fused_mxfp4_linear(x.to(gpu), b.to(gpu), s.to(gpu))
+        wd = O.dequantize_mxfp4_blocks(b.numpy(), s.numpy())
+    xd, wd = x.double().numpy(), wd.astype(np.float64)
+    bound = (2.0 ** -17 + (k + 8) * 2.0 ** -24) * (np.abs(xd) @ np.abs(wd).T)
+    assert (np.abs(got.double().cpu().numpy() - xd @ wd.T) <= bound).all()
