@@ -79,11 +79,16 @@ struct TileSrc {
 // The K loop of the bf16 tiles: acc += A (16 MI rows) . W^T over the whole K.
 // Every step issues the same loads (past the last step through clamped or
 // out-of-range offsets), so the counted waits are exact.
-template <int FMT, int MODE, int MI, bool BIG>
+// bf16 weights, MFMA sub-step q, lane group g: stage A takes activation piece
+// 2 g + q of the step, stage B piece 4 q + g.  Those are the sums, in their
+// order, of the LDS tiles (k_gemm_a_ring, k_gemm_b), so a token's output does
+// not depend on which of the two the batch's size chose.
+template <int FMT, int MODE, int MI, bool STB, bool BIG>
 __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[2], const char* abase, uint32_t abytes,
                                            const TileSrc<TileFmt<FMT>::kACopies>& src, char* lds, f32x4 (&acc)[MI][4]) {
   using F = TileFmt<FMT>;
   constexpr bool I8 = FMT == FTM_FMT_INT8_PACKED;
+  constexpr bool PAIR = FMT == FTM_FMT_BF16 && !STB;  // a lane's two pieces are neighbours
   constexpr int KS = F::kKS, NA = F::kACopies;
   constexpr int NW = 8 + (MODE == kScale128 ? 4 : 0);  // weight and scale loads a step
   typedef __attribute__((address_space(1))) const void* GPtr;
@@ -126,7 +131,7 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) {
     const int row = tile_row(base, nj, m);
-    woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
+    woff[nj] = row < N ? (uint32_t)row * rb + (PAIR ? 32u : 16u) * (uint32_t)g : kOOB;
   }
   // index of the scale of block nj in step kb (rows past N: past the end)
   auto sidx = [&](int kb, int nj) {
@@ -138,8 +143,8 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
       for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload4(sres, (sesz * sidx(kb < nsteps ? kb : 0, nj)) & ~3u);
     }
   };
-  auto load_w = [&](int kb, int i, Wgt& t) {  // 64 bytes of each row
-    const uint32_t ko = kb * KS + (I8 ? 64 : 32) * i < K ? (uint32_t)kb * 128u + 64u * (uint32_t)i : kOOB;
+  auto load_w = [&](int kb, int i, Wgt& t) {  // 64 bytes of each row (bf16: K is whole steps)
+    const uint32_t ko = kb * KS + (I8 ? 64 : 32) * i < K ? (uint32_t)kb * 128u + (PAIR ? 16u : 64u) * (uint32_t)i : kOOB;
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) t.w[nj][i] = bload16(wres, woff[nj] + ko);
   };
@@ -169,11 +174,11 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
     for (auto& r : p)
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) r[nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    // sub-step q's operand: activation piece 4 q + g (INT8: 8 (q / 2) + 2 g +
-    // q % 2, the 16 K of a lane's weight bytes); read during the MFMAs of the
-    // sub-step before
+    // sub-step q's operand: activation piece 4 q + g (PAIR: 2 g + q; INT8: 8 (q
+    // / 2) + 2 g + q % 2, the 16 K of a lane's weight bytes); read during the
+    // MFMAs of the sub-step before
     auto frag = [&](int q, u32x4(&a)[MI]) {
-      const int piece = I8 ? 8 * (q >> 1) + 2 * g + (q & 1) : 4 * q + g;
+      const int piece = I8 ? 8 * (q >> 1) + 2 * g + (q & 1) : PAIR ? 2 * g + q : 4 * q + g;
 #pragma unroll
       for (int mi = 0; mi < MI; ++mi) {
         const int r = 16 * mi + m;
@@ -369,7 +374,7 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  tile_kloop<FMT, MODE, MI, BIG>(W, base, abase, abytes, src, lds, acc);
+  tile_kloop<FMT, MODE, MI, STB, BIG>(W, base, abase, abytes, src, lds, acc);
 
   const int lb[2] = {(STB ? 64 : 32) * wave, STB ? 64 * wave + 32 : kTN / 2 + 32 * wave};
   float bf[4];

@@ -148,3 +148,41 @@ def test_router_mm_bit_exact(gpu, E, shared, H, T):
         assert rel_rms(to_f32(out), want.numpy()) < 2 * REL_RMS  # the gate's own rounding as well
     else:
         assert torch.count_nonzero(out) == 0
+
+
+@pytest.mark.parametrize("H", [256, 320])
+def test_bf16_output_does_not_depend_on_the_tile_kind(gpu, H):
+    """The register-fed tiles (144 tokens: 275 stage-A tiles) and the LDS-ring
+    ones (their first 80 tokens: 231) sum in the same order: the same bits."""
+    cfg = replace(S.SMALL["c1_int8"], fmt="bf16", E=16, k=4, H=H, I=1408)
+    syn = S.generate(cfg, T=144, seed=H).to(gpu)
+    layer = S.build_layer(syn)
+    assert layer.stage_kernel(144, nat.STAGE_W13) == "k_tile" and layer.stage_kernel(80, nat.STAGE_W13) == "k_gemm_a_ring"
+    out, part = layer.forward(syn.x), layer.forward(syn.x[:80].contiguous())
+    torch.cuda.synchronize()
+    assert torch.equal(out[:80], part)
+
+
+@pytest.mark.parametrize("fmt,kernel", [("c3_fp8", "k_gemm_mx"), ("c1_int8", "k_tile")])
+def test_shared_expert_bits_beside_any_experts(gpu, fmt, kernel):
+    """Routed banks of zeros leave the shared expert's output: beside FP8 and
+    INT8 tiles the same bits as beside bf16 experts on the LDS-ring tiles."""
+    T, H, Is = 200, 384, 192
+    outs = []
+    for f, I, want in ((fmt, 128, kernel), ("bf16", 64, "k_gemm_a_ring")):
+        cfg = S.SMALL["c1_int8"] if f == "bf16" else S.SMALL[f]
+        cfg = replace(cfg, fmt=f if f == "bf16" else cfg.fmt, E=8, k=2, H=H, I=I, shared_inter=Is)
+        syn = S.generate(cfg, T=T, seed=1)
+        for n, t in syn.bank.items():
+            if f == "bf16" or n.startswith(("scale", "weight_scale")):
+                t.zero_()
+        if outs:
+            syn.x, syn.gate_w, syn.shared = first.x, first.gate_w, first.shared
+        first = syn
+        dsyn = syn.to(gpu)
+        layer = S.build_layer(dsyn)
+        assert layer.stage_kernel(T, nat.STAGE_W13) == want
+        outs.append(layer.forward(dsyn.x))
+    torch.cuda.synchronize()
+    assert torch.count_nonzero(outs[0]) > 0
+    assert torch.equal(outs[0], outs[1])
