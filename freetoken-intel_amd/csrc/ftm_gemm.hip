@@ -34,8 +34,8 @@ constexpr int kGemmMinRows = 16;
 // Register-fed tiles that cover the chip (at least kGemmWideItems stage-A
 // tiles, one per CU) read the weights once at a higher rate than the GEMV
 // stages, which read them again for every few tokens.  Measured on MI355X (us
-// per layer, GEMV stages / tiles): GPTQ 128 experts of 768 at 2 / 3 / 8 tokens
-// per expert 103 / 124 / 136 against 101 / 104 / 110; 64 INT8 experts of 1024
+// per layer, GEMV stages / tiles): GPTQ 128 experts of 768 at 3 / 8 tokens per
+// expert 126 / 139 against 103 / 111; 64 INT8 experts of 1024
 // at 2 / 8 132 / 172 against 112 / 123; 64 FP8 experts of 1024 at 3 / 12 162 /
 // 237 against 128 / 143; bf16 at 2 / 3 220 / 253 against 241 / 248.
 constexpr int kGemmMinRowsWide = 3;

@@ -76,15 +76,14 @@ __host__ __device__ inline int mx_row_bytes(int H) { return (H + 127) / 128 * kM
 // An internal flag of w13 (ftm_proj.flags): no tiles, so no quantised copies in
 // the workspace (ftm_moe_forward_noalloc, where they would not fit its scratch).
 constexpr int kProjNoTiles = 1 << 30;
-bool tile_gptq_ok(const ftm_moe_layer& L);  // GPTQ layers the scaled-MFMA tiles take (ftm_tile.hip)
+bool tile_gptq_ok(const ftm_moe_layer& L);  // GPTQ layers the bf16 tiles take (ftm_tile.hip)
 bool gemm_path_ok(const ftm_moe_layer& L, int T);
-// Weight formats the scaled-MFMA stages take (bf16 activations): MXFP4, GPTQ
-// with 128-wide groups, and FP8 e4m3 with 128 x 128 blocks (the block scale applied to each K step's
+// Weight formats the scaled-MFMA stages take (bf16 activations): MXFP4, and
+// FP8 e4m3 with 128 x 128 blocks (the block scale applied to each K step's
 // partial sums).
 inline bool mx_fmt(const ftm_moe_layer& L) {
   if (L.act_dtype != FTM_DT_BF16) return false;
   if (L.w13.fmt == FTM_FMT_MXFP4) return true;
-  if (L.w13.fmt == FTM_FMT_GPTQ_INT4) return tile_gptq_ok(L);
   return L.w13.fmt == FTM_FMT_FP8_BLOCK && L.w13.group == 128 && L.w2.group == 128 &&
          L.w13.s_dtype == FTM_DT_F32 && L.w2.s_dtype == FTM_DT_F32 && L.hidden % 128 == 0 && L.inter % 128 == 0;
 }
@@ -158,7 +157,7 @@ const char* gemm_a_kernel_name(const ftm_moe_layer& L, int T);  // the stage A t
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T);  // the stage B tile kernel at T tokens
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready = false);
-// INT8 and bf16 layers the bf16 tiles take above the crossover (ftm_tile.hip).
+// GPTQ, INT8 and bf16 layers the bf16 tiles take above the crossover (ftm_tile.hip).
 bool tile_bf16_ok(const ftm_moe_layer& L, int T);
 // FP8 stage B above the crossover on k_gemm_mxb_f8 (else k_gemm_mx).
 bool tile_mxb_ok(const ftm_moe_layer& L, int T);

@@ -1,7 +1,7 @@
 // ftm_tile.hip -- the MoE expert stages above the token crossover as grouped
 // MFMA tiles whose weights go straight from memory into registers: k_tile
-// (bf16 MFMAs: INT8 and bf16 experts) and, further down, k_gemm_mx (scaled
-// MFMAs: MXFP4, FP8 and GPTQ experts).
+// (bf16 MFMAs: GPTQ, INT8 and bf16 experts) and, further down, k_gemm_mx
+// (scaled MFMAs: MXFP4 and FP8 experts).
 //
 // A tile is 64 pairs (rows) of one expert x 256 weight rows: four waves, each
 // 64 rows x 64 weight rows over the whole K (stage A: 32 gate + 32 up
@@ -19,9 +19,17 @@
 // per layer, LDS-ring tiles (GPTQ: GEMV stages) before / these: 256 FP8
 // experts of 512 + shared at 512 / 2048 tokens 366 / 547 and 226 / 372; 32
 // MXFP4 experts of 2880 at 256 / 4096 343 / 1289 and 187 / 978; 128 GPTQ
-// experts of 768 at 1000 / 4096 464 / 1629 and 216 / 624; 64 INT8 experts of
+// experts of 768 at 1000 / 4096 466 / 1613 and 213 / 550; 64 INT8 experts of
 // 1024 at 256 / 2048 242 / 542 and 128 / 275; 128 bf16 experts of 768 at 333
 // 337 and 279.
+//
+// GPTQ's activations stay the bf16 values that the GEMV stages read (a
+// two-term e4m3 split of them takes the same time, 209 us at 1000 tokens, but
+// drops what lies 2^13 below a 32-block's largest: with one channel of 128 at
+// 1e4 and weights that do not read it the others' result is off by 0.3).  The
+// zero points leave after the loop, acc -= X . (s (z + 1)) on fp32 MFMAs, X the
+// row sums of each step, which a wave takes for its share of the rows by MFMAs
+// against ones and keeps in LDS.
 #include <type_traits>
 
 #include "ftm_layer.h"
@@ -34,7 +42,7 @@ constexpr int kTHPitch = 128 * 2 + 16;  // bytes of a staged h row (stage A's ep
 constexpr int kTStages = 3;    // activation stages in LDS
 
 // How group scales enter: none (bf16), one group over K (applied after the
-// loop), one per K step of 128.
+// loop), one per K step of 128 (GPTQ: with its zero points after the loop).
 enum { kScaleNone = 0, kScaleOne = 1, kScale128 = 2 };
 
 template <int FMT>
@@ -69,6 +77,46 @@ __device__ __forceinline__ float half_word(uint32_t w, int hi, int dt) {
   return dt == FTM_DT_F16 ? f : b;
 }
 
+// One step's packed weights of a wave and the raw words of its scales.
+template <int FMT>
+struct TileW {
+  u32x4 w[4][2];
+  uint32_t s[4];
+};
+template <>
+struct TileW<FTM_FMT_GPTQ_INT4> {
+  u32x2 w[2][4];  // [half][q]: the words of columns 2m, 2m + 1 at K 32 q + 8 g
+  uint32_t s[2];  // [half]: both columns' 16-bit scales
+};
+
+// Eight nibbles (low first) -> the bf16 values 0..15 in natural order, 9 VALU:
+// a nibble, zero-extended to a byte, is the e4m3 code of q 2^-9 (0..15 are the
+// subnormals and the first binade), which the scaled convert makes q exactly.
+__device__ __forceinline__ u32x4 gptq_word_natural(uint32_t w) {
+  const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;  // q0 q2 q4 q6 / q1 q3 q5 q7
+  const uint32_t a = __builtin_amdgcn_perm(hi, lo, 0x05010400u);     // q0 q1 q2 q3
+  const uint32_t b = __builtin_amdgcn_perm(hi, lo, 0x07030602u);     // q4 q5 q6 q7
+  auto pair = [](uint32_t v, auto hi_half) {
+    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8((int)v, 512.0f, hi_half()));
+  };
+  using L = std::integral_constant<bool, false>;
+  using H = std::integral_constant<bool, true>;
+  return (u32x4){pair(a, L{}), pair(a, H{}), pair(b, L{}), pair(b, H{})};
+}
+
+// The bf16 operand of column block nj in sub-step q.
+template <int FMT>
+__device__ __forceinline__ u32x4 tile_weights(const TileW<FMT>& t, int nj, int q) {
+  if constexpr (FMT == FTM_FMT_GPTQ_INT4) {
+    return gptq_word_natural((nj & 1) ? t.w[nj >> 1][q].y : t.w[nj >> 1][q].x);
+  } else if constexpr (FMT == FTM_FMT_INT8_PACKED) {
+    const u32x4 r = t.w[nj][q >> 1];
+    return i8x8_to_bf16(q & 1 ? r.z : r.x, q & 1 ? r.w : r.y);
+  } else {
+    return t.w[nj][q];
+  }
+}
+
 // Activation sources of a wave's copies: byte offsets into the buffer (BIG:
 // addresses).
 template <int N>
@@ -85,12 +133,14 @@ struct TileSrc {
 // not depend on which of the two the batch's size chose.
 template <int FMT, int MODE, int MI, bool STB, bool BIG>
 __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[2], const char* abase, uint32_t abytes,
-                                           const TileSrc<TileFmt<FMT>::kACopies>& src, char* lds, f32x4 (&acc)[MI][4]) {
+                                           const TileSrc<TileFmt<FMT>::kACopies>& src, char* lds, float* Xs,
+                                           f32x4 (&acc)[MI][4]) {
   using F = TileFmt<FMT>;
-  constexpr bool I8 = FMT == FTM_FMT_INT8_PACKED;
+  constexpr bool I8 = FMT == FTM_FMT_INT8_PACKED, GQ = FMT == FTM_FMT_GPTQ_INT4;
+  constexpr bool ONESET = MODE == kScale128;  // one register set of weights (below)
   constexpr bool PAIR = FMT == FTM_FMT_BF16 && !STB;  // a lane's two pieces are neighbours
   constexpr int KS = F::kKS, NA = F::kACopies;
-  constexpr int NW = 8 + (MODE == kScale128 ? 4 : 0);  // weight and scale loads a step
+  constexpr int NW = 8 + (GQ ? 2 : MODE == kScale128 ? 4 : 0);  // weight and scale loads a step
   typedef __attribute__((address_space(1))) const void* GPtr;
   typedef __attribute__((address_space(3))) void* LPtr;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -118,39 +168,50 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
     }
   };
 
-  struct Wgt {
-    u32x4 w[4][2];
-    uint32_t s[4];
-  };
+  using Wgt = TileW<FMT>;
   const uint32_t rb = I8 ? (uint32_t)K : 2u * (uint32_t)K;
-  const Rsrc wres = make_rsrc(W.w, rb * (uint32_t)N);
+  const Rsrc wres = make_rsrc(W.w, GQ ? (uint32_t)(K / 8) * (uint32_t)N * 4u : rb * (uint32_t)N);
   const uint32_t sesz = W.s_dt == FTM_DT_F32 ? 4u : 2u;
-  const int ngrp = I8 ? K / W.group : 0;
+  const int ngrp = I8 || GQ ? K / W.group : 0;
   const Rsrc sres = make_rsrc(W.s, (uint32_t)(N * ngrp) * sesz);
-  uint32_t woff[4];
+  uint32_t woff[4];  // GPTQ: [0] and [2], the halves' first columns in word row g
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) {
     const int row = tile_row(base, nj, m);
-    woff[nj] = row < N ? (uint32_t)row * rb + (PAIR ? 32u : 16u) * (uint32_t)g : kOOB;
+    woff[nj] = row >= N ? kOOB
+               : GQ     ? 4u * (uint32_t)(g * N + row)
+                        : (uint32_t)row * rb + (PAIR ? 32u : 16u) * (uint32_t)g;
   }
   // index of the scale of block nj in step kb (rows past N: past the end)
   auto sidx = [&](int kb, int nj) {
     return (uint32_t)(tile_row(base, nj, m) * ngrp) + (MODE == kScaleOne ? 0u : (uint32_t)(kb * 128 / W.group));
   };
   auto load_s = [&](int kb, Wgt& t) {
-    if constexpr (MODE == kScale128) {
+    if constexpr (GQ) {
+      const uint32_t go = kb < nsteps ? 2u * (uint32_t)(kb * 128 / W.group) * (uint32_t)N : kOOB;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) t.s[h] = bload4(sres, 2u * (uint32_t)tile_row(base, 2 * h, m) + go);
+    } else if constexpr (MODE == kScale128) {
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload4(sres, (sesz * sidx(kb < nsteps ? kb : 0, nj)) & ~3u);
     }
   };
-  auto load_w = [&](int kb, int i, Wgt& t) {  // 64 bytes of each row (bf16: K is whole steps)
-    const uint32_t ko = kb * KS + (I8 ? 64 : 32) * i < K ? (uint32_t)kb * 128u + (PAIR ? 16u : 64u) * (uint32_t)i : kOOB;
+  auto load_w = [&](int kb, int i, Wgt& t) {  // 64 bytes of each row (bf16: K is whole steps); GPTQ: sub-step i
+    if constexpr (GQ) {
+      const uint32_t ko = kb < nsteps ? (uint32_t)kb * 64u * (uint32_t)N : kOOB;
 #pragma unroll
-    for (int nj = 0; nj < 4; ++nj) t.w[nj][i] = bload16(wres, woff[nj] + ko);
+      for (int h = 0; h < 2; ++h)
+        t.w[h][i] = __builtin_amdgcn_raw_buffer_load_b64(wres, woff[2 * h] + ko, 16u * (uint32_t)N * (uint32_t)i, 0);
+    } else {
+      const uint32_t ko = kb * KS + (I8 ? 64 : 32) * i < K ? (uint32_t)kb * 128u + (PAIR ? 16u : 64u) * (uint32_t)i : kOOB;
+#pragma unroll
+      for (int nj = 0; nj < 4; ++nj) t.w[nj][i] = bload16(wres, woff[nj] + ko);
+    }
   };
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // bf16 1.0
 
-  // kScale128 holds one register set beside its partial sums: cur and nxt are
-  // the same, a piece is requested again as soon as its last MFMA has read it
+  // ONESET holds one register set beside its partial sums: cur and nxt are the
+  // same, a piece is requested again as soon as its last MFMA has read it
   auto step = [&](int kb, int slot, Wgt& cur, Wgt& nxt) {
     // the copies of stage kb have landed (younger: this step's weights, the
     // copies of stage kb + 1), then every wave's have, and every wave is done
@@ -158,12 +219,11 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
     wait_vm<NW + NA>();
     asm volatile("s_barrier" ::: "memory");
     issue_a(kb + 2, slot == 0 ? 2 : slot - 1);
-    uint32_t sw[4];
-    if constexpr (MODE == kScale128) {
+    uint32_t sw[std::extent<decltype(cur.s)>::value];
 #pragma unroll
-      for (int nj = 0; nj < 4; ++nj) sw[nj] = cur.s[nj];
-      load_s(kb + 1, nxt);
-    } else {
+    for (int j = 0; j < (int)std::extent<decltype(cur.s)>::value; ++j) sw[j] = cur.s[j];
+    load_s(kb + 1, nxt);
+    if constexpr (!ONESET) {
       load_w(kb + 1, 0, nxt);
       load_w(kb + 1, 1, nxt);
     }
@@ -188,13 +248,7 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
     auto mma = [&](int q, const u32x4(&a)[MI]) {
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) {
-        u32x4 b;
-        if constexpr (I8) {
-          const u32x4 r = cur.w[nj][q >> 1];
-          b = i8x8_to_bf16(q & 1 ? r.z : r.x, q & 1 ? r.w : r.y);
-        } else {
-          b = cur.w[nj][q];
-        }
+        const u32x4 b = tile_weights<FMT>(cur, nj, q);
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) {
           f32x4& d = MODE == kScale128 ? p[mi][nj] : acc[mi][nj];
@@ -202,9 +256,38 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
         }
       }
     };
+    f32x4 x = {0.f, 0.f, 0.f, 0.f};
     u32x4 a0[MI], a1[MI];
-    frag(0, a0);
-    if constexpr (MODE == kScale128) {
+    if constexpr (!GQ) frag(0, a0);
+    if constexpr (GQ) {
+      // a sub-step's four decoded words, requested again at once for the next
+      // step, against one row block after the other, whose operand is read two
+      // blocks ahead (the accumulators leave no room for a sub-step's operands
+      // at once); beside the products, the sums
+      // of row block `wave` over the step (the same in every column), for the
+      // zero points
+      auto row = [&](int blk, int q) {
+        return *(const u32x4*)(st + (16 * blk + m) * F::kARow + 16 * ((4 * q + g) ^ m));
+      };
+      u32x4 a[3] = {row(0, 0), row(1, 0)};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 xa = row(wave, q);
+        u32x4 b[4];
+#pragma unroll
+        for (int nj = 0; nj < 4; ++nj) b[nj] = tile_weights<FMT>(cur, nj, q);
+        load_w(kb + 1, q, nxt);
+#pragma unroll
+        for (int mi = 0; mi < MI; ++mi) {
+          const int i = MI * q + mi;
+          if (i + 2 < 4 * MI) a[(i + 2) % 3] = row((i + 2) % MI, (i + 2) / MI);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int nj = 0; nj < 4; ++nj) p[mi][nj] = mfma_bf16(a[i % 3], b[nj], p[mi][nj]);
+        }
+        x = mfma_bf16(xa, ones, x);
+      }
+    } else if constexpr (ONESET) {
       frag(1, a1);
       __builtin_amdgcn_sched_barrier(0);
       mma(0, a0);
@@ -241,12 +324,23 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
       mma(0, a0);
       mma(1, a1);
     }
-    if constexpr (MODE == kScale128) {
+    if constexpr (ONESET) {
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) {
-        const float sv = decode_scalar_word(sw[nj], sidx(kb, nj), W.s_dt);
+        float sv;
+        if constexpr (GQ) sv = half_word(sw[nj >> 1], nj & 1, W.s_dt);
+        else sv = decode_scalar_word(sw[nj], sidx(kb, nj), W.s_dt);
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) acc[mi][nj] += p[mi][nj] * sv;
+      }
+    }
+    if constexpr (GQ) {
+      // the sums exist before the branch: the compiler has sunk their MFMAs
+      // (and the operand moves, which then skip the masked lanes) into it
+      asm volatile("" : "+v"(x));
+      if (m == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Xs[(16 * wave + 4 * g + r) * (nsteps + 1) + kb] = x[r];
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -255,12 +349,12 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
   Wgt w0, w1;
   issue_a(0, 0);
   load_s(0, w0);
-  load_w(0, 0, w0);
-  load_w(0, 1, w0);
+#pragma unroll
+  for (int i = 0; i < (GQ ? 4 : 2); ++i) load_w(0, i, w0);
   issue_a(1, 1);
   int slot = 0;
   auto next = [&] { slot = slot == 2 ? 0 : slot + 1; };
-  if constexpr (MODE == kScale128) {
+  if constexpr (ONESET) {
     for (int kb = 0; kb < nsteps; ++kb) {
       step(kb, slot, w0, w0);
       next();
@@ -282,9 +376,36 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
       for (int mi = 0; mi < MI; ++mi) acc[mi][nj] *= sv;
     }
   }
-  // the copies past the last step have landed and every wave is done with the ring
+  // the copies past the last step have landed and every wave is done with the
+  // ring and (GPTQ) has written its row sums
   wait_vm<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if constexpr (GQ) {
+    // the zero points: acc -= X . (s (z + 1)), steps t + g of row m / column (nj, m)
+    const Rsrc zres = make_rsrc(W.z, (uint32_t)ngrp * (uint32_t)(N / 8) * 4u);
+    for (int t = 0; t < nsteps; t += 4) {
+      const int kb = t + g;
+      const bool in = kb < nsteps;
+      const uint32_t grp = (uint32_t)(kb * 128 / W.group);
+      float c[4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t row = (uint32_t)tile_row(base, 2 * h, m);
+        const bool ok = in && row < (uint32_t)N;
+        const uint32_t sw = bload4(sres, ok ? 2u * (grp * (uint32_t)N + row) : kOOB);
+        const uint32_t zw = bload4(zres, ok ? 4u * (grp * (uint32_t)(N / 8) + row / 8u) : kOOB) >> (4u * (row & 7u));
+        c[2 * h] = -half_word(sw, 0, W.s_dt) * (float)((zw & 15u) + 1u);
+        c[2 * h + 1] = -half_word(sw, 1, W.s_dt) * (float)(((zw >> 4) & 15u) + 1u);
+      }
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi) {
+        const float xa = in ? Xs[(16 * mi + m) * (nsteps + 1) + kb] : 0.0f;
+#pragma unroll
+        for (int nj = 0; nj < 4; ++nj)
+          acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, c[nj], acc[mi][nj], 0, 0, 0);
+      }
+    }
+  }
 }
 
 // h = act(gate) * up for one 16 x 16 block pair, with the activation fixed at
@@ -350,7 +471,7 @@ __device__ __forceinline__ void tile_store_y(const LayerArgs& a, const ProjSlot&
 
 template <int FMT, int MODE, int MI, bool STB, bool BIG>
 __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                         const int* s_pair, const float* s_w, const float* s_bias) {
+                                         const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
   using F = TileFmt<FMT>;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -374,7 +495,7 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  tile_kloop<FMT, MODE, MI, STB, BIG>(W, base, abase, abytes, src, lds, acc);
+  tile_kloop<FMT, MODE, MI, STB, BIG>(W, base, abase, abytes, src, lds, Xs, acc);
 
   const int lb[2] = {(STB ? 64 : 32) * wave, STB ? 64 * wave + 32 : kTN / 2 + 32 * wave};
   float bf[4];
@@ -396,9 +517,10 @@ __device__ __forceinline__ void tile_run(const LayerArgs& a, const ProjSlot& W, 
 // The tile on the instantiation for its number of 16-row blocks.
 template <int FMT, int MODE, bool STB, bool BIG>
 __device__ __forceinline__ void tile_rows(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                          const int* s_pair, const float* s_w, const float* s_bias) {
-  if (rows > 32) tile_run<FMT, MODE, 4, STB, BIG>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias);
-  else tile_run<FMT, MODE, 2, STB, BIG>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias);
+                                          const int* s_pair, const float* s_w, const float* s_bias,
+                                          float* Xs = nullptr) {
+  if (rows > 32) tile_run<FMT, MODE, 4, STB, BIG>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias, Xs);
+  else tile_run<FMT, MODE, 2, STB, BIG>(a, W, Iu, n0, rows, lds, s_pair, s_w, s_bias, Xs);
 }
 
 extern __shared__ __attribute__((aligned(16))) char ftm_tile_lds[];
@@ -533,21 +655,18 @@ __global__ __launch_bounds__(kBlock, 2) void k_tile(const LayerArgs a) {
     tile_missing<STB>(a, t, s_pair);
     return;
   }
-  tile_rows<FMT, MODE, STB, BIG>(a, proj_slot(PW, t.slot), I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
+  tile_rows<FMT, MODE, STB, BIG>(a, proj_slot(PW, t.slot), I, t.n0, t.rows, lds, s_pair, s_w, s_bias, s_bias + kTN);
 }
 
 // ---------------------------------------------------------------- scaled-MFMA tiles
-// The routed experts of MXFP4, FP8 (128 x 128 blocks) and GPTQ layers: the same
-// tile on v_mfma_scale_f32_16x16x128_f8f6f4 with the decode path's operand
-// layouts (ftm_moe.hip).  The weights go in as stored, straight from the
-// buffer loads (e4m3, or e2m1 with e8m0 as scale_b; GPTQ nibbles as e4m3 codes,
-// 5 VALU a word, their zero points taken out at the end: a wave sums its share
-// of the rows over each step by MFMAs against ones, the sums X[row][step] wait
-// in LDS, and acc -= X . (s (z + 1)) runs on fp32 MFMAs); the activations as their
-// two-term e4m3 split (kMxChunk bytes per row and 128 K: the input by token
-// from the router launch, h by pair from stage A's epilogue).  One K step is
-// one MFMA pair per 16 x 16 block, so FP8's block scale multiplies the pair's
-// sums and no second accumulator set is held.
+// The routed experts of MXFP4 and FP8 (128 x 128 blocks) layers: the same tile
+// on v_mfma_scale_f32_16x16x128_f8f6f4 with the decode path's operand layouts
+// (ftm_moe.hip).  The weights go in as stored, straight from the buffer loads
+// (e4m3, or e2m1 with e8m0 as scale_b); the activations as their two-term e4m3
+// split (kMxChunk bytes per row and 128 K: the input by token from the router
+// launch, h by pair from stage A's epilogue).  One K step is one MFMA pair per
+// 16 x 16 block, so FP8's block scale multiplies the pair's sums and no second
+// accumulator set is held.
 //
 // The activation rows are requested two K steps ahead, by direct buffer->LDS
 // copies into a ring of three stages (buffer copies, not the global ones:
@@ -565,12 +684,6 @@ struct MxW {
   uint32_t s[4];  // MXFP4: the lane's e8m0 byte of block nj; FP8: [0] / [2], the halves' fp32 block scales
 };
 
-template <>
-struct MxW<FTM_FMT_GPTQ_INT4> {
-  u32x2 w[2][4];  // [half][i]: columns 2m, 2m + 1; words of K 16 g, 16 g + 8, 64 + 16 g, 72 + 16 g
-  uint32_t s[2];  // [half]: both columns' 16-bit scales
-};
-
 // Copy i of a wave covers rows 16 wave + 4 i + lane / 16 (16-byte pieces,
 // swizzled), its last one the scale bytes of rows 16 wave + lane / 4.
 using MxRows = TileSrc<5>;
@@ -585,28 +698,16 @@ __device__ __forceinline__ void wait_n(int n) {
 }
 
 // One K step of a wave: 16 MI activation rows of the LDS stage st against its
-// 64 weight rows, into acc.  GPTQ: x = the sums of row block `wave` over the step.
+// 64 weight rows, into acc.
 template <int FMT, int MI>
-__device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, int s_dt, f32x4 (&acc)[MI][4], f32x4& x) {
-  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK, GQ = FMT == FTM_FMT_GPTQ_INT4;
-  constexpr bool POST = F8 || GQ;  // the step's products are scaled into acc
+__device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, f32x4 (&acc)[MI][4]) {
+  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK;  // the step's products are scaled into acc
   const int lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15;
   i32x8 bw[4];
   int sb[4];
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) {
-    if constexpr (GQ) {
-      // a nibble, zero-extended to a byte, is the e4m3 code of q 2^-9 (0..15
-      // are the subnormals and the first binade): scale_b = 2^9 makes it q
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t w = (nj & 1) ? cur.w[nj >> 1][i].y : cur.w[nj >> 1][i].x;
-        const uint32_t lo = w & 0x0f0f0f0fu, hi = (w >> 4) & 0x0f0f0f0fu;       // q0 q2 q4 q6 / q1 q3 q5 q7
-        bw[nj][2 * i] = (int)__builtin_amdgcn_perm(hi, lo, 0x05010400u);      // q0 q1 q2 q3
-        bw[nj][2 * i + 1] = (int)__builtin_amdgcn_perm(hi, lo, 0x07030602u);  // q4 q5 q6 q7
-      }
-      sb[nj] = 127 + 9;
-    } else if constexpr (F8) {
+    if constexpr (F8) {
       const u32x4 r0 = cur.w[nj][0], r1 = cur.w[nj][1];
       bw[nj] = (i32x8){(int)r0.x, (int)r0.y, (int)r0.z, (int)r0.w, (int)r1.x, (int)r1.y, (int)r1.z, (int)r1.w};
       sb[nj] = 127;
@@ -632,38 +733,21 @@ __device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, int
   auto scales = [&](int mi) { return (uint32_t)*(const uint16_t*)(st + kTM * kXRow + 16 * (16 * mi + m) + 2 * g); };
   f32x4 tq[2][4];
   auto fold = [&](int mi) {
-    if constexpr (POST) {
+    if constexpr (F8) {
 #pragma unroll
-      for (int nj = 0; nj < 4; ++nj) {
-        float s;
-        if constexpr (GQ) s = half_word(cur.s[nj >> 1], nj & 1, s_dt);
-        else s = __uint_as_float(cur.s[nj & 2]);
-        acc[mi][nj] += tq[mi & 1][nj] * s;
-      }
+      for (int nj = 0; nj < 4; ++nj) acc[mi][nj] += tq[mi & 1][nj] * __uint_as_float(cur.s[nj & 2]);
     }
   };
-  constexpr int kB = POST ? 0 : 4;  // B format: e4m3 or e2m1
+  constexpr int kB = F8 ? 0 : 4;  // B format: e4m3 or e2m1
   auto mma = [&](int mi, const Term& t, int scale, bool first) {
     const i32x8 av = {(int)t.a.x, (int)t.a.y, (int)t.a.z, (int)t.a.w, (int)t.b.x, (int)t.b.y, (int)t.b.z, (int)t.b.w};
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) {
-      f32x4& d = POST ? tq[mi & 1][nj] : acc[mi][nj];
+      f32x4& d = F8 ? tq[mi & 1][nj] : acc[mi][nj];
       const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-      d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bw[nj], POST && first ? z : d, 0, kB, 0, scale, 0, sb[nj]);
+      d = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bw[nj], F8 && first ? z : d, 0, kB, 0, scale, 0, sb[nj]);
     }
   };
-  if constexpr (GQ) {
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const Term h = term(wave, 0), l = term(wave, 1);
-    const uint32_t xs = scales(wave);
-    const int one = 0x38383838;  // e4m3 1.0
-    const i32x8 ones = {one, one, one, one, one, one, one, one};
-    const i32x8 hv = {(int)h.a.x, (int)h.a.y, (int)h.a.z, (int)h.a.w, (int)h.b.x, (int)h.b.y, (int)h.b.z, (int)h.b.w};
-    const i32x8 lv = {(int)l.a.x, (int)l.a.y, (int)l.a.z, (int)l.a.w, (int)l.b.x, (int)l.b.y, (int)l.b.z, (int)l.b.w};
-    x = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(hv, ones, (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0,
-                                                         (int)(xs & 0xffu), 0, 127);
-    x = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(lv, ones, x, 0, 0, 0, (int)(xs >> 8), 0, 127);
-  }
   Term hi = term(0, 0);
   uint32_t sc = scales(0);
 #pragma unroll
@@ -686,9 +770,9 @@ __device__ __forceinline__ void mx_step(const char* st, const MxW<FMT>& cur, int
 
 template <int FMT, int MI, bool BIG, bool SHORT>
 __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2], const char* abase, uint32_t abytes,
-                                         const MxRows& rows, char* lds, float* Xs, f32x4 (&acc)[MI][4]) {
-  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK, GQ = FMT == FTM_FMT_GPTQ_INT4;
-  constexpr int NA = 5, NW = F8 || GQ ? 10 : 8;  // copies / loads a step
+                                         const MxRows& rows, char* lds, f32x4 (&acc)[MI][4]) {
+  constexpr bool F8 = FMT == FTM_FMT_FP8_BLOCK;
+  constexpr int NA = 5, NW = F8 ? 10 : 8;  // copies / loads a step
   typedef __attribute__((address_space(1))) const void* GPtr;
   typedef __attribute__((address_space(3))) void* LPtr;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -718,67 +802,31 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
 
   const uint32_t rb = F8 ? (uint32_t)K : (uint32_t)K / 2;
   const int nkb = K / 128;
-  const int ngrp = GQ ? K / W.group : 0;
   const Rsrc wres = make_rsrc(W.w, rb * (uint32_t)N);
-  const Rsrc sres = make_rsrc(W.s, F8 ? 4u * (uint32_t)((N + 127) / 128) * (uint32_t)nkb
-                              : GQ ? 2u * (uint32_t)ngrp * (uint32_t)N
-                                   : (uint32_t)N * (uint32_t)(K / 32));
-  uint32_t woff[GQ ? 2 : 4];
-  if constexpr (GQ) {  // the halves' first columns, word row 2 g
+  const Rsrc sres = make_rsrc(W.s, F8 ? 4u * (uint32_t)((N + 127) / 128) * (uint32_t)nkb : (uint32_t)N * (uint32_t)(K / 32));
+  uint32_t woff[4];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int row = tile_row(base, 2 * h, m);
-      woff[h] = row < N ? 4u * (uint32_t)(2 * g * N + row) : kOOB;
-    }
-  } else {
-#pragma unroll
-    for (int nj = 0; nj < 4; ++nj) {
-      const int row = tile_row(base, nj, m);
-      woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
-    }
+  for (int nj = 0; nj < 4; ++nj) {
+    const int row = tile_row(base, nj, m);
+    woff[nj] = row < N ? (uint32_t)row * rb + 16u * (uint32_t)g : kOOB;
   }
   auto load_w = [&](int kb, MxW<FMT>& t) {
-    if constexpr (GQ) {
-      const uint32_t go = kb < nsteps ? 2u * (uint32_t)(kb * 128 / W.group) * (uint32_t)N : kOOB;
-      const uint32_t ko = kb < nsteps ? (uint32_t)kb * 64u * (uint32_t)N : kOOB;
+    const int k0 = F8 ? kb * 128 : kb * 128 + 32 * g;  // FP8: K is whole steps
+    const uint32_t so = k0 < K ? 4u * (uint32_t)kb : kOOB;
+    const uint32_t ko = k0 < K ? (uint32_t)kb * (F8 ? 128u : 64u) : kOOB;
+    if constexpr (F8) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) t.s[h] = bload4(sres, 2u * (uint32_t)tile_row(base, 2 * h, m) + go);
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          t.w[h][i] = __builtin_amdgcn_raw_buffer_load_b64(wres, woff[h] + ko,
-                                                           4u * (uint32_t)N * (uint32_t)((i & 1) + 8 * (i >> 1)), 0);
+      for (int h = 0; h < 4; h += 2) t.s[h] = bload4(sres, 4u * (uint32_t)(base[h >> 1] / 128 * nkb) + so);
     } else {
-      const int k0 = F8 ? kb * 128 : kb * 128 + 32 * g;  // FP8: K is whole steps
-      const uint32_t so = k0 < K ? 4u * (uint32_t)kb : kOOB;
-      const uint32_t ko = k0 < K ? (uint32_t)kb * (F8 ? 128u : 64u) : kOOB;
-      if constexpr (F8) {
+      // the e8m0 byte of a 16-byte piece sits at a sixteenth of its offset
+      // (rows past N: past the scales' end as well)
 #pragma unroll
-        for (int h = 0; h < 4; h += 2) t.s[h] = bload4(sres, 4u * (uint32_t)(base[h >> 1] / 128 * nkb) + so);
-      } else {
-        // the e8m0 byte of a 16-byte piece sits at a sixteenth of its offset
-        // (rows past N: past the scales' end as well)
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload1(sres, (woff[nj] >> 4) + so);
-      }
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj)
-#pragma unroll
-        for (int i = 0; i < (F8 ? 2 : 1); ++i) t.w[nj][i] = bload16(wres, woff[nj] + ko + 64u * (uint32_t)i);
+      for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload1(sres, (woff[nj] >> 4) + so);
     }
-  };
-  // GPTQ: the row sums of step kb (the same in every column)
-  auto put_x = [&](int kb, f32x4 x) {
-    if constexpr (GQ) {
-      // the sums exist before the branch: the compiler has sunk their MFMAs
-      // (and the operand moves, which then skip the masked lanes) into it
-      asm volatile("" : "+v"(x));
-      if (m == 0) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) Xs[(16 * wave + 4 * g + r) * (nsteps + 1) + kb] = x[r];
-      }
-    }
+    for (int nj = 0; nj < 4; ++nj)
+#pragma unroll
+      for (int i = 0; i < (F8 ? 2 : 1); ++i) t.w[nj][i] = bload16(wres, woff[nj] + ko + 64u * (uint32_t)i);
   };
 
   MxW<FMT> w0, w1;
@@ -798,8 +846,7 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
         asm volatile("s_barrier" ::: "memory");
         if (kb + 1 < kXbSteps) load_w(kb + 1, kb & 1 ? w0 : w1);
         __builtin_amdgcn_sched_barrier(0);
-        f32x4 x;
-        mx_step<FMT, MI>(lds + kb * kXStage, cur, W.s_dt, acc, x);
+        mx_step<FMT, MI>(lds + kb * kXStage, cur, acc);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -813,9 +860,7 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
       issue_a(kb + 2, slot == 0 ? 2 : slot - 1);
       load_w(kb + 1, nxt);
       __builtin_amdgcn_sched_barrier(0);
-      f32x4 x;
-      mx_step<FMT, MI>(lds + slot * kXStage, cur, W.s_dt, acc, x);
-      put_x(kb, x);
+      mx_step<FMT, MI>(lds + slot * kXStage, cur, acc);
       __builtin_amdgcn_sched_barrier(0);
     };
     issue_a(0, 0);
@@ -847,32 +892,6 @@ __device__ __forceinline__ void mx_kloop(const ProjSlot& W, const int (&base)[2]
   // the copies past the last step have landed and every wave is done with the ring
   wait_vm<0>();
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  if constexpr (GQ) {
-    // the zero points: acc -= X . (s (z + 1)), steps t + g of row m / column (nj, m)
-    const Rsrc zres = make_rsrc(W.z, (uint32_t)ngrp * (uint32_t)(N / 8) * 4u);
-    for (int t = 0; t < nsteps; t += 4) {
-      const int kb = t + g;
-      const bool in = kb < nsteps;
-      const uint32_t grp = (uint32_t)(kb * 128 / W.group);
-      float c[4];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const uint32_t row = (uint32_t)tile_row(base, 2 * h, m);
-        const bool ok = in && row < (uint32_t)N;
-        const uint32_t sw = bload4(sres, ok ? 2u * (grp * (uint32_t)N + row) : kOOB);
-        const uint32_t zw = bload4(zres, ok ? 4u * (grp * (uint32_t)(N / 8) + row / 8u) : kOOB) >> (4u * (row & 7u));
-        c[2 * h] = -half_word(sw, 0, W.s_dt) * (float)((zw & 15u) + 1u);
-        c[2 * h + 1] = -half_word(sw, 1, W.s_dt) * (float)(((zw >> 4) & 15u) + 1u);
-      }
-#pragma unroll
-      for (int mi = 0; mi < MI; ++mi) {
-        const float xa = in ? Xs[(16 * mi + m) * (nsteps + 1) + kb] : 0.0f;
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj)
-          acc[mi][nj] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa, c[nj], acc[mi][nj], 0, 0, 0);
-      }
-    }
-  }
 }
 
 template <bool STB, bool BIG>
@@ -896,7 +915,7 @@ __device__ __forceinline__ MxRows mx_rows(const LayerArgs& a, int rows, const in
 
 template <int FMT, int MI, bool STB, bool BIG, bool SHORT>
 __device__ __forceinline__ void mx_run(const LayerArgs& a, const ProjSlot& W, int Iu, int n0, int rows, char* lds,
-                                       const int* s_pair, const float* s_w, const float* s_bias, float* Xs) {
+                                       const int* s_pair, const float* s_w, const float* s_bias) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15;
@@ -911,7 +930,7 @@ __device__ __forceinline__ void mx_run(const LayerArgs& a, const ProjSlot& W, in
   for (int mi = 0; mi < MI; ++mi)
 #pragma unroll
     for (int nj = 0; nj < 4; ++nj) acc[mi][nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  mx_kloop<FMT, MI, BIG, SHORT>(W, base, abase, abytes, ar, lds, Xs, acc);
+  mx_kloop<FMT, MI, BIG, SHORT>(W, base, abase, abytes, ar, lds, acc);
 
   const int lb[2] = {(STB ? 64 : 32) * wave, STB ? 64 * wave + 32 : kTN / 2 + 32 * wave};
   float bf[4];
@@ -962,9 +981,8 @@ __device__ __forceinline__ void mx_tile(const LayerArgs& a, int ring) {
     return;
   }
   const ProjSlot W = proj_slot(PW, t.slot);
-  float* Xs = s_bias + kTN;
-  if (t.rows > 32) mx_run<FMT, 4, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias, Xs);
-  else mx_run<FMT, 2, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias, Xs);
+  if (t.rows > 32) mx_run<FMT, 4, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
+  else mx_run<FMT, 2, STB, BIG, SHORT>(a, W, I, t.n0, t.rows, lds, s_pair, s_w, s_bias);
 }
 
 template <int FMT, bool STB, bool BIG>
@@ -981,11 +999,14 @@ __global__ __launch_bounds__(kBlock, 2) void k_gemm_mxb_f8(const LayerArgs a) {
 }
 
 // ---------------------------------------------------------------- launch
-// Dynamic LDS of one projection's scaled-MFMA tiles: activation stages, the
-// tile's pairs, router weights and biases, GPTQ row sums.
-static size_t mx_lds(const ftm_moe_layer& L, bool stb) {
-  const size_t x = L.w13.fmt == FTM_FMT_GPTQ_INT4 ? (size_t)kTM * (size_t)((stb ? L.inter : L.hidden) / 128 + 1) * 4u : 0u;
-  return (size_t)kXStages * kXStage + (size_t)kTM * 8u + (size_t)kTN * 4u + x;
+// Dynamic LDS: activation stages, the tile's pairs, router weights and biases,
+// k_tile on GPTQ: its row sums.
+constexpr size_t kTileTables = (size_t)kTM * 8u + (size_t)kTN * 4u;
+constexpr size_t kMxLds = (size_t)kXStages * kXStage + kTileTables;
+template <int FMT>
+static size_t tile_lds(const ftm_moe_layer& L, bool stb) {
+  const size_t x = FMT == FTM_FMT_GPTQ_INT4 ? (size_t)kTM * (size_t)((stb ? L.inter : L.hidden) / 128 + 1) * 4u : 0u;
+  return (size_t)TileFmt<FMT>::kRing + kTileTables + x;
 }
 
 // GPTQ layers the tiles take: 128-wide groups (or multiples), 16-bit scales,
@@ -995,10 +1016,10 @@ bool tile_gptq_ok(const ftm_moe_layer& L) {
   if (L.w13.group <= 0 || L.w2.group <= 0 || L.w13.group % 128 != 0 || L.w2.group % 128 != 0) return false;
   if (L.hidden % 128 != 0 || L.inter % 128 != 0 || L.hidden % L.w13.group != 0 || L.inter % L.w2.group != 0) return false;
   if (L.w13.s_dtype == FTM_DT_F32 || L.w2.s_dtype == FTM_DT_F32) return false;
-  return mx_lds(L, false) <= 160u * 1024u && mx_lds(L, true) <= 160u * 1024u;
+  return tile_lds<FTM_FMT_GPTQ_INT4>(L, false) <= 160u * 1024u && tile_lds<FTM_FMT_GPTQ_INT4>(L, true) <= 160u * 1024u;
 }
 
-// INT8 and bf16 layers the bf16 tiles take: INT8 groups of whole K steps, or
+// The layers the bf16 tiles take: GPTQ (tile_gptq_ok); INT8 groups of whole K steps, or
 // one over K; bf16 weights where there is a stage-A tile for every CU.  Below
 // that the ring tiles' 64 x 64 channels fill twice as many CUs: 16 bf16 experts
 // of 1024 x 512, top-2, at 256 / 400 / 700 / 1100 / 1500 / 2048 tokens 53.3 /
@@ -1013,6 +1034,7 @@ bool tile_bf16_ok(const ftm_moe_layer& L, int T) {
     const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
     return (pairs / kTM + maxU) * ((L.inter + kTN / 2 - 1) / (kTN / 2)) >= kTileBf16MinItems;
   }
+  if (L.w13.fmt == FTM_FMT_GPTQ_INT4) return tile_gptq_ok(L);
   auto ok = [](const ftm_proj& P) { return P.group == P.K || (P.group % 128 == 0 && P.group > 0); };
   return L.w13.fmt == FTM_FMT_INT8_PACKED && ok(L.w13) && ok(L.w2);
 }
@@ -1051,7 +1073,7 @@ static void launch_tile_t(const LayerArgs& a, hipStream_t st) {
   tile_attr(&k_tile<FMT, MODE, STB, BIG>, attr);
   static_assert(TileFmt<FMT>::kRing >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
   hipLaunchKernelGGL((k_tile<FMT, MODE, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock),
-                     (size_t)TileFmt<FMT>::kRing + (size_t)kTM * 8u + (size_t)kTN * 4u, st, a);
+                     tile_lds<FMT>(a.L, STB), st, a);
 }
 
 template <int FMT, int MODE, bool STB>
@@ -1061,14 +1083,16 @@ static void launch_tile_s(const LayerArgs& a, hipStream_t st) {
 }
 
 void launch_tile_bf16(const LayerArgs& a, hipStream_t st, int which) {
-  const bool i8 = a.L.w13.fmt == FTM_FMT_INT8_PACKED;
+  const bool i8 = a.L.w13.fmt == FTM_FMT_INT8_PACKED, gq = a.L.w13.fmt == FTM_FMT_GPTQ_INT4;
   if (which & 1) {
-    if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, false>(a, st);
+    if (gq) launch_tile_s<FTM_FMT_GPTQ_INT4, kScale128, false>(a, st);
+    else if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, false>(a, st);
     else if (a.L.w13.group == a.L.w13.K) launch_tile_s<FTM_FMT_INT8_PACKED, kScaleOne, false>(a, st);
     else launch_tile_s<FTM_FMT_INT8_PACKED, kScale128, false>(a, st);
   }
   if (which & 2) {
-    if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, true>(a, st);
+    if (gq) launch_tile_s<FTM_FMT_GPTQ_INT4, kScale128, true>(a, st);
+    else if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, true>(a, st);
     else if (a.L.w2.group == a.L.w2.K) launch_tile_s<FTM_FMT_INT8_PACKED, kScaleOne, true>(a, st);
     else launch_tile_s<FTM_FMT_INT8_PACKED, kScale128, true>(a, st);
   }
@@ -1079,7 +1103,7 @@ static void launch_mx_t(const LayerArgs& a, hipStream_t st) {
   static bool attr = false;
   tile_attr(&k_gemm_mx<FMT, STB, BIG>, attr);
   static_assert(kXStages * kXStage >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
-  hipLaunchKernelGGL((k_gemm_mx<FMT, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock), mx_lds(a.L, STB), st, a);
+  hipLaunchKernelGGL((k_gemm_mx<FMT, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock), kMxLds, st, a);
 }
 
 template <int FMT, bool STB>
@@ -1100,20 +1124,18 @@ static void launch_mxb(const LayerArgs& a, hipStream_t st) {
   static bool attr = false;
   tile_attr(&k_gemm_mxb_f8, attr);
   hipLaunchKernelGGL(k_gemm_mxb_f8, dim3(tile_items<true>(a)), dim3(kBlock),
-                     (size_t)kXbSteps * kXStage + (size_t)kTM * 8u + (size_t)kTN * 4u, st, a);
+                     (size_t)kXbSteps * kXStage + kTileTables, st, a);
 }
 
 void launch_tile_mx(const LayerArgs& a, hipStream_t st, int which) {
   const int f = a.L.w13.fmt;
   if (which & 1) {
     if (f == FTM_FMT_FP8_BLOCK) launch_mx_s<FTM_FMT_FP8_BLOCK, false>(a, st);
-    else if (f == FTM_FMT_GPTQ_INT4) launch_mx_s<FTM_FMT_GPTQ_INT4, false>(a, st);
     else launch_mx_s<FTM_FMT_MXFP4, false>(a, st);
   }
   if (which & 2) {
     if (f == FTM_FMT_FP8_BLOCK && tile_mxb_ok(a.L, a.T)) launch_mxb(a, st);
     else if (f == FTM_FMT_FP8_BLOCK) launch_mx_s<FTM_FMT_FP8_BLOCK, true>(a, st);
-    else if (f == FTM_FMT_GPTQ_INT4) launch_mx_s<FTM_FMT_GPTQ_INT4, true>(a, st);
     else launch_mx_s<FTM_FMT_MXFP4, true>(a, st);
   }
 }
