@@ -35,15 +35,15 @@ constexpr int kGemmMinRows = 16;
 // tiles, one per CU) read the weights once at a higher rate than the GEMV
 // stages, which read them again for every few tokens.  Measured on MI355X (us
 // per layer, GEMV stages / tiles): GPTQ 128 experts of 768 at 3 / 8 tokens per
-// expert 126 / 139 against 103 / 111; 64 INT8 experts of 1024
-// at 2 / 8 132 / 172 against 112 / 123; 64 FP8 experts of 1024 at 3 / 12 162 /
-// 237 against 128 / 143; bf16 at 2 / 3 220 / 253 against 241 / 248.
+// expert 126 / 139 against 103 / 111; 64 INT8 experts of 1024 at 2 / 8 132 /
+// 172 against 113 / 123; 64 FP8 experts of 1024 at 4 / 9 / 15 160 / 205 / 284
+// against 145 / 152 / 157; bf16 at 2 / 3 220 / 253 against 241 / 248.
 constexpr int kGemmMinRowsWide = 3;
 constexpr int kGemmWideItems = 256;
-// The lean FP8 shape (256 experts of 512): 2 / 3 / 4 / 6 / 8 tokens per expert
-// 149 / 175 / 199 / 237 / 270 us on its own stages against 168 / 188 / 190 /
-// 201 / 205 on the tiles.  The tiles would win from 4 on; the line lies past 8
-// because the kernels of this shape are named up to 256 tokens
+// The lean FP8 shape (256 experts of 512): 2 / 3 / 4 / 5 / 6 / 8 tokens per
+// expert 150 / 172 / 193 / 213 / 231 / 266 us on its own stages against 180 /
+// 193 / 206 / 208 / 212 / 219 on the tiles.  The tiles would win from 5 on; the
+// line lies past 8 because the kernels of this shape are named up to 256 tokens
 // (ftm_moe_stage_kernel, pinned by the dispatch test).
 constexpr int kGemmMinRowsLean = 9;
 
@@ -805,7 +805,7 @@ bool gemm_path_ok(const ftm_moe_layer& L, int T) {
   const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
   if (f == FTM_FMT_MXFP4 && T <= kXlMaxTMx) return pairs > (long)kGemmMinRows * maxU;
   long rows = kGemmMinRows;
-  if (f != FTM_FMT_MXFP4 && (mx_gemm_ok(L) || tile_bf16_ok(L, T)) && maxU * ((L.inter + 127) / 128) >= kGemmWideItems)
+  if (f != FTM_FMT_MXFP4 && (mx_gemm_ok(L, T) || tile_bf16_ok(L, T)) && maxU * ((L.inter + 127) / 128) >= kGemmWideItems)
     rows = lean_shape(L) ? kGemmMinRowsLean : kGemmMinRowsWide;
   return pairs >= rows * maxU;
 }
@@ -829,10 +829,22 @@ static size_t ring_lds_a(const ftm_moe_layer& L) {
   const int rows = f == FTM_FMT_FP8_BLOCK ? 2 : f == FTM_FMT_INT8_PACKED ? 128 : 0;
   return (size_t)kRingA + (size_t)rows * g * 4;
 }
-bool mx_gemm_ok(const ftm_moe_layer& L) { return mx_fmt(L); }
+
+// FP8 between the wide crossover and 16 tokens per expert runs on the bf16
+// tiles, which read the activations as the GEMV stages below do; the scaled
+// tiles' two-term split keeps only what lies within 2^13 of a 32-block's
+// largest (one channel of 128 at 1e6 that no weight reads: the layer is off by
+// 0.1).  us a layer there, bf16 / scaled: 64 experts of 1024 at 4 / 15 tokens
+// per expert 145 / 157 against 131 / 146, 256 of 512 at 9 / 16 220 / 233
+// against 209 / 224.
+bool mx_gemm_ok(const ftm_moe_layer& L, int T) {
+  const long pairs = (long)T * L.topk;
+  const long maxU = L.num_experts < pairs ? L.num_experts : pairs;
+  return mx_fmt(L) && (L.w13.fmt != FTM_FMT_FP8_BLOCK || pairs >= kGemmMinRows * maxU);
+}
 
 const char* gemm_a_kernel_name(const ftm_moe_layer& L, int T) {
-  return mx_gemm_ok(L) ? "k_gemm_mx" : tile_bf16_ok(L, T) ? "k_tile" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
+  return mx_gemm_ok(L, T) ? "k_gemm_mx" : tile_bf16_ok(L, T) ? "k_tile" : ring_ok(L) ? "k_gemm_a_ring" : "k_gemm_a";
 }
 
 template <int FMT>
@@ -848,7 +860,7 @@ static void ring_lds_attr() {
 
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T) {
   if (tile_bf16_ok(L, T)) return "k_tile";
-  if (!mx_gemm_ok(L)) return "k_gemm_b";
+  if (!mx_gemm_ok(L, T)) return "k_gemm_b";
   return tile_mxb_ok(L, T) ? "k_gemm_mxb_f8" : "k_gemm_mx";
 }
 
@@ -881,7 +893,7 @@ static void launch_gemm_t(const LayerArgs& a, hipStream_t st, int which) {
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready) {
   const LayerArgs a = make_args(L, x, out, T, ws, wl);
-  if (mx_gemm_ok(L)) {
+  if (mx_gemm_ok(L, T)) {
     // stage A over the quantised input, writing h quantised the same way for stage B
     if ((which & 1) && !xq_ready) launch_quant_mx(x, T, L.hidden, a.xq, st);
     launch_tile_mx(a, st, which);

@@ -157,12 +157,12 @@ const char* gemm_a_kernel_name(const ftm_moe_layer& L, int T);  // the stage A t
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T);  // the stage B tile kernel at T tokens
 void launch_gemm_stages(const ftm_moe_layer& L, const void* x, int T, void* out, char* ws, const WsLayout& wl,
                         hipStream_t st, int which, bool xq_ready = false);
-// GPTQ, INT8 and bf16 layers the bf16 tiles take above the crossover (ftm_tile.hip).
+// FP8, GPTQ, INT8 and bf16 layers the bf16 tiles take above the crossover (ftm_tile.hip).
 bool tile_bf16_ok(const ftm_moe_layer& L, int T);
 // FP8 stage B above the crossover on k_gemm_mxb_f8 (else k_gemm_mx).
 bool tile_mxb_ok(const ftm_moe_layer& L, int T);
-// Layers on the scaled-MFMA tiles (k_gemm_mx) above the crossover.
-bool mx_gemm_ok(const ftm_moe_layer& L);
+// Layers on the scaled-MFMA tiles (k_gemm_mx) above the crossover at T tokens.
+bool mx_gemm_ok(const ftm_moe_layer& L, int T);
 // k_quant_mx: the input (T x H bf16) into the xq region's two-term e4m3 split.
 void launch_quant_mx(const void* x, int T, int H, uint8_t* xq, hipStream_t st);
 // The lean FP8 decode kernels (ftm_moe.hip) cover H = 2048 (a 512-element K

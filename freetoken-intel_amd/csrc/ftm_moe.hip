@@ -3932,7 +3932,7 @@ bool mx_stage_a(const ftm_moe_layer& L, int T) {
 }
 
 bool mx_input(const ftm_moe_layer& L, int T) {
-  return mx_stage_a(L, T) || (gemm_path_ok(L, T) && mx_gemm_ok(L));
+  return mx_stage_a(L, T) || (gemm_path_ok(L, T) && mx_gemm_ok(L, T));
 }
 
 void launch_quant_mx(const void* x, int T, int H, uint8_t* xq, hipStream_t st) {

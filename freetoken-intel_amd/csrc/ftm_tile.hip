@@ -1,7 +1,7 @@
 // ftm_tile.hip -- the MoE expert stages above the token crossover as grouped
 // MFMA tiles whose weights go straight from memory into registers: k_tile
-// (bf16 MFMAs: GPTQ, INT8 and bf16 experts) and, further down, k_gemm_mx
-// (scaled MFMAs: MXFP4 and FP8 experts).
+// (bf16 MFMAs: GPTQ, INT8 and bf16 experts, FP8 ones of fewer than 16 tokens)
+// and, further down, k_gemm_mx (scaled MFMAs: MXFP4 and FP8 experts).
 //
 // A tile is 64 pairs (rows) of one expert x 256 weight rows: four waves, each
 // 64 rows x 64 weight rows over the whole K (stage A: 32 gate + 32 up
@@ -112,6 +112,9 @@ __device__ __forceinline__ u32x4 tile_weights(const TileW<FMT>& t, int nj, int q
   } else if constexpr (FMT == FTM_FMT_INT8_PACKED) {
     const u32x4 r = t.w[nj][q >> 1];
     return i8x8_to_bf16(q & 1 ? r.z : r.x, q & 1 ? r.w : r.y);
+  } else if constexpr (FMT == FTM_FMT_FP8_BLOCK) {
+    const u32x4 r = t.w[nj][q >> 1];
+    return fp8x8_to_bf16(q & 1 ? r.z : r.x, q & 1 ? r.w : r.y);
   } else {
     return t.w[nj][q];
   }
@@ -136,11 +139,12 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
                                            const TileSrc<TileFmt<FMT>::kACopies>& src, char* lds, float* Xs,
                                            f32x4 (&acc)[MI][4]) {
   using F = TileFmt<FMT>;
-  constexpr bool I8 = FMT == FTM_FMT_INT8_PACKED, GQ = FMT == FTM_FMT_GPTQ_INT4;
+  constexpr bool I8 = FMT == FTM_FMT_INT8_PACKED, GQ = FMT == FTM_FMT_GPTQ_INT4, F8 = FMT == FTM_FMT_FP8_BLOCK;
+  constexpr bool BYTES = I8 || F8;  // a lane's 16 bytes are 16 K of its weight row
   constexpr bool ONESET = MODE == kScale128;  // one register set of weights (below)
   constexpr bool PAIR = FMT == FTM_FMT_BF16 && !STB;  // a lane's two pieces are neighbours
   constexpr int KS = F::kKS, NA = F::kACopies;
-  constexpr int NW = 8 + (GQ ? 2 : MODE == kScale128 ? 4 : 0);  // weight and scale loads a step
+  constexpr int NW = 8 + (GQ || F8 ? 2 : MODE == kScale128 ? 4 : 0);  // weight and scale loads a step
   typedef __attribute__((address_space(1))) const void* GPtr;
   typedef __attribute__((address_space(3))) void* LPtr;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -169,11 +173,12 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
   };
 
   using Wgt = TileW<FMT>;
-  const uint32_t rb = I8 ? (uint32_t)K : 2u * (uint32_t)K;
+  const uint32_t rb = BYTES ? (uint32_t)K : 2u * (uint32_t)K;
   const Rsrc wres = make_rsrc(W.w, GQ ? (uint32_t)(K / 8) * (uint32_t)N * 4u : rb * (uint32_t)N);
   const uint32_t sesz = W.s_dt == FTM_DT_F32 ? 4u : 2u;
   const int ngrp = I8 || GQ ? K / W.group : 0;
-  const Rsrc sres = make_rsrc(W.s, (uint32_t)(N * ngrp) * sesz);
+  const int nkb = K / 128;  // FP8: fp32 scales of 128 x 128 blocks
+  const Rsrc sres = make_rsrc(W.s, F8 ? 4u * (uint32_t)((N + 127) / 128 * nkb) : (uint32_t)(N * ngrp) * sesz);
   uint32_t woff[4];  // GPTQ: [0] and [2], the halves' first columns in word row g
 #pragma unroll
   for (int nj = 0; nj < 4; ++nj) {
@@ -191,6 +196,10 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
       const uint32_t go = kb < nsteps ? 2u * (uint32_t)(kb * 128 / W.group) * (uint32_t)N : kOOB;
 #pragma unroll
       for (int h = 0; h < 2; ++h) t.s[h] = bload4(sres, 2u * (uint32_t)tile_row(base, 2 * h, m) + go);
+    } else if constexpr (F8) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        t.s[2 * h] = bload4(sres, 4u * (uint32_t)(base[h] / 128 * nkb + (kb < nsteps ? kb : 0)));
     } else if constexpr (MODE == kScale128) {
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) t.s[nj] = bload4(sres, (sesz * sidx(kb < nsteps ? kb : 0, nj)) & ~3u);
@@ -203,7 +212,7 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
       for (int h = 0; h < 2; ++h)
         t.w[h][i] = __builtin_amdgcn_raw_buffer_load_b64(wres, woff[2 * h] + ko, 16u * (uint32_t)N * (uint32_t)i, 0);
     } else {
-      const uint32_t ko = kb * KS + (I8 ? 64 : 32) * i < K ? (uint32_t)kb * 128u + (PAIR ? 16u : 64u) * (uint32_t)i : kOOB;
+      const uint32_t ko = kb * KS + (BYTES ? 64 : 32) * i < K ? (uint32_t)kb * 128u + (PAIR ? 16u : 64u) * (uint32_t)i : kOOB;
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) t.w[nj][i] = bload16(wres, woff[nj] + ko);
     }
@@ -229,21 +238,22 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
     }
     __builtin_amdgcn_sched_barrier(0);
     const char* st = lds + slot * F::kStage;
-    f32x4 p[MODE == kScale128 ? MI : 1][4];
+    f32x4 p[ONESET ? MI : 1][4];
 #pragma unroll
     for (auto& r : p)
 #pragma unroll
       for (int nj = 0; nj < 4; ++nj) r[nj] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    // sub-step q's operand: activation piece 4 q + g (PAIR: 2 g + q; INT8: 8 (q
-    // / 2) + 2 g + q % 2, the 16 K of a lane's weight bytes); read during the
-    // MFMAs of the sub-step before
+    // sub-step q's operand of row block blk: activation piece 4 q + g (PAIR: 2 g
+    // + q; BYTES: 8 (q / 2) + 2 g + q % 2, the 16 K of a lane's weight bytes)
+    auto row = [&](int blk, int q) {
+      const int piece = BYTES ? 8 * (q >> 1) + 2 * g + (q & 1) : PAIR ? 2 * g + q : 4 * q + g;
+      const int r = 16 * blk + m;
+      return *(const u32x4*)(st + r * F::kARow + 16 * (piece ^ tile_fa<FMT>(r)));
+    };
+    // all row blocks of a sub-step, read during the MFMAs of the one before
     auto frag = [&](int q, u32x4(&a)[MI]) {
-      const int piece = I8 ? 8 * (q >> 1) + 2 * g + (q & 1) : PAIR ? 2 * g + q : 4 * q + g;
 #pragma unroll
-      for (int mi = 0; mi < MI; ++mi) {
-        const int r = 16 * mi + m;
-        a[mi] = *(const u32x4*)(st + r * F::kARow + 16 * (piece ^ tile_fa<FMT>(r)));
-      }
+      for (int mi = 0; mi < MI; ++mi) a[mi] = row(mi, q);
     };
     auto mma = [&](int q, const u32x4(&a)[MI]) {
 #pragma unroll
@@ -251,32 +261,30 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
         const u32x4 b = tile_weights<FMT>(cur, nj, q);
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) {
-          f32x4& d = MODE == kScale128 ? p[mi][nj] : acc[mi][nj];
-          d = mfma_bf16(a[mi], b, d);
+          acc[mi][nj] = mfma_bf16(a[mi], b, acc[mi][nj]);
         }
       }
     };
     f32x4 x = {0.f, 0.f, 0.f, 0.f};
     u32x4 a0[MI], a1[MI];
-    if constexpr (!GQ) frag(0, a0);
-    if constexpr (GQ) {
-      // a sub-step's four decoded words, requested again at once for the next
-      // step, against one row block after the other, whose operand is read two
-      // blocks ahead (the accumulators leave no room for a sub-step's operands
-      // at once); beside the products, the sums
-      // of row block `wave` over the step (the same in every column), for the
-      // zero points
-      auto row = [&](int blk, int q) {
-        return *(const u32x4*)(st + (16 * blk + m) * F::kARow + 16 * ((4 * q + g) ^ m));
-      };
+    if constexpr (!ONESET) frag(0, a0);
+    if constexpr (ONESET) {
+      // a sub-step's four operands, their registers requested again for the
+      // next step as soon as all are decoded, against one row block after the
+      // other, whose activations are read two blocks ahead (the accumulators
+      // leave no room for a sub-step's at once); GPTQ: beside the products, the
+      // sums of row block `wave` over the step (the same in every column), for
+      // the zero points
       u32x4 a[3] = {row(0, 0), row(1, 0)};
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const u32x4 xa = row(wave, q);
+        u32x4 xa;
+        if constexpr (GQ) xa = row(wave, q);
         u32x4 b[4];
 #pragma unroll
         for (int nj = 0; nj < 4; ++nj) b[nj] = tile_weights<FMT>(cur, nj, q);
-        load_w(kb + 1, q, nxt);
+        if (GQ) load_w(kb + 1, q, nxt);
+        else if (q & 1) load_w(kb + 1, q >> 1, nxt);
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) {
           const int i = MI * q + mi;
@@ -285,25 +293,8 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
 #pragma unroll
           for (int nj = 0; nj < 4; ++nj) p[mi][nj] = mfma_bf16(a[i % 3], b[nj], p[mi][nj]);
         }
-        x = mfma_bf16(xa, ones, x);
+        if constexpr (GQ) x = mfma_bf16(xa, ones, x);
       }
-    } else if constexpr (ONESET) {
-      frag(1, a1);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(0, a0);
-      frag(2, a0);
-      __builtin_amdgcn_sched_barrier(0);
-      mma(1, a1);
-      __builtin_amdgcn_sched_barrier(0);
-      load_w(kb + 1, 0, nxt);
-      if (kb * 128 + 64 < K) {
-        frag(3, a1);
-        __builtin_amdgcn_sched_barrier(0);
-        mma(2, a0);
-        mma(3, a1);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      load_w(kb + 1, 1, nxt);
     } else if constexpr (I8) {
       // INT8: K may end in a half step, whose zero bytes would decode to -128
       frag(1, a1);
@@ -329,6 +320,7 @@ __device__ __forceinline__ void tile_kloop(const ProjSlot& W, const int (&base)[
       for (int nj = 0; nj < 4; ++nj) {
         float sv;
         if constexpr (GQ) sv = half_word(sw[nj >> 1], nj & 1, W.s_dt);
+        else if constexpr (F8) sv = __uint_as_float(sw[nj & 2]);
         else sv = decode_scalar_word(sw[nj], sidx(kb, nj), W.s_dt);
 #pragma unroll
         for (int mi = 0; mi < MI; ++mi) acc[mi][nj] += p[mi][nj] * sv;
@@ -1019,7 +1011,8 @@ bool tile_gptq_ok(const ftm_moe_layer& L) {
   return tile_lds<FTM_FMT_GPTQ_INT4>(L, false) <= 160u * 1024u && tile_lds<FTM_FMT_GPTQ_INT4>(L, true) <= 160u * 1024u;
 }
 
-// The layers the bf16 tiles take: GPTQ (tile_gptq_ok); INT8 groups of whole K steps, or
+// The layers the bf16 tiles take: GPTQ (tile_gptq_ok); FP8 128 x 128 below 16
+// tokens per expert (mx_gemm_ok); INT8 groups of whole K steps, or
 // one over K; bf16 weights where there is a stage-A tile for every CU.  Below
 // that the ring tiles' 64 x 64 channels fill twice as many CUs: 16 bf16 experts
 // of 1024 x 512, top-2, at 256 / 400 / 700 / 1100 / 1500 / 2048 tokens 53.3 /
@@ -1035,6 +1028,7 @@ bool tile_bf16_ok(const ftm_moe_layer& L, int T) {
     return (pairs / kTM + maxU) * ((L.inter + kTN / 2 - 1) / (kTN / 2)) >= kTileBf16MinItems;
   }
   if (L.w13.fmt == FTM_FMT_GPTQ_INT4) return tile_gptq_ok(L);
+  if (L.w13.fmt == FTM_FMT_FP8_BLOCK) return mx_fmt(L) && !mx_gemm_ok(L, T);
   auto ok = [](const ftm_proj& P) { return P.group == P.K || (P.group % 128 == 0 && P.group > 0); };
   return L.w13.fmt == FTM_FMT_INT8_PACKED && ok(L.w13) && ok(L.w2);
 }
@@ -1083,15 +1077,18 @@ static void launch_tile_s(const LayerArgs& a, hipStream_t st) {
 }
 
 void launch_tile_bf16(const LayerArgs& a, hipStream_t st, int which) {
-  const bool i8 = a.L.w13.fmt == FTM_FMT_INT8_PACKED, gq = a.L.w13.fmt == FTM_FMT_GPTQ_INT4;
+  const int f = a.L.w13.fmt;
+  const bool i8 = f == FTM_FMT_INT8_PACKED;
   if (which & 1) {
-    if (gq) launch_tile_s<FTM_FMT_GPTQ_INT4, kScale128, false>(a, st);
+    if (f == FTM_FMT_GPTQ_INT4) launch_tile_s<FTM_FMT_GPTQ_INT4, kScale128, false>(a, st);
+    else if (f == FTM_FMT_FP8_BLOCK) launch_tile_s<FTM_FMT_FP8_BLOCK, kScale128, false>(a, st);
     else if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, false>(a, st);
     else if (a.L.w13.group == a.L.w13.K) launch_tile_s<FTM_FMT_INT8_PACKED, kScaleOne, false>(a, st);
     else launch_tile_s<FTM_FMT_INT8_PACKED, kScale128, false>(a, st);
   }
   if (which & 2) {
-    if (gq) launch_tile_s<FTM_FMT_GPTQ_INT4, kScale128, true>(a, st);
+    if (f == FTM_FMT_GPTQ_INT4) launch_tile_s<FTM_FMT_GPTQ_INT4, kScale128, true>(a, st);
+    else if (f == FTM_FMT_FP8_BLOCK) launch_tile_s<FTM_FMT_FP8_BLOCK, kScale128, true>(a, st);
     else if (!i8) launch_tile_s<FTM_FMT_BF16, kScaleNone, true>(a, st);
     else if (a.L.w2.group == a.L.w2.K) launch_tile_s<FTM_FMT_INT8_PACKED, kScaleOne, true>(a, st);
     else launch_tile_s<FTM_FMT_INT8_PACKED, kScale128, true>(a, st);

@@ -172,6 +172,9 @@ def test_stage_kernel_names_follow_the_dispatch():
         assert name(c3, T, nat.STAGE_COMBINE) == "", T
     for T in (17, 64, 256):
         assert name(c3, T, nat.STAGE_W2) == "k_stage_b_lean", T
+    for T in (288, 511):  # 9 pairs per expert on: tiles, on bf16 activations below 16 as the stages above
+        assert name(c3, T, nat.STAGE_W13) == "k_tile", T
+        assert name(c3, T, nat.STAGE_W2) == "k_tile", T
     # 512 tokens x top-8 = 16 pairs per expert on all 256 experts: GEMM
     # stages, the routed experts on the scaled-MFMA tiles (FP8 128 x 128 blocks)
     assert name(c3, 512, nat.STAGE_W13) == "k_gemm_mx"

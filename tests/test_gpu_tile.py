@@ -79,22 +79,27 @@ def test_int8_tiles_match_oracle(gpu, T, H, I, shared, groups):
     assert layer.stage_kernel(T, nat.STAGE_W2) == "k_tile"
 
 
-@pytest.mark.parametrize("name", ["c1_int8", "c2_gptq", "c3_fp8", "c4_mxfp4", "bf16", "bf16_wide"])
+@pytest.mark.parametrize("name", ["c1_int8", "c2_gptq", "c3_fp8", "c3_fp8_wide", "c4_mxfp4", "bf16", "bf16_wide"])
 def test_tiles_with_uneven_experts(gpu, name):
     """Experts of 1, 15, 16, 17, 32, 33, 64, 65 and 129 rows, some of none.
     bf16 layers with fewer stage-A tiles than CUs keep the LDS-ring tiles
-    (bf16), with more they take the register-fed ones (bf16_wide)."""
+    (bf16), with more they take the register-fed ones (bf16_wide).  FP8 with
+    fewer than 16 tokens per expert: the bf16 tiles (c3_fp8_wide)."""
     T, E, k = 144, 16, 4
-    cfg = S.SMALL["c1_int8"] if name.startswith("bf16") else S.SMALL[name]
+    cfg = S.SMALL["c1_int8"] if name.startswith("bf16") else S.SMALL[name.removesuffix("_wide")]
     if name == "bf16":
         cfg = replace(cfg, fmt="bf16")
     elif name == "bf16_wide":  # 144 x 4 / 64 + 16 row tiles x 11 of 128 channels
         cfg = replace(cfg, fmt="bf16", I=1408)
+    elif name == "c3_fp8_wide":
+        E, cfg = 64, replace(cfg, I=512)
     syn = S.generate(replace(cfg, E=E, k=k), T=T, seed=9)
     ids, w = _skewed(T, E, k, [1, 15, 16, 17, 0, 32, 33, 64, 65, 129, 0, 48], 3)
     layer = _check(syn, gpu, ids, w)
     if name.startswith("bf16"):
         assert layer.stage_kernel(T, nat.STAGE_W13) == ("k_tile" if name == "bf16_wide" else "k_gemm_a_ring")
+    if name.startswith("c3_fp8"):
+        assert layer.stage_kernel(T, nat.STAGE_W13) == ("k_tile" if name == "c3_fp8_wide" else "k_gemm_mx")
 
 
 @pytest.mark.parametrize("fmt", ["c1_int8", "c2_gptq", "c3_fp8", "bf16"])
@@ -105,8 +110,8 @@ def test_tiles_of_few_rows(gpu, fmt, T):
     below."""
     cfg = replace(S.SMALL["c1_int8"], fmt="bf16") if fmt == "bf16" else S.SMALL[fmt]
     layer = _check(S.generate(replace(cfg, E=64, k=4, H=256, I=512, shared_inter=0), T=T, seed=T), gpu)
-    tile = {"c1_int8": "k_tile", "bf16": "k_tile", "c2_gptq": "k_tile", "c3_fp8": "k_gemm_mx"}[fmt]
-    assert (layer.stage_kernel(T, nat.STAGE_W13) == tile) == (T >= 48)
+    assert (layer.stage_kernel(T, nat.STAGE_W13) == "k_tile") == (T >= 48)
+    assert (layer.stage_kernel(T, nat.STAGE_W2) == "k_tile") == (T >= 48)
 
 
 @pytest.mark.parametrize("E,shared,H,T", [
@@ -170,6 +175,21 @@ def test_gptq_tiles_take_outlier_channels(gpu):
     ids = np.stack([rng.choice(16, k, replace=False) for _ in range(T)]).astype(np.int32)
     layer = _check(syn, gpu, ids, O.round_bf16(rng.rand(T, k).astype(np.float32)))
     assert layer.stage_kernel(T, nat.STAGE_W13) == "k_tile"
+
+
+@pytest.mark.parametrize("T,H,kernel", [(100, 384, "k_tile"), (200, 2048, "k_stage_a_lean"), (300, 2048, "k_tile")])
+def test_fp8_below_16_tokens_takes_outlier_channels(gpu, T, H, kernel):
+    """Below 16 tokens per expert FP8 layers read bf16 activations, on the GEMV
+    stages and on the tiles: a channel of each 128 at 1e6 that no weight reads
+    leaves the others exact."""
+    E, k = (64, 4) if H == 384 else (256, 8)
+    syn = S.generate(replace(S.SMALL["c3_fp8"], E=E, k=k, H=H, I=512, shared_inter=0), T=T, seed=6)
+    syn.bank["weight_gate_up"].view(torch.uint8)[:, :, 5::128] = 0
+    syn.x[:, 5::128] = 1e6
+    rng = np.random.RandomState(3)
+    ids = np.stack([rng.choice(E, k, replace=False) for _ in range(T)]).astype(np.int32)
+    layer = _check(syn, gpu, ids, O.round_bf16(rng.rand(T, k).astype(np.float32)))
+    assert layer.stage_kernel(T, nat.STAGE_W13) == kernel
 
 
 @pytest.mark.parametrize("H", [256, 320])
