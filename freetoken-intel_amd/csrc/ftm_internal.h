@@ -115,9 +115,10 @@ inline WsLayout ws_layout(const ftm_moe_layer& L, int T) {
   w.hbuf = o;   o = align_up(o + act * Tt * w.KP * w.Imax, 256);
   w.ybuf = o;   o = align_up(o + 4 * Tt * w.KP * (size_t)L.hidden, 256);
   // layers the scaled-MFMA stages take: the input and h quantised (kMxChunk
-  // layout, by token and by pair); GPTQ: above the crossover only (its decode
-  // stages read the bf16 input)
-  const bool mx = mx_fmt(L) && (L.w13.fmt != FTM_FMT_GPTQ_INT4 || gemm_path_ok(L, T));
+  // layout, by token and by pair).  Nothing here may depend on which kernels T
+  // tokens take: ftm_expert_forward runs a one-expert view of the layer, which
+  // crosses over at other T, in the bytes of the layer itself.
+  const bool mx = mx_fmt(L);
   w.hq = o;     o = align_up(o + (mx ? Tt * w.KP * (size_t)mx_row_bytes(w.Imax) : 0), 256);
   w.xq = o;     o = align_up(o + (mx ? Tt * (size_t)mx_row_bytes(L.hidden) : 0), 256);
   w.total = o;

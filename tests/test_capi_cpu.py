@@ -149,6 +149,27 @@ def test_device_lru_and_copy_argument_errors():
     assert cp(mx=0) == nat.OK  # nothing to copy: no launch
 
 
+@pytest.mark.parametrize("fmt,group", [(nat.FMT_GPTQ_INT4, 128), (nat.FMT_FP8_BLOCK, 128), (nat.FMT_INT8_PACKED, 256),
+                                       (nat.FMT_MXFP4, 32), (nat.FMT_BF16, 0)])
+def test_layer_bytes_cover_an_expert_call(fmt, group):
+    """ftm_expert_forward checks the workspace for the one-expert view of the
+    layer; callers size it by the layer (the slot pool's is top-1 over its
+    slots), whichever of the two has crossed over to the tiles."""
+    lib = nat.lib()
+    for slots in (1, 8, 16, 128):
+        L = _layer(E=slots, H=2048, I=768, k=1)
+        z = 0x3000 if fmt == nat.FMT_GPTQ_INT4 else None
+        L.w13 = _proj(N=2 * 768, K=2048, num_slots=slots, fmt=fmt, group=group, z=z)
+        L.w2 = _proj(N=2048, K=768, num_slots=slots, fmt=fmt, group=group, z=z)
+        if fmt == nat.FMT_GPTQ_INT4:
+            L.w13.s_dtype = L.w2.s_dtype = nat.DT_F16
+        one = type(L).from_buffer_copy(L)
+        one.num_experts = 1
+        for rows in (1, 15, 16, 17, 40, 255, 256, 383, 384, 1000, 2048):
+            have = lib.ftm_moe_workspace_bytes(ctypes.byref(L), rows)
+            assert have >= lib.ftm_moe_workspace_bytes(ctypes.byref(one), rows), (slots, rows)
+
+
 def test_stage_kernel_names_follow_the_dispatch():
     """ftm_moe_stage_kernel names the kernel each stage launches: the lean FP8
     decode stages for the 2048x512 shape below the token crossover, the tiled

@@ -136,6 +136,30 @@ def test_accessor_get_and_expert_forward(gpu):
     assert fp8[0].shape == (2 * cfg.I, cfg.H) and fp8[4] == 128
 
 
+@pytest.mark.parametrize("rows", [16, 40])
+def test_gptq_accessor_expert_forward_on_a_fresh_workspace(gpu, rows):
+    """A slot's expert from 16 rows on (the tiles) in the workspace that the
+    pool's own top-1 layer asks for, on a stream that has none yet."""
+    cfg = S.SMALL["c2_gptq"]
+    syn = S.generate(cfg, T=rows, seed=5)
+    c = OffloadMoeCache(1, cfg.E, cfg.E, gpu, quant_format="gptq_int4")
+    c.set_bank_sources({b: [syn.bank[b]] for b in c.bank_schema})
+    c.gptq_group_size = cfg.group
+    c.materialize_layer(0)
+    c.copy_missing()
+    x, slot = syn.x.to(gpu), 3
+    e = int(c.id_of_slot[slot])
+    acc = SlotWeightAccessor(c, cfg.I, torch.bfloat16)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        got = acc.expert_forward(slot, x)
+    torch.cuda.synchronize()
+    spec13 = oracle_proj(cfg.fmt, syn.bank, "gate_up", 2 * cfg.I, cfg.H, cfg.group)
+    spec2 = oracle_proj(cfg.fmt, syn.bank, "down", cfg.H, cfg.I, cfg.group)
+    ref = O.expert_forward(spec13, spec2, e, O.bf16_bits_to_f32(np_(syn.x)))
+    assert_close(to_f32(got), ref, what=f"GPTQ expert, {rows} rows")
+
+
 def _zipf_steps(E, T, k, steps, seed):
     """C5 routing: per token k distinct experts drawn Zipf(1.1) over ranks mapped
     through a seeded permutation; weights the softmax of N(0, 1) logits, bf16."""
