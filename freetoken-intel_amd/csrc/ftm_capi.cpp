@@ -249,15 +249,7 @@ int ftm_moe_forward_noalloc(const ftm_moe_layer* layer, const void* x, int32_t n
   if (num_tokens == 0) return FTM_OK;
   if (x == nullptr || out == nullptr) return FTM_ERR_NULL;
   if (!aligned16(x)) return FTM_ERR_ALIGN;
-  size_t need = ws_layout(*layer, num_tokens).total;
-  ftm_moe_layer lean;
-  if (need > (size_t)FTM_NOALLOC_SCRATCH_BYTES) {
-    // a GPTQ layer's quantised copies are all that does not fit: its stages without them
-    lean = *layer;
-    lean.w13.flags |= kProjNoTiles;
-    layer = &lean;
-    need = ws_layout(lean, num_tokens).total;
-  }
+  const size_t need = ws_layout(*layer, num_tokens).total;
   if (need > (size_t)FTM_NOALLOC_SCRATCH_BYTES) return FTM_ERR_WORKSPACE;
   void* ws = nullptr;
   rc = scratch_of_current_device(&ws);

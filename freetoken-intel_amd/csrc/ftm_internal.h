@@ -73,9 +73,6 @@ constexpr int kMaxColTiles = FTM_WS_CTRL_BYTES / 4 - kCtrlTileCnt;
 // size are zeros).
 constexpr int kMxChunk = 272;
 __host__ __device__ inline int mx_row_bytes(int H) { return (H + 127) / 128 * kMxChunk; }
-// An internal flag of w13 (ftm_proj.flags): no tiles, so no quantised copies in
-// the workspace (ftm_moe_forward_noalloc, where they would not fit its scratch).
-constexpr int kProjNoTiles = 1 << 30;
 bool tile_gptq_ok(const ftm_moe_layer& L);  // GPTQ layers the bf16 tiles take (ftm_tile.hip)
 bool gemm_path_ok(const ftm_moe_layer& L, int T);
 // Weight formats the scaled-MFMA stages take (bf16 activations): MXFP4, and

@@ -1004,7 +1004,7 @@ static size_t tile_lds(const ftm_moe_layer& L, bool stb) {
 // GPTQ layers the tiles take: 128-wide groups (or multiples), 16-bit scales,
 // whole K steps, and row sums that fit the LDS beside the ring.
 bool tile_gptq_ok(const ftm_moe_layer& L) {
-  if (L.w13.fmt != FTM_FMT_GPTQ_INT4 || L.act_dtype != FTM_DT_BF16 || (L.w13.flags & kProjNoTiles) != 0) return false;
+  if (L.w13.fmt != FTM_FMT_GPTQ_INT4 || L.act_dtype != FTM_DT_BF16) return false;
   if (L.w13.group <= 0 || L.w2.group <= 0 || L.w13.group % 128 != 0 || L.w2.group % 128 != 0) return false;
   if (L.hidden % 128 != 0 || L.inter % 128 != 0 || L.hidden % L.w13.group != 0 || L.inter % L.w2.group != 0) return false;
   if (L.w13.s_dtype == FTM_DT_F32 || L.w2.s_dtype == FTM_DT_F32) return false;

@@ -73,3 +73,22 @@ def test_noalloc_refuses_layers_beyond_its_scratch(gpu):
     rc = nat.lib().ftm_moe_forward_noalloc(ctypes.byref(layer.c()), x.data_ptr(), 512, out.data_ptr(), None, None,
                                            None, nat.stream_of(x))
     assert rc == nat.ERR_WORKSPACE
+
+
+def test_noalloc_runs_the_same_kernels_up_to_its_scratch(gpu):
+    """128 GPTQ experts of 768 on the tiles (48 tokens on) fill the scratch at
+    about 200 tokens: the workspace call's bits up to there, FTM_ERR_WORKSPACE
+    past it, as ftm_moe_workspace_bytes tells."""
+    syn = S.generate(S.CONFIGS["c2_gptq"], T=230, seed=8, device=gpu)
+    layer = S.build_layer(syn)
+    for T in (48, 190, 205, 230):
+        x = syn.x[:T].contiguous()
+        assert layer.stage_kernel(T, nat.STAGE_W13) == "k_tile"
+        if layer.workspace_bytes(T) > nat.NOALLOC_SCRATCH_BYTES:
+            with pytest.raises(nat.FtmError, match="workspace"):
+                _noalloc(layer, x)
+            continue
+        got, ref = _noalloc(layer, x), layer.forward(x)
+        torch.cuda.synchronize()
+        assert torch.equal(got, ref), T
+    assert layer.workspace_bytes(205) <= nat.NOALLOC_SCRATCH_BYTES < layer.workspace_bytes(230)
