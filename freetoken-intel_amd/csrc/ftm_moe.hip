@@ -3606,18 +3606,15 @@ struct LinArgs {
   int bias_dt, final_dt;
 };
 
-// A workgroup takes 16 rows x 64 columns, K split over its four waves: every
-// wave has all 64 columns, so an activation fragment is loaded once per
+// A workgroup takes 16 rows x 64 columns.  KS: K split over its four waves,
+// every wave has all 64 columns, so an activation fragment is loaded once per
 // workgroup and feeds four MFMAs, and a wave's chain of dependent loads is a
-// quarter of K.  Bound by the loads through L1 (activations and packed weights)
-// at many rows, by latency at few.  The K-major formats took 16 columns a wave
-// over the whole K before, the four waves reading the same activations.
-// us a call (host part about 14.5), before -> after: 1024 rows of 2048 x 1536
-// FP8 bf16 76.6 -> 42.1, fp32 127 -> 51; INT8 67.9 -> 43.6, 112 -> 53; MXFP4
-// 57.0 -> 26.6, 101 -> 42; 32 rows FP8 fp32 22.5 -> 14.6.
-// K = 512 leaves a wave half a chunk of loads: FP8 26.5 -> 24.3, MXFP4 21.5 ->
-// 19.9, INT8 25.2 -> 25.8 (1024 rows, N 2048).
-template <int FMT, int AT>
+// quarter of K.  Else (K-major formats) a wave has 16 columns over the whole K
+// and no sums to exchange; linear_ksplit says which.  Bound by the loads through
+// L1 (activations and packed weights) at many rows, by latency at few.
+// us a call without its host part, columns / KS, 1024 rows of 2048 x 1536: FP8
+// bf16 77 / 42, fp32 127 / 50; INT8 67 / 44, 112 / 52; MXFP4 57 / 27, 101 / 41.
+template <int FMT, int AT, bool KS>
 __global__ __launch_bounds__(kBlock) void k_linear(const LinArgs a) {
   constexpr bool kG = FMT == FTM_FMT_GPTQ_INT4;
   constexpr int XB = AType<AT>::kBytes;
@@ -3626,11 +3623,27 @@ __global__ __launch_bounds__(kBlock) void k_linear(const LinArgs a) {
   const int N = W.N, K = W.K;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nt = blockIdx.x, mt = blockIdx.y;
-  int lo, hi;
-  wave_k_range<FMT>(W, wave, 4, lo, hi);
   const Rsrc xres = make_rsrc(a.x, (uint32_t)a.M * (uint32_t)K * XB);
   const int m = mt * 16 + (lane & 15);
   const uint32_t arow = (m < a.M) ? (uint32_t)m * (uint32_t)K * XB : kOOB;
+  auto emit = [&](int m2, int n, float y) {
+    if (m2 < a.M && n < N) {
+      float v = round_to(y, a.out_dt);
+      if (a.bias != nullptr) v = round_to(v + load_scalar(a.bias, n, a.bias_dt), a.final_dt);
+      store_scalar(a.out, (size_t)m2 * N + n, a.final_dt, v);
+    }
+  };
+  int lo, hi;
+  wave_k_range<FMT>(W, KS ? wave : 0, KS ? 4 : 1, lo, hi);
+  if constexpr (!KS) {
+    static_assert(!kG, "GPTQ splits K");
+    const int col0[1] = {nt * 64 + 16 * wave};
+    f32x4 acc[1] = {(f32x4){0.f, 0.f, 0.f, 0.f}};
+    wave_gemm_kmajor<FMT, 1, AT>(W, col0, lo, hi, xres, arow, acc);
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) emit(mt * 16 + 4 * (lane >> 4) + rr, col0[0] + (lane & 15), acc[0][rr]);
+    return;
+  }
   // column block c, MFMA column j <-> output column nt * 64 + (GPTQ: 4 j + c, else 16 c + j)
   if constexpr (kG) {
     const int col0[1] = {nt * 64};
@@ -3650,13 +3663,6 @@ __global__ __launch_bounds__(kBlock) void k_linear(const LinArgs a) {
     for (int c = 0; c < 4; ++c) red[(wave * 4 + c) * 64 + lane] = acc[c];
   }
   __syncthreads();
-  auto emit = [&](int m2, int n, float y) {
-    if (m2 < a.M && n < N) {
-      float v = round_to(y, a.out_dt);
-      if (a.bias != nullptr) v = round_to(v + load_scalar(a.bias, n, a.bias_dt), a.final_dt);
-      store_scalar(a.out, (size_t)m2 * N + n, a.final_dt, v);
-    }
-  };
   if constexpr (kG) {
     for (int idx = threadIdx.x; idx < 16 * 64; idx += kBlock) {
       const int i = idx / 64, j = idx % 64;
@@ -4335,14 +4341,47 @@ const char* stage_kernel_name(const ftm_moe_layer& L, int T, int stage) {
   }
 }
 
+// Whether k_linear splits K over a workgroup's waves.  The split shortens a
+// wave's chain of load groups (512 K; fp32 activations and FP8 or INT8, and
+// bf16 weights: 256) and costs an exchange of about 1.3 us, so it loses where K
+// is one group, at few rows also a little above; at many rows it saves the
+// other waves' copies of the activations as well.  Columns / split, us: FP8
+// bf16, 16 rows of N 2048, K 256 / 512 / 768 / 2048 4.5 / 5.4 / 7.4 / 13.8
+// against 5.6 / 5.9 / 6.3 / 10.5; 1 row 3.4 / 3.7 / 5.0 / 8.6 against 5.0 / 5.2 /
+// 5.5 / 9.2; INT8 bf16 1 row of 2048 x 1536 8.1 against 10.1, 1024 rows of K 256
+// 18.1 against 22.5; FP8 fp32 16 rows K 256 / 512 4.9 / 7.3 against 5.9 / 6.4;
+// MXFP4 fp32 16 / 1024 rows of K 256 4.9 / 24.1 against 5.7 / 18.7.
+static bool linear_ksplit(const ftm_proj& P, int x_dt, int M) {
+  const int K = P.K;
+  const long wgs = (long)((P.N + 63) / 64) * ((M + 15) / 16);
+  const bool f32 = x_dt == FTM_DT_F32, bf = x_dt == FTM_DT_BF16;
+  switch (P.fmt) {
+    case FTM_FMT_BF16: return (K > 256 && M >= (bf ? 4 : f32 && K <= 768 ? 4 : 1)) || (K >= 256 && wgs >= 512);
+    case FTM_FMT_FP8_BLOCK:
+      return (K > 512 && M >= (bf ? 8 : f32 && K <= 768 ? 4 : 1)) || (f32 && K > 256 && M >= 16) || (K >= 384 && wgs >= 1536);
+    case FTM_FMT_INT8_PACKED:
+      return (K > 512 && M >= (f32 ? 1 : 16)) || (f32 && K > 256 && M >= 16) || (!bf && K > 768);
+    default:  // MXFP4
+      return (K > 512 && M >= 8) || (K > 1024 && M >= (bf ? 2 : 1)) || (wgs >= 512 && (K <= 256 || bf || f32));
+  }
+}
+
+template <int FMT, bool KS>
+static void launch_linear_k(const LinArgs& a, dim3 grid, int x_dt, hipStream_t st) {
+  if (x_dt == FTM_DT_F32)
+    hipLaunchKernelGGL((k_linear<FMT, FTM_DT_F32, KS>), grid, dim3(kBlock), 0, st, a);
+  else if (x_dt == FTM_DT_F16)
+    hipLaunchKernelGGL((k_linear<FMT, FTM_DT_F16, KS>), grid, dim3(kBlock), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_linear<FMT, FTM_DT_BF16, KS>), grid, dim3(kBlock), 0, st, a);
+}
+
 template <int FMT>
 static void launch_linear_t(const LinArgs& a, dim3 grid, int x_dt, hipStream_t st) {
-  if (x_dt == FTM_DT_F32)
-    hipLaunchKernelGGL((k_linear<FMT, FTM_DT_F32>), grid, dim3(kBlock), 0, st, a);
-  else if (x_dt == FTM_DT_F16)
-    hipLaunchKernelGGL((k_linear<FMT, FTM_DT_F16>), grid, dim3(kBlock), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_linear<FMT, FTM_DT_BF16>), grid, dim3(kBlock), 0, st, a);
+  if constexpr (FMT != FTM_FMT_GPTQ_INT4) {
+    if (!linear_ksplit(a.P, x_dt, a.M)) return launch_linear_k<FMT, false>(a, grid, x_dt, st);
+  }
+  launch_linear_k<FMT, true>(a, grid, x_dt, st);
 }
 
 hipError_t launch_linear(const ftm_proj& P, int slot, const void* x, int x_dt, int M, void* out, int out_dt,

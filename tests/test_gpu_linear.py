@@ -277,3 +277,44 @@ def test_linear_k_split(gpu, fmt, k, n, m):
     xd, wd = x.double().numpy(), wd.astype(np.float64)
     bound = (2.0 ** -17 + (k + 8) * 2.0 ** -24) * (np.abs(xd) @ np.abs(wd).T)
     assert (np.abs(got.double().cpu().numpy() - xd @ wd.T) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("fmt,m,k,n", [
+    # one row, and the rows from which a format's longer K is split
+    ("fp8", 1, 512, 72), ("fp8", 7, 640, 72), ("fp8", 8, 640, 72), ("fp8", 16, 384, 200), ("fp8", 400, 384, 4040),
+    ("int8", 1, 1024, 72), ("int8", 15, 576, 72), ("int8", 16, 576, 40), ("int8", 33, 512, 136),
+    ("mxfp4", 1, 1056, 40), ("mxfp4", 7, 544, 72), ("mxfp4", 8, 544, 72),
+    # a chip full of workgroups, waves without a range
+    ("mxfp4", 500, 32, 1048), ("mxfp4", 500, 288, 1048),
+    ("bf16", 3, 264, 72), ("bf16", 4, 264, 72), ("bf16", 33, 256, 40), ("bf16", 500, 256, 1048)])
+def test_linear_on_both_sides_of_the_k_split(gpu, fmt, m, k, n, dtype):
+    """The sizes at which a projection goes from columns over the whole K to K
+    split over the waves.  Errors: activations beyond bf16 as two terms (2^-17
+    of each product, fp16 exact), fp32 sums 2^-24 a step."""
+    from ftmoe.banks import Proj
+    from ftmoe.kernel._common import run_linear
+
+    g = torch.Generator().manual_seed(k + n + m)
+    w, x = torch.randn(n, k, generator=g) * 0.1, torch.randn(m, k, generator=g).to(dtype)
+    f32 = torch.float32
+    if fmt == "fp8":
+        wq, s = quant.quantize_block_fp8(w, block=128)
+        got = fused_fp8_linear(x.to(gpu), wq.to(gpu), s.to(gpu), block=128, out_dtype=f32)
+        wd = O.dequantize_block_fp8(np_(wq), s.numpy(), 128)
+    elif fmt == "int8":
+        s = (w.abs().amax(dim=1, keepdim=True) / 127.0).clamp_min(1e-12)
+        q = (w / s).round().clamp(-127, 127)
+        wq = (q + 128).to(torch.uint8).contiguous().view(torch.int32)
+        got = fused_int8_linear(x.to(gpu), wq.to(gpu), s.to(gpu), k=k, out_dtype=f32)
+        wd = q.double().numpy() * s.double().numpy()
+    elif fmt == "mxfp4":
+        b, s = quant.quantize_mxfp4_blocks(w)
+        got = fused_mxfp4_linear(x.to(gpu), b.to(gpu), s.to(gpu), out_dtype=f32)
+        wd = O.dequantize_mxfp4_blocks(b.numpy(), s.numpy())
+    else:
+        wd = w.bfloat16().double().numpy()
+        got = run_linear(Proj("bf16", w.bfloat16()[None].contiguous().to(gpu), n, k), x.to(gpu), out_dtype=f32, bias=None)
+    xd, wd = x.double().numpy(), wd.astype(np.float64)
+    bound = (2.0 ** -17 + (k + 8) * 2.0 ** -24) * (np.abs(xd) @ np.abs(wd).T)
+    assert (np.abs(got.double().cpu().numpy() - xd @ wd.T) <= bound).all()
