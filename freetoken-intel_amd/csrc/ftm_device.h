@@ -247,6 +247,20 @@ __device__ __forceinline__ u32x4 i8x8_to_bf16(uint32_t w0, uint32_t w1) {
   return (u32x4){a.x, a.y, b.x, b.y};
 }
 
+// The same values by unsigned converts and a subtraction: 20 VALU a word pair
+// where i8x8_to_bf16 has 14, but none of them SDWA.  k_linear on bf16 and fp16
+// activations is faster with it (us, SDWA / this: 8 rows of 4096 x 2048 20.3 /
+// 19.0, 1024 rows of 3072 x 2048 87.8 / 78.1), the layers' stages and tiles and
+// fp32 activations are slower (16 tokens of 64 experts of 1024 97.0 / 98.9, 777
+// tokens of 16 experts of 512 49.2 / 50.2, 1024 fp32 rows of 1536 x 2048 61 / 68).
+__device__ __forceinline__ uint32_t u8pair_to_bf16(uint32_t w, int hi) {
+  const uint32_t b0 = (w >> (16 * hi)) & 0xffu, b1 = (w >> (16 * hi + 8)) & 0xffu;
+  return pack_bf16x2((float)b0 - 128.0f, (float)b1 - 128.0f);
+}
+__device__ __forceinline__ u32x4 u8x8_to_bf16(uint32_t w0, uint32_t w1) {
+  return (u32x4){u8pair_to_bf16(w0, 0), u8pair_to_bf16(w0, 1), u8pair_to_bf16(w1, 0), u8pair_to_bf16(w1, 1)};
+}
+
 // 8 e2m1 nibbles (one dword, low nibble = even element) scaled by the block's
 // e8m0 factor -> 8 bf16.  LUT * 2^e is exact in bf16 for every e8m0 byte >= 2.
 __device__ __forceinline__ u32x4 fp4x8_to_bf16(uint32_t w, float scale) {
@@ -571,7 +585,8 @@ struct Chunk {
 // Rows >= N and k >= K read as zero.  For post-scaled formats the partial sum of
 // each quantisation group is multiplied by the group's fp32 scale before it
 // joins acc (FP8: one scale per 128x128 block; INT8: one per (row, group)).
-template <int FMT, int NR, int AT>
+// U8: INT8 bytes through u8x8_to_bf16.
+template <int FMT, int NR, int AT, bool U8 = false>
 __device__ __forceinline__ void wave_gemm_kmajor(const ProjSlot& W, const int (&col0)[NR], int L_lo, int L_hi,
                                                  Rsrc ares, uint32_t arow, f32x4 (&acc)[NR]) {
   using F = KMajor<FMT>;
@@ -693,7 +708,8 @@ __device__ __forceinline__ void wave_gemm_kmajor(const ProjSlot& W, const int (&
           if constexpr (FMT == FTM_FMT_FP8_BLOCK) {
             bq = q == 0 ? fp8x8_to_bf16(raw[r][b].x, raw[r][b].y) : fp8x8_to_bf16(raw[r][b].z, raw[r][b].w);
           } else if constexpr (FMT == FTM_FMT_INT8_PACKED) {
-            bq = q == 0 ? i8x8_to_bf16(raw[r][b].x, raw[r][b].y) : i8x8_to_bf16(raw[r][b].z, raw[r][b].w);
+            const uint32_t w0 = q == 0 ? raw[r][b].x : raw[r][b].z, w1 = q == 0 ? raw[r][b].y : raw[r][b].w;
+            bq = U8 ? u8x8_to_bf16(w0, w1) : i8x8_to_bf16(w0, w1);
           } else if constexpr (FMT == FTM_FMT_MXFP4) {
             const uint32_t wq = q == 0 ? raw[r][b].x : q == 1 ? raw[r][b].y : q == 2 ? raw[r][b].z : raw[r][b].w;
             bq = fp4x8_to_bf16(wq, sc[r][b]);

@@ -3639,7 +3639,7 @@ __global__ __launch_bounds__(kBlock) void k_linear(const LinArgs a) {
     static_assert(!kG, "GPTQ splits K");
     const int col0[1] = {nt * 64 + 16 * wave};
     f32x4 acc[1] = {(f32x4){0.f, 0.f, 0.f, 0.f}};
-    wave_gemm_kmajor<FMT, 1, AT>(W, col0, lo, hi, xres, arow, acc);
+    wave_gemm_kmajor<FMT, 1, AT, AT != FTM_DT_F32>(W, col0, lo, hi, xres, arow, acc);
 #pragma unroll
     for (int rr = 0; rr < 4; ++rr) emit(mt * 16 + 4 * (lane >> 4) + rr, col0[0] + (lane & 15), acc[0][rr]);
     return;
@@ -3658,7 +3658,7 @@ __global__ __launch_bounds__(kBlock) void k_linear(const LinArgs a) {
     f32x4 acc[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    wave_gemm_kmajor<FMT, 4, AT>(W, col0, lo, hi, xres, arow, acc);
+    wave_gemm_kmajor<FMT, 4, AT, AT != FTM_DT_F32>(W, col0, lo, hi, xres, arow, acc);
 #pragma unroll
     for (int c = 0; c < 4; ++c) red[(wave * 4 + c) * 64 + lane] = acc[c];
   }
