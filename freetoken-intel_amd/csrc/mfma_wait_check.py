@@ -10,18 +10,26 @@ K slice).  The kernels are written to keep such reads in the MFMA's own block;
 this script makes the build fail if any kernel breaks that rule.
 
 For every MFMA it walks all control-flow paths forward and reports a non-MFMA
-instruction that reads the MFMA's destination registers fewer than ``--need``
-wait states later, counting one state per instruction and N+1 per
-``s_nop N``.  The default of 8 is what the compiler itself places in-block for
-the 16x16x32 bf16 MFMA used here.  It also reports a VALU write that an MFMA
-reads across a block boundary within 3 states.
+instruction that reads the MFMA's destination registers fewer than its opcode's
+wait states (``NEED``) later, counting one state per instruction and N+1 per
+``s_nop N``.  It also reports an MFMA opcode that ``NEED`` does not name, and a
+VALU write that an MFMA reads across a block boundary within 3 states.
 
-Usage: mfma_wait_check.py [--need N] file.s [file.s ...]   (exit 1 on findings)
+Usage: mfma_wait_check.py file.s [file.s ...]   (exit 1 on findings)
 """
 from __future__ import annotations
 
 import re
 import sys
+
+# Wait states between an MFMA and a reader of its result, as the compiler places
+# them where both sit in one basic block.
+NEED = {
+    "v_mfma_f32_16x16x32_bf16": 8,
+    "v_mfma_f32_16x16x4_f32": 10,
+    "v_mfma_scale_f32_16x16x128_f8f6f4": 12,  # with an e4m3 operand (fp4 x fp4 would need fewer)
+    "v_mfma_f32_32x32x1_2b_f32": 18,
+}
 
 _FUNC = re.compile(r"\n(_Z\w+):[^\n]*\n(.*?)\.Lfunc_end", re.S)
 _RANGE = re.compile(r"([av])\[(\d+):(\d+)\]")
@@ -130,7 +138,7 @@ def _early_mfma_reads(insts, labels, i, dst):
     return hits
 
 
-def check(path: str, need: int) -> list:
+def check(path: str) -> list:
     findings = []
     src = open(path).read()
     for name, body in _FUNC.findall(src):
@@ -139,6 +147,10 @@ def check(path: str, need: int) -> list:
             if not args:
                 continue
             if op.startswith("v_mfma"):
+                need = NEED.get(op)
+                if need is None:
+                    findings.append(f"{path}: {name}: '{txt}': no wait states known for {op}")
+                    continue
                 for p, reader, left in _late_reads(insts, labels, i + 1, _regs(args[0]), need, set(), []):
                     findings.append(f"{path}: {name}: '{txt}' read {need - left} states later "
                                     f"via {p or 'fallthrough'} by '{reader}'")
@@ -151,22 +163,14 @@ def check(path: str, need: int) -> list:
 
 
 def main(argv) -> int:
-    need = 8
-    files = []
-    it = iter(argv)
-    for a in it:
-        if a == "--need":
-            need = int(next(it))
-        else:
-            files.append(a)
-    findings = [f for p in files for f in check(p, need)]
+    findings = [f for p in argv for f in check(p)]
     for f in findings:
         print(f)
     if findings:
-        print(f"mfma_wait_check: {len(findings)} MFMA result(s) read too early; "
-              "keep MFMA consumers in the MFMA's basic block", file=sys.stderr)
+        print(f"mfma_wait_check: {len(findings)} finding(s); keep MFMA consumers in the MFMA's basic block",
+              file=sys.stderr)
         return 1
-    print(f"mfma_wait_check: {len(files)} file(s) clean")
+    print(f"mfma_wait_check: {len(argv)} file(s) clean")
     return 0
 
 
