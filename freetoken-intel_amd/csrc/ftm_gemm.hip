@@ -849,13 +849,8 @@ const char* gemm_a_kernel_name(const ftm_moe_layer& L, int T) {
 
 template <int FMT>
 static void ring_lds_attr() {
-  static bool done = false;  // once per instantiation (setting it twice is harmless)
-  if (!done) {
-    // a failure here surfaces as the launch error that follows
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_gemm_a_ring<FMT>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, kRingA + kRingScaleBytes);
-    done = true;
-  }
+  static DeviceBits done;
+  (void)allow_lds(done, reinterpret_cast<const void*>(&k_gemm_a_ring<FMT>), kRingA + kRingScaleBytes);
 }
 
 const char* gemm_b_kernel_name(const ftm_moe_layer& L, int T) {

@@ -7,6 +7,7 @@
 
 #include "ftm_device.h"
 #include "ftm_internal.h"
+#include "ftm_once.h"
 
 namespace ftm {
 
@@ -61,6 +62,17 @@ inline LayerArgs make_args(const ftm_moe_layer& L, const void* x, void* out, int
   a.hq = (uint8_t*)(ws + wl.hq);
   a.xq = (uint8_t*)(ws + wl.xq);
   return a;
+}
+
+// Allows `kernel` dynamic LDS of `bytes` on the current device (`done`: one a
+// kernel).  A failure also surfaces as the error of the launch that follows.
+inline hipError_t allow_lds(DeviceBits& done, const void* kernel, int bytes) {
+  int dev = -1;
+  const hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  return (hipError_t)once_per_device(done, dev, [&] {
+    return (int)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  });
 }
 
 // The expert stages above the crossover on the register-fed tiles

@@ -3712,9 +3712,9 @@ hipError_t launch_router(const ftm_moe_layer& L, const void* x, int T, int row_b
   const int nq = quant && T < kTopkBlkMinT && mx_input(L, T) ? (quant_mx_threads(T, L.hidden) + kBlock - 1) / kBlock : 0;
   const int qx = (nq + ty - 1) / ty;
   if (router_by_mm(row_end - row_begin, T, L.hidden)) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_router_mm),
-                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kRmLds);
-    if (attr != hipSuccess) return attr;
+    static DeviceBits done;
+    const hipError_t e = allow_lds(done, reinterpret_cast<const void*>(&k_router_mm), kRmLds);
+    if (e != hipSuccess) return e;
     const int rows = row_end - row_begin;
     hipLaunchKernelGGL(k_router_mm, dim3((rows - router_mm_rest(rows) + kRmT - 1) / kRmT * ((T + kRmT - 1) / kRmT)),
                        dim3(64 * kRmWaves), kRmLds, st, a, row_begin, row_end);
@@ -3913,13 +3913,9 @@ static void launch_tok(const LayerArgs& a, int maxU, hipStream_t st) {
   constexpr int kload = FMT == FTM_FMT_MXFP4 ? 128 : FMT == FTM_FMT_BF16 ? 32 : 64;
   const int K = STB ? a.L.inter : a.L.hidden;
   const size_t lds = (size_t)tok_rows(K, kload) * 2u * (size_t)tok_pitch(K, kload);
-  static bool attr = false;
-  if (!attr) {
-    const void* fn = STB ? reinterpret_cast<const void*>(&k_stage_tok_b<FMT>)
-                         : reinterpret_cast<const void*>(&k_stage_tok_a<FMT>);
-    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kTokLdsMax);
-    attr = true;
-  }
+  static DeviceBits done;
+  (void)allow_lds(done, STB ? reinterpret_cast<const void*>(&k_stage_tok_b<FMT>)
+                            : reinterpret_cast<const void*>(&k_stage_tok_a<FMT>), kTokLdsMax);
   const int cols = STB ? 16 * kTokWaves : 8 * kTokWaves;
   const int nct = ((STB ? a.L.hidden : a.L.inter) + cols - 1) / cols;
   // column tiles per workgroup: about one workgroup per CU (one fits a CU's LDS)
@@ -4033,12 +4029,8 @@ static bool bcks_fused(const ftm_moe_layer& L, int T) {
 }
 template <int FMT, int LPG, int NLW>
 static void launch_bcks(const LayerArgs& a, hipStream_t st) {
-  static bool attr = false;
-  if (!attr) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_stage_bc_ks<FMT, LPG, NLW>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBcKsLdsMax);
-    attr = true;
-  }
+  static DeviceBits done;
+  (void)allow_lds(done, reinterpret_cast<const void*>(&k_stage_bc_ks<FMT, LPG, NLW>), (int)kBcKsLdsMax);
   hipLaunchKernelGGL((k_stage_bc_ks<FMT, LPG, NLW>), dim3(a.L.hidden / 16), dim3(64 * kBcKsWaves), bcks_lds<FMT>(a.L),
                      st, a);
 }

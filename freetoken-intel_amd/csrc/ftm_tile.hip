@@ -1047,13 +1047,8 @@ static unsigned tile_items(const LayerArgs& a) {
 }
 
 template <class K>
-static void tile_attr(K* kernel, bool& done) {
-  if (!done) {
-    // a failure here surfaces as the launch error that follows
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    done = true;
-  }
+static void tile_attr(K* kernel, DeviceBits& done) {
+  (void)allow_lds(done, reinterpret_cast<const void*>(kernel), 160 * 1024);
 }
 
 // BIG: activation rows past what one buffer descriptor's 32-bit offsets span.
@@ -1063,7 +1058,7 @@ static bool tile_big(const LayerArgs& a, bool stb, size_t row_bytes) {
 
 template <int FMT, int MODE, bool STB, bool BIG>
 static void launch_tile_t(const LayerArgs& a, hipStream_t st) {
-  static bool attr = false;
+  static DeviceBits attr;
   tile_attr(&k_tile<FMT, MODE, STB, BIG>, attr);
   static_assert(TileFmt<FMT>::kRing >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
   hipLaunchKernelGGL((k_tile<FMT, MODE, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock),
@@ -1097,7 +1092,7 @@ void launch_tile_bf16(const LayerArgs& a, hipStream_t st, int which) {
 
 template <int FMT, bool STB, bool BIG>
 static void launch_mx_t(const LayerArgs& a, hipStream_t st) {
-  static bool attr = false;
+  static DeviceBits attr;
   tile_attr(&k_gemm_mx<FMT, STB, BIG>, attr);
   static_assert(kXStages * kXStage >= TileFmt<FTM_FMT_BF16>::kRing, "the shared expert's stages fit");
   hipLaunchKernelGGL((k_gemm_mx<FMT, STB, BIG>), dim3(tile_items<STB>(a)), dim3(kBlock), kMxLds, st, a);
@@ -1118,7 +1113,7 @@ bool tile_mxb_ok(const ftm_moe_layer& L, int T) {
 }
 
 static void launch_mxb(const LayerArgs& a, hipStream_t st) {
-  static bool attr = false;
+  static DeviceBits attr;
   tile_attr(&k_gemm_mxb_f8, attr);
   hipLaunchKernelGGL(k_gemm_mxb_f8, dim3(tile_items<true>(a)), dim3(kBlock),
                      (size_t)kXbSteps * kXStage + kTileTables, st, a);
