@@ -24,11 +24,11 @@ pytestmark = pytest.mark.gpu
 REL_RMS = 4e-3
 
 
-def _check(syn, gpu, ids=None, w=None):
+def _check(syn, gpu, ids=None, w=None, cast=lambda n, t: t):
     T = syn.x.shape[0]
     ref = O.layer_reference(oracle_spec(syn), np_(syn.x), ids=ids, w=w)
     dsyn = syn.to(gpu)
-    layer = S.build_layer(dsyn)
+    layer = S.build_layer(dsyn, bank={n: cast(n, t) for n, t in dsyn.bank.items()})
     if ids is None:
         run = lambda: layer.forward(dsyn.x)  # noqa: E731
     else:
@@ -228,3 +228,60 @@ def test_shared_expert_bits_beside_any_experts(gpu, fmt, kernel):
     torch.cuda.synchronize()
     assert torch.count_nonzero(outs[0]) > 0
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("name,T,H,I,shared,group,kernel", [
+    ("int8", 64, 256, 256, 0, 64, "k_gemm_a_ring"),     # four groups of 64
+    ("int8", 130, 384, 384, 192, 192, "k_gemm_a_ring"),  # two of 192: one and a half K steps of the bf16 tiles
+    ("int8", 70, 2112, 128, 0, 64, "k_gemm_a"),          # 33 groups: their scales do not fit beside the ring
+    ("fp8", 64, 320, 384, 0, 128, "k_gemm_a_ring"),      # H and its scale blocks end in a half block
+    ("fp8", 130, 256, 192, 192, 64, "k_gemm_a_ring"),    # 64 x 64 blocks
+    ("fp8_bf16_scales", 90, 256, 256, 128, 128, "k_gemm_a_ring"),
+])
+def test_lds_tiles_match_oracle(gpu, name, T, H, I, shared, group, kernel):
+    """Quantised layers above the crossover that the register-fed tiles do not
+    take stay on the LDS tiles."""
+    cast = lambda n, t: t  # noqa: E731
+    if name == "int8":
+        cfg = replace(S.SMALL["c1_int8"], H=H, I=I, shared_inter=shared, int8_num_groups=H // group)
+        if I % (64 * (H // group)) and I != H:  # w2 per channel
+            syn = S.generate(replace(cfg, int8_num_groups=1), T=T, seed=T)
+            w = torch.randn(cfg.E, 2 * I, H, generator=torch.Generator().manual_seed(T)) * 0.02
+            syn.bank.update(S.quantize_bank(cfg.fmt, w, "gate_up", int8_num_groups=H // group))
+        else:
+            syn = S.generate(cfg, T=T, seed=T)
+    else:
+        syn = S.generate(replace(S.SMALL["c3_fp8"], E=8, k=2, H=H, I=I, shared_inter=shared, group=group), T=T, seed=T)
+    if name == "fp8_bf16_scales":
+        for n in ("scale_gate_up", "scale_down"):
+            syn.bank[n] = syn.bank[n].bfloat16().float()
+        cast = lambda n, t: t.bfloat16() if n.startswith("scale") else t  # noqa: E731
+    layer = _check(syn, gpu, cast=cast)
+    assert layer.stage_kernel(T, nat.STAGE_W13) == kernel
+    assert layer.stage_kernel(T, nat.STAGE_W2) == "k_gemm_b"
+
+
+@pytest.mark.parametrize("name", ["c4_mxfp4", "c3_fp8", "c2_gptq", "c1_int8", "c1_int8_groups", "bf16"])
+def test_tiles_of_rows_past_32_bit_offsets(gpu, name):
+    """Activation rows that span more than 4 GiB go by 64-bit addresses: the
+    first and last tokens of 270000 have the bits that they have by
+    themselves."""
+    from ftmoe import layer as L
+
+    k, E, I = 8, 16, 1024
+    T = 270_000  # h: T x k rows of 2048 bytes and more
+    cfg = S.SMALL["c1_int8" if name in ("bf16", "c1_int8_groups") else name]
+    cfg = replace(cfg, E=E, k=k, H=256, I=I, shared_inter=0, expert_bias=False,
+                  int8_num_groups=2 if name == "c1_int8_groups" else 1, fmt="bf16" if name == "bf16" else cfg.fmt)
+    syn = S.generate(cfg, T=64, seed=11, device=gpu)
+    layer = S.build_layer(syn)
+    x = torch.randn(T, 256, device=gpu, generator=torch.Generator(device=gpu).manual_seed(1)).bfloat16()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        torch.cuda.current_stream().wait_stream(torch.cuda.default_stream())
+        out = layer.forward(x)
+        parts = [(sl, layer.forward(x[sl].contiguous())) for sl in (slice(0, 4096), slice(T - 4096, T))]
+        torch.cuda.synchronize()
+        L._WS.pop(L._ws_key(x.device))  # the stream's workspace of 7 GB and more
+    for sl, part in parts:
+        assert layer.stage_kernel(4096, nat.STAGE_W2) == layer.stage_kernel(T, nat.STAGE_W2)
+        assert torch.equal(out[sl], part)
