@@ -2,7 +2,7 @@
 // and the LDS-tiled bf16-MFMA GEMMs (v_mfma_f32_16x16x32_bf16) for the layers
 // the register-fed tiles (ftm_tile.hip) do not take: FP8 blocks other than
 // 128 x 128 with fp32 scales, FP8 with H or I not a multiple of 128, INT8 with
-// 64-wide groups, bf16 layers with fewer tiles than CUs.
+// groups other than K or whole 128s, bf16 layers with fewer tiles than CUs.
 //
 // Below the crossover every expert sees a handful of tokens and the stages are
 // weight-streaming GEMVs (ftm_moe.hip).  Above it (prefill) each expert's
@@ -868,11 +868,13 @@ static void launch_gemm_t(const LayerArgs& a, hipStream_t st, int which) {
   const long mt_shared = L.shared_inter > 0 ? (a.T + kGM - 1) / kGM : 0;
   const long items_a = mt_routed * (L.inter / 64) + mt_shared * (L.shared_inter > 0 ? L.shared_inter / 64 : 0);
   const long items_b = (mt_routed + mt_shared) * (L.hidden / 64);
-  // Stage A on the ring tiles where they apply (measured on MI355X, C3 FP8:
-  // w13 285 us against 343 at T=2048, 179 against 239 at T=512; C1 INT8 T=1024:
-  // 29 against 42).  Stage B keeps the register-staged tiles: with K = I its
-  // tiles are 8 K steps long and 4 workgroups per CU beat the deeper ring
-  // (C3 T=2048 w2 259 us against 377).
+  // Stage A on the ring tiles where they apply (us a layer on MI355X, ring /
+  // register-staged: 16 INT8 experts of 1024 with 64-wide groups at 256 / 1024
+  // tokens 70 / 110 against 73 / 125, 64 of 2048 at 512 / 2048 468 / 936 against
+  // 471 / 1087; 16 bf16 experts of 512 at 256 / 700 52.0 / 55.6 against 55.4 /
+  // 57.5).  Stage B keeps the register-staged tiles: with K = I its tiles are a
+  // few K steps long and 4 workgroups per CU beat the deeper ring (256 FP8
+  // experts of 512, 2048 tokens, w2 259 us against 377).
   const bool ring = ring_ok(L);
   if (which & 1) {
     if (ring) {

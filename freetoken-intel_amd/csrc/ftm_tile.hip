@@ -7,9 +7,12 @@
 // 64 rows x 64 weight rows over the whole K (stage A: 32 gate + 32 up
 // channels of w13, so the activation needs no exchange; stage B: 64 output
 // columns of w2).  A wave owns its weight rows, so the weights are loaded once
-// per tile by buffer loads into VGPRs, one K step ahead of their use; only the
-// activations, which all four waves read, go through LDS: a three-stage ring
-// filled by direct global->LDS copies two K steps ahead.  One barrier per K
+// per tile by buffer loads into VGPRs, one K step ahead of their use (in the
+// loops whose second step of a pair is behind a branch, bf16, INT8 with one
+// scale and MXFP4, in every second step only: in the other the compiler waits
+// for a step's weights before it requests the next); only the activations,
+// which all four waves read, go through LDS: a three-stage ring filled by
+// direct global->LDS copies two K steps ahead.  One barrier per K
 // step of 128 (64 for bf16 weights), two workgroups per CU (MXFP4: three).
 // Quantisation-group scales multiply the fp32 partial sums of each group, as
 // in the GEMV path.
@@ -17,11 +20,11 @@
 // Bound by the bytes a CU keeps in flight where an expert has about a tile of
 // rows, by LDS reads and MFMA issue where it has many.  Measured on MI355X, us
 // per layer, LDS-ring tiles (GPTQ: GEMV stages) before / these: 256 FP8
-// experts of 512 + shared at 512 / 2048 tokens 366 / 547 and 226 / 372; 32
-// MXFP4 experts of 2880 at 256 / 4096 343 / 1289 and 187 / 978; 128 GPTQ
+// experts of 512 + shared at 512 / 2048 tokens 352 / 549 and 223 / 355; 32
+// MXFP4 experts of 2880 at 256 / 4096 340 / 1287 and 189 / 972; 128 GPTQ
 // experts of 768 at 1000 / 4096 466 / 1613 and 213 / 550; 64 INT8 experts of
-// 1024 at 256 / 2048 242 / 542 and 128 / 275; 128 bf16 experts of 768 at 333
-// 337 and 279.
+// 1024 at 256 / 2048 237 / 523 and 127 / 259; 128 bf16 experts of 768 at 333
+// 334 and 284.
 //
 // GPTQ's activations stay the bf16 values that the GEMV stages read (a
 // two-term e4m3 split of them takes the same time, 209 us at 1000 tokens, but
@@ -521,7 +524,7 @@ extern __shared__ __attribute__((aligned(16))) char ftm_tile_lds[];
 // Items run expert by expert (ascending compact index), within an expert over
 // its M tiles first: the workgroups in flight on an XCD then share an
 // expert's weight columns and its activation rows in that XCD's L2.  The
-// shared expert's items come last.  rows <= 0: no item.
+// shared expert's items come first.  rows <= 0: no item.
 struct TileItem {
   const int32_t* list;  // the expert's pairs (null: the shared expert)
   int m0, rows, n0, slot;

@@ -55,7 +55,7 @@ WS_ERR_SLOT = 1
 WS_ERR_ID = 2
 WS_ERR_LIST = 4
 
-PROJ_RING_B = 1  # ftm_proj.flags: FP8 stage B on the ring tile (FTM_PROJ_RING_B)
+PROJ_RING_B = 1  # ftm_proj.flags: FP8 stage B on the three-stage ring (FTM_PROJ_RING_B)
 STAGE_ROUTER = 0
 STAGE_TOPK = 1
 STAGE_W13 = 2

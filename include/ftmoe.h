@@ -104,10 +104,12 @@ typedef struct ftm_proj {
   int32_t flags;        /* 0, or FTM_PROJ_* below */
 } ftm_proj;
 
-/* ftm_proj.flags.  FTM_PROJ_RING_B, on w2: FP8 stage B above the token
- * crossover runs on the ring tile (k_gemm_mx) even where the register-fed
- * tile (k_gemm_mxb_f8) would; both compute the same products, block scales
- * and epilogue in the same order, and tests compare their outputs bitwise. */
+/* ftm_proj.flags.  FTM_PROJ_RING_B, on w2: FP8 stage B from 16 tokens per
+ * expert on keeps its activations in a ring of three LDS stages (k_gemm_mx)
+ * even where K = inter of up to 512 has a stage for every K step
+ * (k_gemm_mxb_f8).  The two share the K step, the weight loads and the
+ * epilogue and differ in staging and waits alone; tests compare their outputs
+ * bitwise. */
 #define FTM_PROJ_RING_B 1
 
 /* One MoE layer: routed banks (w13 = gate||up [2I, H], w2 = down [H, I]),

@@ -199,12 +199,12 @@ def test_stage_kernel_names_follow_the_dispatch():
     # 512 tokens x top-8 = 16 pairs per expert on all 256 experts: GEMM
     # stages, the routed experts on the scaled-MFMA tiles (FP8 128 x 128 blocks)
     assert name(c3, 512, nat.STAGE_W13) == "k_gemm_mx"
-    # stage B: I = 512 (a multiple of 128 up to 512) keeps the tile's h rows
-    # in LDS and feeds the weights from registers; I = 640 takes the ring tile
+    # stage B: K = I of up to four 128-wide steps has an LDS stage for each;
+    # I = 640 takes the ring of three
     assert name(c3, 512, nat.STAGE_W2) == "k_gemm_mxb_f8"
     wide = _layer(E=256, H=2048, I=640, k=8)
     assert name(wide, 512, nat.STAGE_W2) == "k_gemm_mx"
-    c3.w2.flags = nat.PROJ_RING_B  # the ring tile on request (tests compare the two)
+    c3.w2.flags = nat.PROJ_RING_B  # the ring on request (tests compare the two)
     assert name(c3, 512, nat.STAGE_W2) == "k_gemm_mx"
     c3.w2.flags = 0
     # the GPU test's shapes (32 experts, top-4, 512 tokens) reach the register-fed tile

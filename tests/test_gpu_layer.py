@@ -325,22 +325,21 @@ def test_many_experts_routing(gpu, E, k):
 # ---------------------------------------------------------------- above the token crossover (tiled GEMMs)
 @pytest.mark.parametrize("name,T", [("c3_fp8", 512), ("c1_int8", 256), ("c4_mxfp4", 256), ("c3_fp8", 700)])
 def test_prefill_gemm_path_matches_oracle(gpu, name, T):
-    """At >= 16 tokens per routed expert the expert stages are the LDS-tiled
-    GEMMs (FP8 block, INT8 per-channel, MXFP4 with biases and the clamped
-    SwiGLU, the bf16 shared expert); same contract as the GEMV path."""
+    """At >= 16 tokens per routed expert the expert stages are tiles (FP8 block,
+    INT8 per-channel, MXFP4 with biases and the clamped SwiGLU, the bf16 shared
+    expert); same contract as the GEMV path."""
     syn = S.generate(S.SMALL[name], T=T, seed=40 + T)
     _run_and_check(syn, gpu)
 
 
 @pytest.mark.parametrize("H,I,bias", [(384, 384, False), (256, 128, False), (256, 256, True), (640, 512, False)])
 def test_fp8_prefill_register_fed_stage_b_shapes(gpu, H, I, bias):
-    """FP8 above the crossover with stage B on the register-fed tile
-    (k_gemm_mxb_f8, asserted by name): K = I of three, one, two and four
-    128-wide steps (the tile unrolls four), an odd number of 128-column N
-    tiles (H = 384, 640: 3 and 5; the workgroup's last N tile is then past
-    its range), bf16 expert biases (the tile's 16-bit bias loads).  Its
-    output equals the ring tile's stage B (k_gemm_mx, forced by
-    FTM_PROJ_RING_B on the same banks) bit for bit."""
+    """FP8 above the crossover with stage B on k_gemm_mxb_f8 (asserted by name):
+    K = I of three, one, two and four 128-wide steps (the kernel unrolls four),
+    a 256-column tile half past H (384, 640), bf16 expert biases.  Its output
+    equals k_gemm_mx's (forced by FTM_PROJ_RING_B on the same banks) bit for
+    bit: the two share the K step, the weight loads and the epilogue, so this
+    compares their staging and waits; the oracle checks the values."""
     from dataclasses import replace
 
     from ftmoe import _native as nat
@@ -359,7 +358,7 @@ def test_fp8_prefill_register_fed_stage_b_shapes(gpu, H, I, bias):
 
 @pytest.mark.parametrize("T", [256, 600])
 def test_mxfp4_tiles_wide_range_inputs(gpu, T):
-    """MXFP4 above the crossover: stage A on the scaled-MFMA tiles (128-token
+    """MXFP4 above the crossover: stage A on the scaled-MFMA tiles (64-token
     M tiles, partly filled at 64 and 150 tokens per expert; H = 320 ends in a
     half K step) with inputs spanning 2^-14 .. 2^3 inside each 32-wide block:
     the output stays at bf16 precision (relative RMS MX_REL_RMS).  Caller

@@ -205,18 +205,20 @@ def test_bf16_output_does_not_depend_on_the_tile_kind(gpu, H):
     assert torch.equal(out[:80], part)
 
 
-@pytest.mark.parametrize("fmt,kernel", [("c3_fp8", "k_gemm_mx"), ("c1_int8", "k_tile")])
+@pytest.mark.parametrize("fmt,kernel", [("c3_fp8", "k_gemm_mx"), ("c1_int8", "k_tile"), ("c2_gptq", "k_tile"),
+                                        ("c4_mxfp4", "k_gemm_mx")])
 def test_shared_expert_bits_beside_any_experts(gpu, fmt, kernel):
-    """Routed banks of zeros leave the shared expert's output: beside FP8 and
-    INT8 tiles the same bits as beside bf16 experts on the LDS-ring tiles."""
+    """Routed banks of zeros leave the shared expert's output: beside every
+    format's tiles the same bits as beside bf16 experts on the LDS-ring tiles."""
     T, H, Is = 200, 384, 192
     outs = []
     for f, I, want in ((fmt, 128, kernel), ("bf16", 64, "k_gemm_a_ring")):
         cfg = S.SMALL["c1_int8"] if f == "bf16" else S.SMALL[f]
-        cfg = replace(cfg, fmt=f if f == "bf16" else cfg.fmt, E=8, k=2, H=H, I=I, shared_inter=Is)
+        cfg = replace(cfg, fmt=f if f == "bf16" else cfg.fmt, E=8, k=2, H=H, I=I, shared_inter=Is, act="silu",
+                      route_mode="softmax_topk", gate_bias=False, expert_bias=False)
         syn = S.generate(cfg, T=T, seed=1)
         for n, t in syn.bank.items():
-            if f == "bf16" or n.startswith(("scale", "weight_scale")):
+            if f == "bf16" or n.startswith(("scale", "weight_scale", "blocks")):
                 t.zero_()
         if outs:
             syn.x, syn.gate_w, syn.shared = first.x, first.gate_w, first.shared
